@@ -2,14 +2,14 @@
 // (CliqueArgs in kernels.h).
 //
 // Start vertices with at most 64 upper neighbours are counted by
-// CliqueSmallKernel: one wave per vertex, lane i holding row i in a register,
-// so every set below a row is one u64 and every step of the count is a
-// readlane, an AND and a popcount.  Larger neighbourhoods are counted in
-// batches: CliqueRowsKernel writes each vertex's rows to device memory (one
-// wave per row, its lanes testing 64 candidates at a time by binary search
-// in the row vertex's own upper list), then CliqueCountKernel takes one row
-// i per wave, keeps the sets it derives from row i in LDS and counts the
-// last level by AND + popcount over whole words, 64 clique members per word.
+// CliqueSmallKernel: a row is one u64, so every set below a row is one u64 and
+// every step of the count is an LDS load, an AND and a popcount.  Larger
+// neighbourhoods are counted in batches: CliqueRowsKernel writes each vertex's
+// rows to device memory (one wave per row, its lanes testing 64 candidates at
+// a time by binary search in the row vertex's own upper list), then
+// CliqueCountKernel takes one row i per wave, keeps the sets it derives from
+// row i in LDS and counts the last level by AND + popcount over whole words,
+// 64 clique members per word.
 //
 // The reference counts the same cliques by intersecting sorted adjacency
 // lists level by level (src/gpu/impl/light/op/LIGHTCompute.cuh,
@@ -17,13 +17,13 @@
 // neighbourhood become bit rows, and one word operation replaces up to 64
 // membership probes.
 #include "kernels.h"
+#include "wave.h"
 
 namespace sme {
 
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kWave = 64;
 constexpr int kWaves = kThreads / kWave;
 constexpr uint32_t kWordsMax = kLocalMax / 64;  // words of the longest row
 static_assert(2 * kRowsHashSmall <= (1u << 10) && 2 * kRowsHashMax <= (1u << 13), "hash tables at most half full");
@@ -37,27 +37,8 @@ uint64_t Grid(uint64_t n, uint64_t per_block) {
   return g > kMaxGrid ? kMaxGrid : g;
 }
 
-// Orders the LDS accesses of a wave: every lane's earlier accesses complete
-// before any lane's later ones.
-__device__ __forceinline__ void Sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-__device__ __forceinline__ u64 Sum64(u64 v) {
-#pragma unroll
-  for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return v;
-}
-
 __device__ __forceinline__ uint32_t Lane32(uint32_t v, uint32_t lane) {
   return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), static_cast<int>(lane)));
-}
-
-__device__ __forceinline__ u64 Lane64(u64 v, uint32_t lane) {
-  return (static_cast<u64>(Lane32(static_cast<uint32_t>(v >> 32), lane)) << 32) |
-         Lane32(static_cast<uint32_t>(v), lane);
 }
 
 __device__ __forceinline__ u64 First64(u64 v) {
@@ -81,158 +62,268 @@ __device__ __forceinline__ bool Holds(const uint32_t* a, uint64_t lo, uint64_t h
   return lo < end && a[lo] == key;
 }
 
-// Largest bucket index b with bounds[b] <= v.
-__device__ __forceinline__ uint64_t BucketIndex(const BucketRef& b, uint32_t v) {
-  if (b.table) return b.table[v - b.base];
-  uint64_t lo = 0, hi = b.nbuckets - 1;
-  while (lo < hi) {
-    const uint64_t mid = (lo + hi + 1) >> 1;
-    if (b.bounds[mid] <= v)
-      lo = mid;
-    else
-      hi = mid - 1;
-  }
-  return lo;
-}
-
 __device__ __forceinline__ void AddBucket(const BucketRef& b, uint32_t v, u64 per_lane, int lane) {
-  const u64 tot = Sum64(per_lane);
-  if (lane == 0 && tot) atomicAdd(b.counts + BucketIndex(b, v), tot);
+  const u64 tot = WaveSum(per_lane);
+  if (lane == 0 && tot) atomicAdd(b.counts + BucketOf(b, v), tot);
 }
 
 __device__ __forceinline__ void Flush(unsigned long long* acc, int j, u64 v, int lane) {
-  v = Sum64(v);
+  v = WaveSum(v);
   if (lane == 0 && v) atomicAdd(acc + j, v);
 }
 
 // ---------------------------------------------------------------------------
-// One wave per start vertex with d <= 64.  Lane i builds row i: for each i
-// the wave searches u_j (lane j > i) in N+(u_i) and the ballot is row i.
+// Start vertices with d <= 64.  A wave takes kSmallGroup consecutive start
+// vertices, packs as many whole ones as fit into 64 upper entries (lane =
+// entry u_i of some N+(v)) and walks their entries' work as one flat list of
+// items, 64 per step, so short neighbourhoods share a step.  An entry's work
+// is the cheaper of
+//   stream: the values x of N+(u_i), each looked up among the u_j (j > i)
+//           staged in LDS (one coalesced load and at most 6 LDS steps);
+//   search: the u_j (j > i), each searched in N+(u_i) (a chain of dependent
+//           loads, log2 |N+(u_i)| long).
+// A hit (i, j) is a triangle.  From K = 4 on it sets bit j of row i in LDS,
+// and lane = row then counts the larger cliques by AND + popcount.
+//
+// Bound by the latency of the gathers (list bounds, then list values).  One
+// wave per start vertex, searching one row after another with most lanes
+// idle, took 10.2 ms on 1,000 packed G(n, m) members (5.4e7 entries, 13 per
+// vertex) and 3.7 ms on R-MAT scale 20 (degree-ranked, 6 per vertex); the
+// flat items take 3.1 and 1.4 ms.  Groups of 8 or 16 start vertices were
+// slower (1.6, 1.7 ms on R-MAT: the heavy groups end last), and so was
+// choosing the mode on rem * steps < len (67 against 87 us, R-MAT scale 14).
+constexpr uint32_t kSmallGroup = 4;  // start vertices per wave step
+constexpr uint32_t kSmallStream = 32;    // lists up to this length are streamed
+// up to here one start vertex per wave step: 4,096 waves of 4 vertices would
+// leave half the chip idle (R-MAT scale 14: 67 us against 130 us)
+constexpr uint64_t kSmallAlone = 16384;
+constexpr uint64_t kSmallGrid = 2048;    // workgroups: 8 per CU
+
+struct SmallLds {
+  uint64_t beg[kWave];    // entry: N+(u_i) begins at cols[beg]
+  u64 row[kWave];         // entry: row i (K >= 4)
+  uint32_t key[kWave];    // entry: u_i
+  uint32_t len[kWave];    // entry: |N+(u_i)|
+  uint32_t base[kWave];   // entry: its vertex's first entry
+  uint32_t last[kWave];   // entry: one past its vertex's last entry
+  uint32_t start[kWave];  // k-th entry with work: its first item
+  uint32_t edge[kWave];   // k-th entry with work: the entry, bit 31: search
+  uint32_t flag[kWave];   // item of this step starts an entry
+  uint32_t cnt[kWave];    // entry: triangles (per-edge counts or buckets)
+};
+
 template <int K>
 __global__ __launch_bounds__(kThreads) void CliqueSmallKernel(CliqueArgs a) {
+  __shared__ SmallLds lds_all[kWaves];
+  __shared__ u64 lds_sum[kCliqueMaxK + 1];
   const int lane = threadIdx.x & (kWave - 1);
+  SmallLds& s = lds_all[threadIdx.x / kWave];
+  const u64 upto = ~0ull >> (kWave - 1 - lane);  // lanes 0..lane
   const uint64_t wave = (blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x) / kWave;
   const uint64_t nwaves = static_cast<uint64_t>(gridDim.x) * blockDim.x / kWave;
   const uint64_t nv = a.v_end - a.v_begin;
+  const bool counted = a.tc || a.bk.bounds;  // triangles are kept per entry
   u64 c1 = 0, c2 = 0, c3 = 0, c4 = 0, c5 = 0, c6 = 0;
-  for (uint64_t t = wave; t < nv; t += nwaves) {
-    const uint32_t v = a.v_begin + static_cast<uint32_t>(t);
-    const uint64_t nb = a.up[v];
-    const uint64_t d = a.rp[v + 1] - nb;
-    if (d > kLocalSmall) {
-      // (big == nullptr: the caller already holds these lists)
-      if (lane == 0 && d <= kLocalMax) {
-        if (a.big) {
-          const u64 pos = atomicAdd(a.nbig, 1ull);
-          a.big[pos] = v;
-          a.big_d[pos] = static_cast<uint32_t>(d);
-        }
+  BucketAcc bacc{kNoBucket, 0};
+  const uint64_t ngroups = (nv + a.group - 1) / a.group;
+  for (uint64_t t = wave; t < ngroups; t += nwaves) {
+    const uint64_t first = t * a.group;
+    const uint32_t gn = static_cast<uint32_t>(first + a.group < nv ? a.group : nv - first);
+    uint64_t nb_l = 0, d_l = 0;  // lane q: vertex q of the group
+    if (static_cast<uint32_t>(lane) < gn) {
+      const uint32_t v = a.v_begin + static_cast<uint32_t>(first) + lane;
+      nb_l = a.up[v];
+      d_l = a.rp[v + 1] - nb_l;
+      if (d_l <= kLocalMax) {
         c1 += 1;
-        c2 += d;
-      } else if (lane == 0 && a.huge) {
-        a.huge[atomicAdd(a.nhuge, 1ull)] = v;
+        c2 += d_l;
       }
-      continue;
-    }
-    if (lane == 0) {
-      c1 += 1;
-      c2 += d;
-    }
-    if (d < 2) continue;
-    const uint32_t du = static_cast<uint32_t>(d);
-    const uint32_t uj = static_cast<uint32_t>(lane) < du ? a.cols[nb + lane] : 0u;
-    u64 row = 0;     // lane i: row i
-    uint32_t col = 0;  // lane j: rows i < j holding bit j
-    // rows i and i + 1 together: their two searches run in lockstep, so two
-    // independent loads are in flight per step
-    for (uint32_t i = 0; i + 1 < du; i += 2) {
-      const uint32_t ua = Lane32(uj, i);
-      const uint32_t ub = Lane32(uj, i + 1);
-      uint64_t lo1 = a.up[ua], hi1 = a.rp[ua + 1], lo2 = a.up[ub], hi2 = a.rp[ub + 1];
-      const uint64_t end1 = hi1, end2 = hi2;
-      const bool act1 = static_cast<uint32_t>(lane) > i && static_cast<uint32_t>(lane) < du;
-      const bool act2 = static_cast<uint32_t>(lane) > i + 1 && static_cast<uint32_t>(lane) < du;
-      if (!act1) lo1 = hi1;
-      if (!act2) lo2 = hi2;
-      while (lo1 < hi1 || lo2 < hi2) {
-        const bool g1 = lo1 < hi1, g2 = lo2 < hi2;
-        const uint64_t m1 = (lo1 + hi1) >> 1, m2 = (lo2 + hi2) >> 1;
-        const uint32_t x1 = g1 ? a.cols[m1] : 0u;
-        const uint32_t x2 = g2 ? a.cols[m2] : 0u;
-        if (g1) {
-          if (x1 < uj)
-            lo1 = m1 + 1;
-          else
-            hi1 = m1;
+      if (d_l > kLocalSmall) {
+        // (big == nullptr: the caller already holds these lists)
+        if (d_l <= kLocalMax) {
+          if (a.big) {
+            const u64 pos = atomicAdd(a.nbig, 1ull);
+            a.big[pos] = v;
+            a.big_d[pos] = static_cast<uint32_t>(d_l);
+          }
+        } else if (a.huge) {
+          a.huge[atomicAdd(a.nhuge, 1ull)] = v;
         }
-        if (g2) {
-          if (x2 < uj)
-            lo2 = m2 + 1;
-          else
-            hi2 = m2;
-        }
+        d_l = 0;
       }
-      const bool ok1 = act1 && lo1 < end1 && a.cols[lo1] == uj;
-      const bool ok2 = act2 && lo2 < end2 && a.cols[lo2] == uj;
-      const u64 r1 = __ballot(ok1);
-      const u64 r2 = __ballot(ok2);
-      if (static_cast<uint32_t>(lane) == i) row = r1;
-      if (static_cast<uint32_t>(lane) == i + 1) row = r2;
-      if (a.tc) {
-        // edges (u_i, u_j): triangles (v, u_i, u_j)
-        if (ok1) {
-          atomicAdd(a.tc + lo1, 1u);
-          ++col;
-        }
-        if (ok2) {
-          atomicAdd(a.tc + lo2, 1u);
-          ++col;
-        }
-      }
+      if (d_l < 2) d_l = 0;  // no triangle from v
     }
-    const u64 tri = __popcll(row);
-    // edge (v, u_i): the triangles (v, u_i, x) counted from v
-    if (a.tc && static_cast<uint32_t>(lane) < du && tri + col)
-      atomicAdd(a.tc + nb + lane, static_cast<uint32_t>(tri) + col);
-    c3 += tri;
-    u64 vk = K == 3 ? tri : 0;  // this lane's share of the k-cliques from v
-    if (K >= 4) {
-      for (uint32_t i = 0; i + 2 < du; ++i) {
-        const u64 s1 = Lane64(row, i);
-        if (!s1) continue;
-        const u64 x4 = ((s1 >> lane) & 1) ? __popcll(s1 & row) : 0;
-        c4 += x4;
-        if (K == 4) {
-          vk += x4;
+    uint32_t dq[kSmallGroup];
+    uint64_t nbq[kSmallGroup];
+#pragma unroll
+    for (uint32_t q = 0; q < kSmallGroup; ++q) {
+      dq[q] = Lane32(static_cast<uint32_t>(d_l), q);
+      nbq[q] = (static_cast<uint64_t>(Lane32(static_cast<uint32_t>(nb_l >> 32), q)) << 32) |
+               Lane32(static_cast<uint32_t>(nb_l), q);
+    }
+    for (uint32_t q0 = 0; q0 < gn;) {
+      // vertices q0.. of the group whose entries fit the wave together
+      uint32_t ne = 0, d = 0, i = 0, end = 0, q1 = q0, mine = q0;
+      uint64_t nb = 0;
+      bool open = true;
+#pragma unroll
+      for (uint32_t q = 0; q < kSmallGroup; ++q) {
+        if (q < q0 || q >= gn) continue;
+        if (!open || ne + dq[q] > kWave) {
+          open = false;
           continue;
         }
+        if (static_cast<uint32_t>(lane) >= ne && static_cast<uint32_t>(lane) < ne + dq[q]) {
+          d = dq[q];
+          nb = nbq[q];
+          i = static_cast<uint32_t>(lane) - ne;
+          end = ne + dq[q];
+          mine = q;
+        }
+        ne += dq[q];
+        q1 = q + 1;
+      }
+      q0 = q1;
+      if (ne == 0) continue;
+      const bool entry = static_cast<uint32_t>(lane) < ne;
+      uint32_t u = 0, len = 0;
+      uint64_t lb = 0;
+      if (entry) {
+        u = a.cols[nb + i];
+        if (i + 1 < d) {
+          lb = a.up[u];
+          len = static_cast<uint32_t>(a.rp[u + 1] - lb);
+        }
+      }
+      const uint32_t rem = len ? d - 1 - i : 0;  // u_j above u_i
+      const uint32_t steps = 32 - static_cast<uint32_t>(__clzll(static_cast<long long>(len))) + 32;
+      // (a wave whose items mix both pays for both: short lists always stream)
+      const bool search = len > kSmallStream && rem * steps < 2 * len;
+      const uint32_t items = search ? rem : (rem ? len : 0);
+      uint32_t total;
+      const uint32_t start = WavePrefix(items, lane, &total);
+      if (total == 0) continue;
+      const u64 work = __ballot(items != 0);
+      WaveSync();  // the previous step's readers are done
+      s.key[lane] = u;
+      s.beg[lane] = lb;
+      s.len[lane] = len;
+      s.base[lane] = end - d;
+      s.last[lane] = end;
+      if (K >= 4) s.row[lane] = 0;
+      if (counted) s.cnt[lane] = 0;
+      if (items) {
+        const int at = static_cast<int>(__popcll(work & (upto >> 1)));
+        s.start[at] = start;
+        s.edge[at] = static_cast<uint32_t>(lane) | (search ? 0x80000000u : 0u);
+      }
+      uint32_t before = 0;  // entries with work that started before this step
+      for (uint32_t t0 = 0; t0 < total; t0 += kWave) {
+        s.flag[lane] = 0;
+        WaveSync();
+        if (items && start >= t0 && start - t0 < kWave) s.flag[start - t0] = 1;
+        WaveSync();
+        const u64 starts = __ballot(s.flag[lane] != 0);
+        const uint32_t own = before + static_cast<uint32_t>(__popcll(starts & upto)) - 1;
+        before += static_cast<uint32_t>(__popcll(starts));
+        const uint32_t it = t0 + static_cast<uint32_t>(lane);
+        if (it < total) {
+          const uint32_t packed = s.edge[own];
+          const uint32_t e = packed & 0x7fffffffu, k = it - s.start[own];
+          uint64_t lo = s.beg[e];
+          uint32_t j = e + 1;  // entry of the vertex holding the value
+          bool hit;
+          if (packed >> 31) {
+            j += k;
+            const uint32_t x = s.key[j];
+            const uint64_t le = lo + s.len[e];
+            uint64_t hi = le;
+            while (lo < hi) {
+              const uint64_t mid = (lo + hi) >> 1;
+              if (a.cols[mid] < x)
+                lo = mid + 1;
+              else
+                hi = mid;
+            }
+            hit = lo < le && a.cols[lo] == x;
+          } else {
+            lo += k;
+            const uint32_t x = a.cols[lo], je = s.last[e];
+            uint32_t hi = je;
+            while (j < hi) {
+              const uint32_t mid = (j + hi) >> 1;
+              if (s.key[mid] < x)
+                j = mid + 1;
+              else
+                hi = mid;
+            }
+            hit = j < je && s.key[j] == x;
+          }
+          if (hit) {
+            if (K == 3) {
+              ++c3;
+              if (counted) atomicAdd(s.cnt + e, 1u);
+              if (a.tc) {
+                atomicAdd(s.cnt + j, 1u);
+                atomicAdd(a.tc + lo, 1u);  // edge (u_i, u_j)
+              }
+            } else {
+              atomicOr(s.row + e, 1ull << (j - s.base[e]));
+            }
+          }
+        }
+      }
+      WaveSync();
+      u64 vk = 0;  // this entry's share of the k-cliques from its vertex
+      if (K == 3) {
+        // edges (v, u_i): the triangles (v, u_i, x)
+        if (counted) vk = s.cnt[lane];
+        if (a.tc && entry && vk) atomicAdd(a.tc + nb + i, static_cast<uint32_t>(vk));
+      } else if (entry) {
+        const uint32_t base = end - d;
+        const u64 s1 = s.row[lane];
+        c3 += __popcll(s1);
         for (u64 m1 = s1; m1; m1 &= m1 - 1) {
-          const u64 s2 = s1 & Lane64(row, static_cast<uint32_t>(__builtin_ctzll(m1)));
-          if (!s2) continue;
-          const u64 x5 = ((s2 >> lane) & 1) ? __popcll(s2 & row) : 0;
-          c5 += x5;
-          if (K == 5) {
-            vk += x5;
+          const u64 s2 = s1 & s.row[base + static_cast<uint32_t>(__builtin_ctzll(m1))];
+          const u64 x4 = __popcll(s2);
+          c4 += x4;
+          if (K == 4) {
+            vk += x4;
             continue;
           }
           for (u64 m2 = s2; m2; m2 &= m2 - 1) {
-            const u64 s3 = s2 & Lane64(row, static_cast<uint32_t>(__builtin_ctzll(m2)));
-            if (!s3) continue;
-            const u64 x6 = ((s3 >> lane) & 1) ? __popcll(s3 & row) : 0;
-            c6 += x6;
-            vk += x6;
+            const u64 s3 = s2 & s.row[base + static_cast<uint32_t>(__builtin_ctzll(m2))];
+            const u64 x5 = __popcll(s3);
+            c5 += x5;
+            if (K == 5) {
+              vk += x5;
+              continue;
+            }
+            for (u64 m3 = s3; m3; m3 &= m3 - 1) {
+              const u64 x6 = __popcll(s3 & s.row[base + static_cast<uint32_t>(__builtin_ctzll(m3))]);
+              c6 += x6;
+              vk += x6;
+            }
           }
         }
       }
+      if (a.bk.bounds)
+        BucketAccAdd(a.bk, &bacc, entry ? BucketOf(a.bk, a.v_begin + static_cast<uint32_t>(first) + mine) : kNoBucket, vk);
     }
-    if (a.bk.bounds) AddBucket(a.bk, v, vk, lane);
   }
-  Flush(a.acc, 1, c1, lane);
-  Flush(a.acc, 2, c2, lane);
-  Flush(a.acc, 3, c3, lane);
-  if (K >= 4) Flush(a.acc, 4, c4, lane);
-  if (K >= 5) Flush(a.acc, 5, c5, lane);
-  if (K >= 6) Flush(a.acc, 6, c6, lane);
+  if (a.bk.bounds) BucketFlush(a.bk, &bacc);
+  // one atomic per workgroup and level
+  if (threadIdx.x <= static_cast<unsigned>(kCliqueMaxK)) lds_sum[threadIdx.x] = 0;
+  __syncthreads();
+  Flush(lds_sum, 1, c1, lane);
+  Flush(lds_sum, 2, c2, lane);
+  Flush(lds_sum, 3, c3, lane);
+  if (K >= 4) Flush(lds_sum, 4, c4, lane);
+  if (K >= 5) Flush(lds_sum, 5, c5, lane);
+  if (K >= 6) Flush(lds_sum, 6, c6, lane);
+  __syncthreads();
+  if (threadIdx.x >= 1 && threadIdx.x <= static_cast<unsigned>(K) && lds_sum[threadIdx.x])
+    atomicAdd(a.acc + threadIdx.x, lds_sum[threadIdx.x]);
 }
 
 // ---------------------------------------------------------------------------
@@ -367,7 +458,7 @@ __global__ __launch_bounds__(kThreads) void CliqueRowsHashKernel(CliqueArgs a) {
         le_next = a.rp[u + 1];
       }
       for (uint32_t w = lane; w < W; w += kWave) row[w] = 0;
-      Sync();
+      WaveSync();
       uint32_t bits = 0;
       // chunks of 64 entries, the next chunk's load issued before this
       // chunk's lookups
@@ -399,19 +490,19 @@ __global__ __launch_bounds__(kThreads) void CliqueRowsHashKernel(CliqueArgs a) {
           }
         }
       }
-      Sync();
+      WaveSync();
       for (uint32_t w = lane; w < W; w += kWave) rows[static_cast<uint64_t>(w) * d + i] = row[w];
       if (a.tc) {
         // edge (v, u_i): one triangle per bit of row i (only the per-edge
         // pass needs the row's popcount here; otherwise the count kernel
         // takes it)
-        const u64 tot = Sum64(bits);
+        const u64 tot = WaveSum(bits);
         if (lane == 0) {
           if (tot) atomicAdd(a.tc + nb + i, static_cast<uint32_t>(tot));
           c3 += tot;
         }
       }
-      Sync();
+      WaveSync();
     }
     if (a.tc) {
       __syncthreads();
@@ -446,21 +537,21 @@ __device__ __forceinline__ u64 LastLevel(const u64* s, uint32_t lo, uint32_t W, 
     if ((bits >> lane) & 1) q[qn + __popcll(bits & below)] = c * 64 + static_cast<uint32_t>(lane);
     qn += __popcll(bits);
     if (qn >= static_cast<uint32_t>(kWave)) {
-      Sync();
+      WaveSync();
       sum += Probe(s, W, d, rows, q[lane]);
       const uint32_t rest = qn - kWave;
       const uint32_t carry = static_cast<uint32_t>(lane) < rest ? q[kWave + lane] : 0u;
-      Sync();
+      WaveSync();
       if (static_cast<uint32_t>(lane) < rest) q[lane] = carry;
       qn = rest;
-      Sync();
+      WaveSync();
     }
   }
   if (qn) {
-    Sync();
+    WaveSync();
     if (static_cast<uint32_t>(lane) < qn) sum += Probe(s, W, d, rows, q[lane]);
   }
-  Sync();
+  WaveSync();
   return sum;
 }
 
@@ -481,7 +572,7 @@ __device__ __forceinline__ u64 CountRow(const u64* rows, uint32_t d, uint32_t i,
   const u64* ri = rows + i;
   const uint32_t lo1 = (i + 1) >> 6;
   u64 vk = 0;
-  Sync();
+  WaveSync();
   for (uint32_t w = lo1 + lane; w < W; w += kWave) {
     const u64 xw = ri[static_cast<uint64_t>(w) * d];
     if (K >= 4) s1[w] = xw;
@@ -489,7 +580,7 @@ __device__ __forceinline__ u64 CountRow(const u64* rows, uint32_t d, uint32_t i,
     if (K == 3) vk += __popcll(xw);
   }
   if (K < 4) return vk;
-  Sync();
+  WaveSync();
   if (K == 4) {
     const u64 y = LastLevel(s1, lo1, W, d, rows, q, lane);
     cs->c4 += y;
@@ -501,7 +592,7 @@ __device__ __forceinline__ u64 CountRow(const u64* rows, uint32_t d, uint32_t i,
       const u64* rj = rows + j;
       const uint32_t lo2 = (j + 1) >> 6;
       u64 nz = 0;
-      Sync();
+      WaveSync();
       for (uint32_t w = lo2 + lane; w < W; w += kWave) {
         const u64 xw = s1[w] & rj[static_cast<uint64_t>(w) * d];
         s2[w] = xw;
@@ -509,7 +600,7 @@ __device__ __forceinline__ u64 CountRow(const u64* rows, uint32_t d, uint32_t i,
         nz |= xw;
       }
       if (!__ballot(nz != 0)) continue;
-      Sync();
+      WaveSync();
       if (K == 5) {
         const u64 y = LastLevel(s2, lo2, W, d, rows, q, lane);
         cs->c5 += y;
@@ -522,7 +613,7 @@ __device__ __forceinline__ u64 CountRow(const u64* rows, uint32_t d, uint32_t i,
           const u64* rl = rows + l;
           const uint32_t lo3 = (l + 1) >> 6;
           u64 nz3 = 0;
-          Sync();
+          WaveSync();
           for (uint32_t w = lo3 + lane; w < W; w += kWave) {
             const u64 xw = s2[w] & rl[static_cast<uint64_t>(w) * d];
             s3[w] = xw;
@@ -530,7 +621,7 @@ __device__ __forceinline__ u64 CountRow(const u64* rows, uint32_t d, uint32_t i,
             nz3 |= xw;
           }
           if (!__ballot(nz3 != 0)) continue;
-          Sync();
+          WaveSync();
           const u64 y = LastLevel(s3, lo3, W, d, rows, q, lane);
           cs->c6 += y;
           vk += y;
@@ -589,12 +680,17 @@ __global__ __launch_bounds__(kThreads) void CliqueCountKernel(CliqueArgs a) {
 
 void LaunchCliqueSmall(const CliqueArgs& a, hipStream_t stream) {
   if (a.v_end <= a.v_begin) return;
-  const dim3 grid(Grid(a.v_end - a.v_begin, kWaves)), block(kThreads);
+  // few start vertices: one per wave, so that the launch spreads over the chip
+  const uint64_t nv = a.v_end - a.v_begin;
+  CliqueArgs b = a;
+  b.group = nv > kSmallAlone ? kSmallGroup : 1;
+  const uint64_t need = Grid((nv + b.group - 1) / b.group, kWaves);
+  const dim3 grid(need < kSmallGrid ? need : kSmallGrid), block(kThreads);
   switch (a.k) {
-    case 3: hipLaunchKernelGGL(CliqueSmallKernel<3>, grid, block, 0, stream, a); break;
-    case 4: hipLaunchKernelGGL(CliqueSmallKernel<4>, grid, block, 0, stream, a); break;
-    case 5: hipLaunchKernelGGL(CliqueSmallKernel<5>, grid, block, 0, stream, a); break;
-    case 6: hipLaunchKernelGGL(CliqueSmallKernel<6>, grid, block, 0, stream, a); break;
+    case 3: hipLaunchKernelGGL(CliqueSmallKernel<3>, grid, block, 0, stream, b); break;
+    case 4: hipLaunchKernelGGL(CliqueSmallKernel<4>, grid, block, 0, stream, b); break;
+    case 5: hipLaunchKernelGGL(CliqueSmallKernel<5>, grid, block, 0, stream, b); break;
+    case 6: hipLaunchKernelGGL(CliqueSmallKernel<6>, grid, block, 0, stream, b); break;
   }
 }
 

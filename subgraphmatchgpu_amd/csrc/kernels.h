@@ -357,6 +357,7 @@ struct CliqueArgs {
   // are appended to (big, big_d), those with d > kLocalMax to huge (not when
   // big / huge are null: the caller holds these lists already).
   uint32_t v_begin, v_end;
+  uint32_t group;                // start vertices per wave step (set by the launcher)
   uint32_t* big;
   uint32_t* big_d;
   unsigned long long* nbig;

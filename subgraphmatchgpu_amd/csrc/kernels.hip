@@ -4,13 +4,13 @@
 // owns a chunk of 64 consecutive items, so the validity of a chunk is one
 // __ballot word and stable compaction needs only a popcount prefix.
 #include "kernels.h"
+#include "wave.h"
 
 namespace sme {
 
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kWave = 64;
 constexpr int kWavesPerBlock = kThreads / kWave;
 constexpr uint64_t kMaxGrid = 16384;
 constexpr uint32_t kStageCap = kStageEntries;
@@ -55,76 +55,8 @@ __device__ __forceinline__ uint64_t SegmentOf(const ItemArgs& a, uint64_t c, uin
   return lo;
 }
 
-__device__ __forceinline__ u64 WaveSum(u64 v) {
-#pragma unroll
-  for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return v;
-}
-
 __device__ __forceinline__ uint64_t SegIndex(const CandRef& c, uint64_t p) {
   return c.idx ? c.idx[p] : p;
-}
-
-constexpr u64 kNoBucket = ~0ull;
-
-// Bucket of start vertex v: largest k with bounds[k] <= v.
-__device__ __forceinline__ u64 BucketOf(const BucketRef& b, uint32_t v) {
-  if (b.table) return b.table[v - b.base];
-  uint64_t lo = 0, hi = b.nbuckets - 1;
-  while (lo < hi) {
-    const uint64_t mid = (lo + hi + 1) >> 1;
-    if (b.bounds[mid] <= v)
-      lo = mid;
-    else
-      hi = mid - 1;
-  }
-  return lo;
-}
-
-// Per-wave running bucket sum (wave-uniform).  Bucket counts are added
-// into it while the wave's keys stay on one bucket and written with one
-// atomic when the bucket changes, so a wave issues about one atomic per
-// bucket it touches instead of one per chunk (a few buckets would otherwise
-// serialize every wave on the same counters).
-struct BucketAcc {
-  u64 key;
-  u64 sum;
-};
-
-__device__ __forceinline__ void BucketFlush(const BucketRef& b, BucketAcc* acc) {
-  if ((threadIdx.x & (kWave - 1)) == 0 && acc->sum && acc->key != kNoBucket)
-    atomicAdd(b.counts + acc->key, acc->sum);
-  acc->key = kNoBucket;
-  acc->sum = 0;
-}
-
-// Adds each lane's value under its bucket key (keys non-decreasing across
-// the wave; kNoBucket for lanes with nothing).  Must be reached by all 64
-// lanes.  Runs before the wave's last bucket are written at once; the last
-// one stays in the accumulator.
-__device__ __forceinline__ void BucketAccAdd(const BucketRef& b, BucketAcc* acc, u64 key, u64 val) {
-  const int lane = threadIdx.x & (kWave - 1);
-  if (__ballot(key != kNoBucket && key != acc->key) == 0) {
-    acc->sum += WaveSum(val);
-    return;
-  }
-  BucketFlush(b, acc);
-  u64 v = val;
-#pragma unroll
-  for (int o = 1; o < kWave; o <<= 1) {
-    const u64 y = __shfl_up(v, o);
-    const u64 k2 = __shfl_up(key, o);
-    if (lane >= o && k2 == key) v += y;
-  }
-  const u64 next = __shfl_down(key, 1);
-  const bool run_end = lane == kWave - 1 || next != key;
-  const u64 live = __ballot(key != kNoBucket);  // not 0: some key differed from acc
-  const int last = kWave - 1 - __clzll(static_cast<long long>(live));
-  const u64 last_key = __shfl(key, last);
-  const u64 last_sum = __shfl(v, last);
-  if (run_end && key != kNoBucket && key != last_key && v) atomicAdd(b.counts + key, v);
-  acc->key = last_key;
-  acc->sum = last_sum;
 }
 
 // ThreadCountWithComputedVertex (CheckConstraintsCommon.cuh:131-155): how
@@ -468,14 +400,6 @@ __device__ __forceinline__ u64 GenericChunk(const ItemArgs& a, uint64_t c, int l
     BucketAccAdd(a.bk, bacc, key, val);
   }
   return val;
-}
-
-// Wave-level ordering point for LDS staging: every lane's earlier LDS
-// accesses complete before any lane's later ones.
-__device__ __forceinline__ void WaveSync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 __device__ __forceinline__ uint64_t Uniform64(uint64_t v) {

@@ -1,0 +1,100 @@
+"""Sizes at which the counting kernels change tile, table or schedule, against
+the oracle: on the CPU through the stand-in runtime of tests/emu (under
+AddressSanitizer) and on the GPU.  Counts are whole numbers and must be equal."""
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+import oracle
+import subgraphmatchgpu_amd as sme
+from conftest import ROOT, clique
+
+EMU_DIR = os.path.join(ROOT, "tests", "emu")
+
+
+@pytest.fixture(scope="module")
+def emu(tmp_path_factory):
+    """Counts through the CPU build: (graph, query) -> (count, levels)."""
+    subprocess.run(["make", "-C", EMU_DIR, "-s", "all"], check=True)
+    path = str(tmp_path_factory.mktemp("hot") / "g.bin")
+
+    def go(g, q, vb=0, ve=None, cl=3, bounds=None, budget=1 << 30, hub=None, **env):
+        sme.write_bin(path, g)
+        e = dict(os.environ, ASAN_OPTIONS="detect_leaks=0", **{k: str(v) for k, v in env.items()})
+        if bounds is not None:
+            e["BUCKETS"] = ",".join(map(str, bounds))
+        cmd = [os.path.join(EMU_DIR, "emu_driver"), path, "6", str(q), str(cl), "1", str(vb),
+               str(g.n if ve is None else ve), str(budget)] + ([str(hub)] if hub else [])
+        r = subprocess.run(cmd, capture_output=True, text=True, env=e, timeout=600)
+        assert r.returncode == 0, r.stderr[-3000:]
+        parts = r.stdout.split()
+        out = int(parts[0].split("=")[1]), [int(x) for x in parts[1].split("=")[1].split(",")]
+        if bounds is not None:
+            return out + ([int(x) for x in r.stdout.split("buckets=")[1].split(",")],)
+        return out
+
+    return go
+
+
+@pytest.fixture(scope="module")
+def dev():
+    d = sme.Device(0, budget_bytes=2 << 30)
+    yield d
+    d.close()
+
+
+def on_gpu(dev, g, q, vb=0, ve=None, cl=3):
+    print(f"case q={q} cl={cl} n={g.n} nnz={g.nnz} [{vb},{ve})", flush=True)
+    dg = dev.upload(g)
+    r = dev.count(dg, sme.Plan(q, compress_level=cl), vb, ve)
+    dg.release()
+    return r.count, r.levels
+
+
+def union(*graphs):
+    """Disjoint union, ids in order."""
+    rp, cols, n = [np.zeros(1, dtype=np.uint64)], [], 0
+    for g in graphs:
+        rp.append(g.row_ptrs[1:] + rp[-1][-1])
+        cols.append(g.cols + np.uint32(n))
+        n += g.n
+    return sme.Graph(np.concatenate(rp), np.concatenate(cols).astype(np.uint32))
+
+
+# upper neighbourhoods of 0 .. 66 (63 and 64 fill a wave, 65 leaves it), alone and beside one another
+def small_graphs(n):
+    """Cliques whose upper neighbourhoods straddle 64, then sparse vertices up to n of them."""
+    dense = union(clique(66), clique(3), sme.gen_er(90, 1500, seed=3))
+    return union(dense, sme.gen_er(n - dense.n, 2 * n, seed=n)) if n > dense.n else dense
+
+
+@pytest.mark.parametrize("q", [0, 3, 7, 11])
+def test_emu_small_neighbourhoods(emu, q):
+    """One start vertex per wave step (few start vertices)."""
+    g = small_graphs(0)
+    want = oracle.light_count(g.row_ptrs, g.cols, q, 3)
+    assert emu(g, q) == (want[0], want[1])
+    bounds = [0, 1, 2, 65, 70, g.n]
+    want = [oracle.light_count(g.row_ptrs, g.cols, q, 3, v_begin=a, v_end=b)[0] for a, b in zip(bounds, bounds[1:])]
+    assert emu(g, q, bounds=bounds)[2] == want
+
+
+def test_emu_small_neighbourhood_groups(emu):
+    """Four start vertices per wave step, the last step part full."""
+    g = small_graphs(16387)
+    want = oracle.light_count(g.row_ptrs, g.cols, 3, 3)
+    assert emu(g, 3) == (want[0], want[1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [0, 16384, 16385, 16390])
+@pytest.mark.parametrize("q", [0, 3, 7])
+def test_small_neighbourhoods(dev, n, q):
+    g = small_graphs(n)
+    want = oracle.light_count(g.row_ptrs, g.cols, q, 3)
+    assert on_gpu(dev, g, q) == (want[0], want[1])
+    vb, ve = 7, g.n - 3
+    want = oracle.light_count(g.row_ptrs, g.cols, q, 3, v_begin=vb, v_end=ve)
+    assert on_gpu(dev, g, q, vb, ve) == (want[0], want[1])
