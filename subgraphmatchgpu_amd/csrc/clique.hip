@@ -350,7 +350,7 @@ __global__ __launch_bounds__(kThreads) void CliqueRowsKernel(CliqueArgs a) {
   const int lane = threadIdx.x & (kWave - 1);
   const uint64_t wave = (blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x) / kWave;
   const uint64_t nwaves = static_cast<uint64_t>(gridDim.x) * blockDim.x / kWave;
-  u64 c3 = 0;  // triangles, when no count kernel follows (per-edge counts)
+  u64 c3 = 0;  // triangles, when no count kernel follows (rows == nullptr)
   for (uint64_t t = wave; t < a.nitems; t += nwaves) {
     const uint64_t x = ItemVertex(a, t);
     const uint32_t v = a.verts[x];
@@ -370,7 +370,7 @@ __global__ __launch_bounds__(kThreads) void CliqueRowsKernel(CliqueArgs a) {
       const u64 w = __ballot(ok);
       if ((c & 63u) == static_cast<uint32_t>(lane)) keep = w;
       if ((c & 63u) == 63u || c + 1 == W) {
-        if (static_cast<uint32_t>(lane) <= (c & 63u))
+        if (a.rows && static_cast<uint32_t>(lane) <= (c & 63u))
           rows[static_cast<uint64_t>((c & ~63u) + lane) * d + i] = keep;
       }
       if (ok && a.tc) {
@@ -382,8 +382,9 @@ __global__ __launch_bounds__(kThreads) void CliqueRowsKernel(CliqueArgs a) {
     // edge (v, u_i): one triangle per bit of row i
     if (a.tc && lane == 0 && bits) atomicAdd(a.tc + nb + i, bits);
     if (lane == 0) c3 += bits;
+    if (!a.rows && a.bk.bounds) AddBucket(a.bk, v, lane == 0 ? bits : 0u, lane);
   }
-  if (a.tc) Flush(a.acc, 3, c3, lane);
+  if (!a.rows) Flush(a.acc, 3, c3, lane);
 }
 
 // Chunk t of a batch: largest x with chunk_first[x] - chunk_first[0] <= t.
@@ -398,6 +399,151 @@ __device__ __forceinline__ uint64_t ChunkVertex(const CliqueArgs& a, uint64_t t)
       hi = mid - 1;
   }
   return lo;
+}
+
+// Is vertex v (d upper neighbours from `base` to `vmax`) taken by
+// CliqueRowsTableKernel?
+__device__ __forceinline__ bool TableTakes(uint32_t d, uint32_t base, uint32_t vmax) {
+  return d <= kRowsTableMax && vmax - base < kRowsTableRange;
+}
+
+// Rows of a vertex v whose N+(v) spans fewer than kRowsTableRange ids: a
+// workgroup takes kTableRows rows at a time (every gridDim.y-th such part).  N+(v) becomes an LDS
+// table with, per 32 consecutive ids, the bits of those in N+(v) and the local
+// index of the first, so one 8-byte LDS load decides an entry of N+(u_i) and
+// gives its j, without the probe chains of a hash.  Each wave streams N+(u_i)
+// up to the largest value of N+(v), 128 consecutive entries per step, the next
+// step's loads issued before this step's lookups.  kMode: kRowsBits sets bit j
+// of row i (an LDS OR) and writes the row; kRowsCount counts the triangles;
+// kRowsEdges adds each triangle to its three edges' counts.
+//
+// Bound by the wave instructions of the lookups and, with per-edge counts, by
+// the device atomics (about 3.7 ms of the 6.5 ms below).  R-MAT scale 20
+// (degree-ranked; 60,395 vertices, 3.0e9 entries streamed): rows 7.0 -> 2.8 ms,
+// per-edge counts 10.4 -> 6.5 ms against the LDS hash, whose probe chains
+// diverge (64 lanes wait for the longest).  The span of 65,536 ids is the
+// largest whose table (16 KB) still lets 32 waves share a CU; on a ranked
+// graph the 60,000 vertices with d > 64 all lie within it.
+enum RowsMode : int { kRowsBits = 0, kRowsCount = 1, kRowsEdges = 2 };
+constexpr uint32_t kTableRows = 256;
+
+template <int kMode>
+__global__ __launch_bounds__(kThreads) void CliqueRowsTableKernel(CliqueArgs a) {
+  __shared__ u64 tab[kRowsTableRange / 32];  // bits 0..31: members, 32..: index of the first
+  __shared__ u64 lds_row[kMode == kRowsBits ? kWaves : 1][kRowsTableMax / 64];
+  // triangles through edge (v, u_j), two 16-bit counts per word (at most one
+  // per row of the part), flushed with one atomic per j
+  __shared__ uint32_t lds_col[kMode == kRowsEdges ? kRowsTableMax / 2 : 1];
+  const int lane = threadIdx.x & (kWave - 1);
+  const uint32_t wid = threadIdx.x / kWave;
+  u64* row = lds_row[kMode == kRowsBits ? wid : 0];
+  u64 c3 = 0;
+  for (uint64_t x = blockIdx.x; x < a.nverts; x += gridDim.x) {
+    const uint32_t v = a.verts[x];
+    const uint64_t nb = a.up[v];
+    const uint32_t d = static_cast<uint32_t>(a.rp[v + 1] - nb);
+    if (blockIdx.y * kTableRows >= d) continue;
+    const uint32_t base = a.cols[nb], vmax = a.cols[nb + d - 1];
+    if (!TableTakes(d, base, vmax)) continue;
+    const uint32_t range = vmax - base + 1;
+    const uint32_t W = (d + 63) / 64;
+    __syncthreads();  // the previous vertex's lookups are done
+    for (uint32_t k = threadIdx.x; k < (range + 31) / 32; k += kThreads) tab[k] = 0;
+    __syncthreads();
+    for (uint32_t j = threadIdx.x; j < d; j += kThreads) {
+      const uint32_t off = a.cols[nb + j] - base;
+      u64 add = 1ull << (off & 31);
+      if (j == 0 || (a.cols[nb + j - 1] - base) >> 5 != off >> 5) add |= static_cast<u64>(j) << 32;
+      atomicOr(tab + (off >> 5), add);
+    }
+    u64 mine = 0;  // triangles from v found by this lane
+    for (uint32_t r0 = blockIdx.y * kTableRows; r0 < d; r0 += gridDim.y * kTableRows) {
+      const uint32_t r1 = r0 + kTableRows < d ? r0 + kTableRows : d;
+      if (kMode == kRowsEdges)
+        for (uint32_t k = threadIdx.x; k < (d + 1) / 2; k += kThreads) lds_col[k] = 0;
+      __syncthreads();
+      // the next row's list bounds are loaded while this row streams
+      uint32_t i = r0 + wid;
+      uint64_t lb_next = 0, le_next = 0;
+      if (i < r1) {
+        const uint32_t u = a.cols[nb + i];
+        lb_next = a.up[u];
+        le_next = a.rp[u + 1];
+      }
+      for (; i < r1; i += kWaves) {
+        const uint64_t lb = lb_next;
+        const uint32_t len = static_cast<uint32_t>(le_next - lb_next);
+        if (i + kWaves < r1) {
+          const uint32_t u = a.cols[nb + i + kWaves];
+          lb_next = a.up[u];
+          le_next = a.rp[u + 1];
+        }
+        if (kMode == kRowsBits) {
+          for (uint32_t w = lane; w < W; w += kWave) row[w] = 0;
+          WaveSync();
+        }
+        const uint32_t* list = a.cols + lb;
+        constexpr uint32_t kNone = 0xffffffffu;
+        uint32_t w0 = static_cast<uint32_t>(lane) < len ? list[lane] : kNone;
+        uint32_t w1 = static_cast<uint32_t>(lane) + kWave < len ? list[lane + kWave] : kNone;
+        uint32_t bits = 0;
+        for (uint32_t e0 = 0; e0 < len; e0 += 2 * kWave) {
+          // N+(u_i) is sorted: a step starting above the largest value of N+(v)
+          // ends the row (lane 0 holds the step's first entry)
+          if (static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(w0))) > vmax) break;
+          const uint32_t x0 = w0, x1 = w1, e = e0 + static_cast<uint32_t>(lane);
+          w0 = e + 2 * kWave < len ? list[e + 2 * kWave] : kNone;
+          w1 = e + 3 * kWave < len ? list[e + 3 * kWave] : kNone;
+          // every entry lies above u_i, so above base
+          const uint32_t o0 = x0 - base, o1 = x1 - base;
+          const u64 t0 = o0 < range ? tab[o0 >> 5] : 0, t1 = o1 < range ? tab[o1 >> 5] : 0;
+  #pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const uint32_t o = h ? o1 : o0;
+            const u64 t = h ? t1 : t0;
+            if (!((t >> (o & 31)) & 1)) continue;
+            ++bits;
+            if (kMode == kRowsCount) continue;
+            const uint32_t j = static_cast<uint32_t>(t >> 32) +
+                               static_cast<uint32_t>(__popcll(t & ((1ull << (o & 31)) - 1)));
+            if (kMode == kRowsBits) atomicOr(row + (j >> 6), 1ull << (j & 63));
+            if (kMode == kRowsEdges) {
+              atomicAdd(a.tc + lb + e + h * kWave, 1u);  // edge (u_i, u_j)
+              atomicAdd(lds_col + (j >> 1), 1u << (16 * (j & 1)));  // edge (v, u_j)
+            }
+          }
+        }
+        if (kMode == kRowsBits) {
+          u64* rows = a.rows + (a.word_first[x] - a.word_first[0]);
+          WaveSync();
+          for (uint32_t w = lane; w < W; w += kWave) rows[static_cast<uint64_t>(w) * d + i] = row[w];
+          WaveSync();
+        } else if (kMode == kRowsEdges) {
+          // edge (v, u_i): one triangle per bit of row i
+          const u64 tot = WaveSum(bits);
+          if (lane == 0) {
+            if (tot) atomicAdd(a.tc + nb + i, static_cast<uint32_t>(tot));
+            c3 += tot;
+          }
+        } else {
+          mine += bits;
+        }
+      }
+      if (kMode == kRowsEdges) {
+        __syncthreads();
+        for (uint32_t j = threadIdx.x; j < d; j += kThreads) {
+          const uint32_t c = (lds_col[j >> 1] >> (16 * (j & 1))) & 0xffffu;
+          if (c) atomicAdd(a.tc + nb + j, c);
+        }
+        __syncthreads();  // before the next part clears the counts
+      }
+    }
+    if (kMode == kRowsCount) {
+      c3 += mine;
+      if (a.bk.bounds) AddBucket(a.bk, v, mine, lane);
+    }
+  }
+  if (kMode != kRowsBits) Flush(a.acc, 3, c3, lane);
 }
 
 // One workgroup per chunk of 64 rows of one vertex v.  N+(v) goes into an LDS
@@ -428,6 +574,7 @@ __global__ __launch_bounds__(kThreads) void CliqueRowsHashKernel(CliqueArgs a) {
     const uint32_t r0 = static_cast<uint32_t>(t - (a.chunk_first[x] - a.chunk_first[0])) * 64;
     const uint32_t r1 = r0 + 64 < d ? r0 + 64 : d;
     const uint64_t nb = a.up[v];
+    if (TableTakes(d, a.cols[nb], a.cols[nb + d - 1])) continue;
     u64* rows = a.rows + (a.word_first[x] - a.word_first[0]);
     __syncthreads();  // the previous chunk's lookups are done
     for (uint32_t k = threadIdx.x; k < kSlots; k += kThreads) lds_key[k] = kEmptyKey;
@@ -450,6 +597,7 @@ __global__ __launch_bounds__(kThreads) void CliqueRowsHashKernel(CliqueArgs a) {
       lb_next = a.up[u];
       le_next = a.rp[u + 1];
     }
+    u64 mine = 0;  // triangles from v found by this lane
     for (; i < r1; i += kWaves) {
       const uint64_t lb = lb_next, le = le_next;
       if (i + kWaves < r1) {
@@ -481,7 +629,7 @@ __global__ __launch_bounds__(kThreads) void CliqueRowsHashKernel(CliqueArgs a) {
           while ((k = lds_key[h]) != w && k != kEmptyKey) h = (h + 1) & (kSlots - 1);
           if (k == w) {
             const uint32_t j = lds_idx[h];
-            atomicOr(row + (j >> 6), 1ull << (j & 63));
+            if (a.rows) atomicOr(row + (j >> 6), 1ull << (j & 63));
             ++bits;
             if (a.tc) {
               atomicAdd(a.tc + e, 1u);     // edge (u_i, u_j)
@@ -491,26 +639,28 @@ __global__ __launch_bounds__(kThreads) void CliqueRowsHashKernel(CliqueArgs a) {
         }
       }
       WaveSync();
-      for (uint32_t w = lane; w < W; w += kWave) rows[static_cast<uint64_t>(w) * d + i] = row[w];
-      if (a.tc) {
-        // edge (v, u_i): one triangle per bit of row i (only the per-edge
-        // pass needs the row's popcount here; otherwise the count kernel
-        // takes it)
+      if (a.rows)
+        for (uint32_t w = lane; w < W; w += kWave) rows[static_cast<uint64_t>(w) * d + i] = row[w];
+      if (!a.rows) {
+        // edge (v, u_i): one triangle per bit of row i (with rows the count
+        // kernel takes the row's popcount)
         const u64 tot = WaveSum(bits);
         if (lane == 0) {
-          if (tot) atomicAdd(a.tc + nb + i, static_cast<uint32_t>(tot));
+          if (a.tc && tot) atomicAdd(a.tc + nb + i, static_cast<uint32_t>(tot));
           c3 += tot;
         }
+        mine += bits;
       }
       WaveSync();
     }
+    if (!a.rows && a.bk.bounds) AddBucket(a.bk, v, mine, lane);
     if (a.tc) {
       __syncthreads();
       for (uint32_t j = threadIdx.x; j < d; j += kThreads)
         if (lds_col[j]) atomicAdd(a.tc + nb + j, lds_col[j]);
     }
   }
-  if (a.tc) Flush(a.acc, 3, c3, lane);
+  if (!a.rows) Flush(a.acc, 3, c3, lane);
 }
 
 // |s & row_j| over the words of row j that can be non-zero (bits above j).
@@ -575,11 +725,9 @@ __device__ __forceinline__ u64 CountRow(const u64* rows, uint32_t d, uint32_t i,
   WaveSync();
   for (uint32_t w = lo1 + lane; w < W; w += kWave) {
     const u64 xw = ri[static_cast<uint64_t>(w) * d];
-    if (K >= 4) s1[w] = xw;
+    s1[w] = xw;
     cs->c3 += __popcll(xw);
-    if (K == 3) vk += __popcll(xw);
   }
-  if (K < 4) return vk;
   WaveSync();
   if (K == 4) {
     const u64 y = LastLevel(s1, lo1, W, d, rows, q, lane);
@@ -634,7 +782,7 @@ __device__ __forceinline__ u64 CountRow(const u64* rows, uint32_t d, uint32_t i,
 
 __device__ __forceinline__ void FlushSums(unsigned long long* acc, int K, CliqueSums* cs, int lane) {
   Flush(acc, 3, cs->c3, lane);
-  if (K >= 4) Flush(acc, 4, cs->c4, lane);
+  Flush(acc, 4, cs->c4, lane);
   if (K >= 5) Flush(acc, 5, cs->c5, lane);
   if (K >= 6) Flush(acc, 6, cs->c6, lane);
 }
@@ -642,7 +790,7 @@ __device__ __forceinline__ void FlushSums(unsigned long long* acc, int K, Clique
 // One wave per row i of a big vertex, rows in device memory.
 template <int K>
 __global__ __launch_bounds__(kThreads) void CliqueCountKernel(CliqueArgs a) {
-  constexpr int kBufs = K >= 4 ? K - 3 : 1;
+  constexpr int kBufs = K - 3;
   __shared__ u64 lds_s[kWaves][kBufs][kWordsMax];
   __shared__ uint32_t lds_q[kWaves][2 * kWave];
   const int lane = threadIdx.x & (kWave - 1);
@@ -699,6 +847,22 @@ void LaunchCliqueRows(const CliqueArgs& a, hipStream_t stream) {
   hipLaunchKernelGGL(CliqueRowsKernel, dim3(Grid(a.nitems, kWaves)), dim3(kThreads), 0, stream, a);
 }
 
+void LaunchCliqueRowsTable(const CliqueArgs& a, uint32_t dmax, hipStream_t stream) {
+  if (a.nverts == 0) return;
+  if (dmax > kRowsTableMax) dmax = kRowsTableMax;
+  // parts of one vertex run side by side where the vertices alone would not
+  // fill the chip several times over
+  uint32_t parts = (dmax + kTableRows - 1) / kTableRows;
+  if (a.nverts > 4096 && parts > 4) parts = 4;
+  const dim3 grid(Grid(a.nverts, 1), parts), block(kThreads);
+  if (a.tc)
+    hipLaunchKernelGGL(CliqueRowsTableKernel<kRowsEdges>, grid, block, 0, stream, a);
+  else if (a.rows)
+    hipLaunchKernelGGL(CliqueRowsTableKernel<kRowsBits>, grid, block, 0, stream, a);
+  else
+    hipLaunchKernelGGL(CliqueRowsTableKernel<kRowsCount>, grid, block, 0, stream, a);
+}
+
 void LaunchCliqueRowsHash(const CliqueArgs& a, bool small_table, hipStream_t stream) {
   if (a.nchunks == 0) return;
   const dim3 grid(Grid(a.nchunks, 1)), block(kThreads);
@@ -712,7 +876,6 @@ void LaunchCliqueCount(const CliqueArgs& a, hipStream_t stream) {
   if (a.nitems == 0) return;
   const dim3 grid(Grid(a.nitems, kWaves)), block(kThreads);
   switch (a.k) {
-    case 3: hipLaunchKernelGGL(CliqueCountKernel<3>, grid, block, 0, stream, a); break;
     case 4: hipLaunchKernelGGL(CliqueCountKernel<4>, grid, block, 0, stream, a); break;
     case 5: hipLaunchKernelGGL(CliqueCountKernel<5>, grid, block, 0, stream, a); break;
     case 6: hipLaunchKernelGGL(CliqueCountKernel<6>, grid, block, 0, stream, a); break;

@@ -193,6 +193,7 @@ class DevGraph {
     uint64_t* drf = nullptr;
     uint64_t* dwf = nullptr;
     uint64_t* dcf = nullptr;
+    bool wide = false;  // some of verts' N+(v) spans kRowsTableRange ids or more
   } upper;
   int device = -1;
   // hub adjacency bitmaps (nhub rows of hub_words u32 words)

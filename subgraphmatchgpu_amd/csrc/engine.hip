@@ -174,6 +174,7 @@ Status DevGraph::Upload(Context* ctx, const uint64_t* row_ptrs, const uint32_t* 
     if (dp > kLocalMax) {
       upper.huge.push_back(static_cast<uint32_t>(v));
     } else if (dp > kLocalSmall) {
+      upper.wide |= e[-1] - e[-static_cast<int64_t>(dp)] >= kRowsTableRange;
       upper.verts.push_back(static_cast<uint32_t>(v));
       upper.d.push_back(static_cast<uint32_t>(dp));
     }
@@ -1484,6 +1485,8 @@ void LocalCliqueRange(Context* ctx, const DevGraph* g, const EnginePlan* plan, u
   const uint64_t* drf = whole ? g->upper.drf : drf_local.get();
   const uint64_t* dwf = whole ? g->upper.dwf : dwf_local.get();
   const uint64_t* dcf = whole ? g->upper.dcf : dcf_local.get();
+  // some N+(v) may span more ids than the row kernel's table (or be longer)
+  const bool wide = (g->n > kRowsTableRange && g->upper.wide) || g->max_up_degree > kRowsTableMax;
   if (nbig && !whole) {
     hv.resize(nbig);
     hd.resize(nbig);
@@ -1532,7 +1535,8 @@ void LocalCliqueRange(Context* ctx, const DevGraph* g, const EnginePlan* plan, u
       uint64_t x1 = x0 + 1;
       while (x1 < nbig && wf[x1 + 1] - wf[x0] <= cap_words) ++x1;
       const uint64_t words = wf[x1] - wf[x0];
-      Buf<unsigned long long> rows(ctx, words);
+      // triangles are counted as the rows are found: nothing to keep
+      Buf<unsigned long long> rows(ctx, K > 3 ? words : 0);
       a.verts = dverts + x0;
       a.nverts = x1 - x0;
       a.nitems = rf[x1] - rf[x0];
@@ -1565,6 +1569,18 @@ void LocalCliqueRange(Context* ctx, const DevGraph* g, const EnginePlan* plan, u
           b.nitems = rf[hash_from] - rf[x0];
           LaunchCliqueRows(b, s);
         }
+        // from the first vertex that the table kernel may take
+        const uint64_t table_from = std::partition_point(hd_sorted.begin() + x0, hd_sorted.begin() + x1,
+                                                         [](uint32_t d) { return d > kRowsTableMax; }) -
+                                    hd_sorted.begin();
+        if (table_from < x1) {
+          CliqueArgs b = a;
+          b.verts = dverts + table_from;
+          b.nverts = x1 - table_from;
+          b.word_first = dwf + table_from;
+          b.rows = K > 3 ? rows.get() + (wf[table_from] - wf[x0]) : nullptr;
+          LaunchCliqueRowsTable(b, hd_sorted[table_from], s);
+        }
         for (int cls = 0; cls < 2; ++cls) {
           const uint64_t xa = cls ? small_from : hash_from, xb = cls ? x1 : small_from;
           if (xb <= xa) continue;
@@ -1575,11 +1591,11 @@ void LocalCliqueRange(Context* ctx, const DevGraph* g, const EnginePlan* plan, u
           b.word_first = dwf + xa;
           b.chunk_first = dcf + xa;
           b.nchunks = cf[xb] - cf[xa];
-          b.rows = rows.get() + (wf[xa] - wf[x0]);
-          LaunchCliqueRowsHash(b, cls == 1, s);
+          b.rows = K > 3 ? rows.get() + (wf[xa] - wf[x0]) : nullptr;
+          if (wide) LaunchCliqueRowsHash(b, cls == 1, s);
         }
       }
-      if (!tc) {
+      if (K > 3) {
         // every row word read at least once
         Timed t(ctx, s, kSlotCliqueCount, 8.0 * static_cast<double>(words), a.nitems);
         LaunchCliqueCount(a, s);

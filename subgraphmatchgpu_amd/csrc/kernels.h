@@ -371,7 +371,7 @@ struct CliqueArgs {
   uint64_t nitems;               // row_first[nverts] - row_first[0]
   const uint64_t* row_first;
   const uint64_t* word_first;
-  unsigned long long* rows;
+  unsigned long long* rows;      // nullptr (k == 3): no rows are written, the row kernels count
   // CliqueRowsKernel with a hash of N+(v) in LDS (d <= kRowsHashMax): vertex
   // t owns chunks [chunk_first[t], chunk_first[t+1]) - chunk_first[0] of 64
   // rows each
@@ -432,6 +432,12 @@ void LaunchHouseWedgeReduce(const HouseArgs& a, hipStream_t stream);
 
 void LaunchCliqueSmall(const CliqueArgs& a, hipStream_t stream);
 void LaunchCliqueRows(const CliqueArgs& a, hipStream_t stream);
+// Rows of the vertices with d <= kRowsTableMax whose N+(v) spans fewer than
+// kRowsTableRange ids (the others are left alone), from an LDS table over that
+// span; dmax: the largest d of the batch.  The hash kernel skips them.
+constexpr uint32_t kRowsTableMax = 4096;
+constexpr uint32_t kRowsTableRange = 65536;
+void LaunchCliqueRowsTable(const CliqueArgs& a, uint32_t dmax, hipStream_t stream);
 // Rows of vertices with d <= kRowsHashMax: a workgroup per chunk of 64 rows
 // keeps N+(v) as a hash (value -> local index) in LDS and streams each row
 // vertex's upper list, 64 consecutive entries per load; `small_table`: every

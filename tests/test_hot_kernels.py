@@ -98,3 +98,51 @@ def test_small_neighbourhoods(dev, n, q):
     vb, ve = 7, g.n - 3
     want = oracle.light_count(g.row_ptrs, g.cols, q, 3, v_begin=vb, v_end=ve)
     assert on_gpu(dev, g, q, vb, ve) == (want[0], want[1])
+
+
+def fan(n, d, stride, extra, seed):
+    """Vertex 0 joined to every stride-th vertex up to d of them, plus random edges among those: one
+    upper neighbourhood of d vertices spanning about d * stride ids."""
+    rng = np.random.default_rng(seed)
+    ends = np.arange(1, 1 + d) * stride
+    adj = [[] for _ in range(n)]
+    pairs = {(0, int(e)) for e in ends}
+    for a, b in rng.integers(0, d, size=(extra, 2)):
+        if a != b:
+            pairs.add((int(ends[min(a, b)]), int(ends[max(a, b)])))
+    for a, b in pairs:
+        adj[a].append(b)
+        adj[b].append(a)
+    return sme.from_adjacency(adj)
+
+
+# (d, stride): the row table takes d <= 4,096 and a span below 65,536 ids, the hash (tables for d <= 512
+# and d <= 4,096) wider spans, the search longer lists; 256 rows per part
+ROW_SHAPES = [(65, 1), (255, 1), (256, 2), (257, 1), (1024, 1), (1025, 1), (90, 728), (90, 729), (90, 737),
+              (513, 150), (4096, 1), (4100, 1)]
+
+
+@pytest.mark.parametrize("d,stride", [(257, 1), (90, 728), (90, 737), (1025, 1)])
+def test_emu_row_shapes(emu, d, stride):
+    g = fan(d * stride + 2, d, stride, 3 * d, d)
+    for q in (0, 3):
+        want = oracle.light_count(g.row_ptrs, g.cols, q, 3)
+        assert emu(g, q) == (want[0], want[1])
+    bounds = [0, 1, g.n // 2, g.n]
+    want = [oracle.light_count(g.row_ptrs, g.cols, 0, 3, v_begin=a, v_end=b)[0] for a, b in zip(bounds, bounds[1:])]
+    assert emu(g, 0, bounds=bounds)[2] == want
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,stride", ROW_SHAPES)
+def test_row_shapes(dev, d, stride):
+    g = fan(d * stride + 2, d, stride, 12 * d, d + stride)
+    for q in (0, 2, 3, 7):
+        want = oracle.light_count(g.row_ptrs, g.cols, q, 3)
+        assert on_gpu(dev, g, q) == (want[0], want[1])
+    bounds = [0, 1, g.n // 2, g.n]
+    dg = dev.upload(g)
+    for q in (0, 3):
+        want = [oracle.light_count(g.row_ptrs, g.cols, q, 3, v_begin=a, v_end=b)[0] for a, b in zip(bounds, bounds[1:])]
+        assert dev.count_buckets(dg, sme.Plan(q), bounds)[0].tolist() == want
+    dg.release()
