@@ -39,7 +39,7 @@ enum KernelSlot : int {
   kSlotCliqueRows,  // clique counting, bit rows of larger neighbourhoods
   kSlotCliqueCount, // clique counting over those rows
   kSlotHouseMirror, // house: mirrored triangle counts and wedge loads
-  kSlotHouseWedge,  // house: 4-cycle wedges per apex
+  kSlotHouseWedge,  // house and 4-cycle: wedges per apex or start vertex
   kSlotMisc,
   kNumSlots
 };
@@ -180,6 +180,8 @@ class DevGraph {
   // isomorphic degree-ranked copy (RankByDegree), or nullptr
   DevGraph* ranked = nullptr;
   bool self_loops = false;
+  bool symmetric = false;      // every entry (v, u) has its mirror (u, v)
+  bool check_symmetry = true;  // let Upload find out (off for a ranked copy)
   uint64_t max_degree = 0;     // largest |N(v)|
   uint64_t max_up_degree = 0;  // largest |N+(v)| (neighbours above v)
   // Built at upload for the clique bitmap path over all start vertices:

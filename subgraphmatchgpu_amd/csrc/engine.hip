@@ -268,6 +268,20 @@ Status DevGraph::Upload(Context* ctx, const uint64_t* row_ptrs, const uint32_t* 
     return kErrOom;
   }
   LaunchUpperStart(rp, cols, nv, up, ctx->stream());
+  // (an isomorphic copy is as symmetric as its original)
+  if (check_symmetry && !loops) {
+    if (uint32_t* flag = static_cast<uint32_t*>(ctx->Alloc(sizeof(uint64_t)))) {
+      LaunchFill32(flag, 1, 0, ctx->stream());
+      LaunchAsymmetric(rp, cols, nv, ne, flag, ctx->stream());
+      uint32_t* pin = reinterpret_cast<uint32_t*>(ctx->pinned());
+      const hipError_t e = hipMemcpyAsync(pin, flag, sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream());
+      const hipError_t f = hipStreamSynchronize(ctx->stream());
+      ctx->Free(flag, sizeof(uint64_t));
+      SME_HIP(e);
+      SME_HIP(f);
+      symmetric = *pin == 0;
+    }
+  }
   SME_HIP(hipStreamSynchronize(ctx->stream()));
   if (ctx->rank_order && nv) {
     std::vector<uint64_t> rrp;
@@ -280,6 +294,8 @@ Status DevGraph::Upload(Context* ctx, const uint64_t* row_ptrs, const uint32_t* 
       ~Restore() { c->rank_order = true; }
     } restore{ctx};
     ctx->rank_order = false;
+    ranked->check_symmetry = false;
+    ranked->symmetric = symmetric;
     const Status s = ranked->Upload(ctx, rrp.data(), rcols.data(), nv, ne, err);
     if (s != kOk) return s;
   }
@@ -1816,6 +1832,68 @@ void LocalHouse(Context* ctx, const DevGraph* g, uint64_t* count, RunStats* st) 
 }
 
 
+// ---------------------------------------------------------------------------
+// 4-cycle and house over any start range (and per bucket) from wedges per
+// start vertex (wedge.hip).  Level outputs follow from sums over the start
+// vertices: the frames of the plan before its count are start vertices a,
+// edges (a, b) with b > a, wedges, or edges with a further neighbour of a.
+bool WedgeApplies(const Context* ctx, const DevGraph* g, const EnginePlan* plan) {
+  return !ctx->tuning.clique_level_engine && !ctx->tuning.census_level_engine && plan->algo == kAlgoLight &&
+         plan->enable_ordering && g->symmetric && !g->self_loops;
+}
+
+bool SquareApplies(const Context* ctx, const DevGraph* g, const EnginePlan* plan, uint64_t range) {
+  return plan->query_type == 1 && WedgeApplies(ctx, g, plan) && g->max_up_degree <= kWedgeDegreeMax &&
+         4 * range + (1 << 12) <= ctx->RunAvailable() / 4;
+}
+
+constexpr int kWedgeAcc = 6;
+
+// Shared by both: argument block, accumulators [acc, nheavy, next], and the
+// read of acc at the end.
+WedgeArgs WedgeBase(const DevGraph* g, uint32_t vb, uint32_t ve, const BucketRef& bk, unsigned long long* acc) {
+  WedgeArgs w{};
+  w.rp = g->rp;
+  w.cols = g->cols;
+  w.up = g->up;
+  w.n = static_cast<uint32_t>(g->n);
+  w.v_begin = vb;
+  w.v_end = ve;
+  w.acc = acc;
+  w.next = acc + kWedgeAcc + 1;
+  w.bk = bk;
+  return w;
+}
+
+void LocalSquare(Context* ctx, const DevGraph* g, const EnginePlan* plan, uint32_t vb, uint32_t ve,
+                 const BucketRef& bk, uint64_t* count, uint64_t* levels, RunStats* st) {
+  hipStream_t s = ctx->stream();
+  *st = RunStats{};
+  st->batches = 1;
+  Buf<unsigned long long> acc(ctx, kWedgeAcc + 2);
+  Buf<uint32_t> heavy(ctx, ve - vb);
+  LaunchFill64(reinterpret_cast<uint64_t*>(acc.get()), kWedgeAcc + 2, 0, s);
+  WedgeArgs w = WedgeBase(g, vb, ve, bk, acc.get());
+  w.heavy = heavy.get();
+  w.nheavy = acc.get() + kWedgeAcc;
+  {
+    Timed t(ctx, s, kSlotHouseWedge, 24.0 * (ve - vb), ve - vb);
+    LaunchSquareLight(w, s);
+    LaunchWedgeTiles(w, kWedgeSquare, s);
+  }
+  uint64_t* pin = ctx->pinned();
+  SME_HIP(hipMemcpyAsync(pin, acc.get(), kWedgeAcc * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
+  SME_HIP(hipStreamSynchronize(s));
+  st->d2h_syncs++;
+  *count = pin[0];
+  if (levels)
+    for (int L = 0; L < plan->nops; ++L) {
+      const OpDesc& o = plan->ops[L];
+      const bool set = o.kind == kCompute || o.kind == kMaterialize;
+      levels[L] = set && o.u == 0 ? ve - vb : set && o.u == 1 ? pin[1] : set && o.u == 2 ? pin[2] : pin[0];
+    }
+}
+
 // Diamond (Q2, LIGHT, ordering on) over all start vertices: every level
 // output is a whole-graph count -- start vertices n, edges m, triangles
 // through an edge summed over edges (3T), and the count D = sum_e
@@ -1930,6 +2008,8 @@ Status RunPlan(Context* ctx, const DevGraph* g, const EnginePlan* plan, uint32_t
     } else if (full && LocalDiamondApplies(ctx, dg, plan) &&
                census([&] { LocalDiamond(ctx, dg, plan, count, level_counts, &st); })) {
       on_ranked = dg != g;
+    } else if (SquareApplies(ctx, rg, plan, v_end - v_begin)) {
+      LocalSquare(ctx, rg, plan, v_begin, v_end, BucketRef{}, count, level_counts, &st);
     } else if (LocalCliqueApplies(ctx, plan)) {
       LocalClique(ctx, rg, plan, v_begin, v_end, BucketRef{}, count, level_counts, &st);
     } else {
@@ -2020,13 +2100,15 @@ Status RunPlanBuckets(Context* ctx, const DevGraph* g, const EnginePlan* plan, c
     Buf<uint32_t> table(ctx, use_table ? range : 0);
     if (use_table) LaunchBucketTable(dbounds.get(), nbuckets, range, table.get(), ctx->stream());
     RunStats st;
-    if (LocalCliqueApplies(ctx, plan)) {
-      BucketRef bk{};
-      bk.bounds = dbounds.get();
-      bk.nbuckets = nbuckets;
-      bk.counts = dcounts.get();
-      bk.table = table.get();
-      bk.base = bounds[0];
+    BucketRef bk{};
+    bk.bounds = dbounds.get();
+    bk.nbuckets = nbuckets;
+    bk.counts = dcounts.get();
+    bk.table = table.get();
+    bk.base = bounds[0];
+    if (SquareApplies(ctx, g, plan, range)) {
+      LocalSquare(ctx, g, plan, bounds[0], bounds[nbuckets], bk, count, level_counts, &st);
+    } else if (LocalCliqueApplies(ctx, plan)) {
       LocalClique(ctx, g, plan, bounds[0], bounds[nbuckets], bk, count, level_counts, &st);
     } else {
       Runner r(ctx, g, plan);

@@ -447,6 +447,52 @@ constexpr uint32_t kRowsHashSmall = 512;
 void LaunchCliqueRowsHash(const CliqueArgs& a, bool small_table, hipStream_t stream);
 void LaunchCliqueCount(const CliqueArgs& a, hipStream_t stream);
 
+// ---------------------------------------------------------------------------
+// Wedges counted per start vertex (wedge.hip).  On a symmetric graph without
+// self-loops the patterns built on 4-cycles need only, for a start vertex a
+// and every vertex w, the number c(a, w) of middles b with a - b - w.
+//
+// 4-cycle from its lowest vertex a (match order 0, 1, 2, 3): middles b > a,
+// ends w > a, count = sum_w c (c - 1) / 2.
+//
+// House from a = query vertex 1 (match order 1, 2, 3, 0, 4; b = query vertex 2
+// > a, apex x, 4-cycle a - b - w - v3 - a): with all middles and ends,
+//   houses(a) = sum_{b > a} [ t(a, b) sum_{w in N(b), w != a} (c(a, w) - 1)
+//                 - sum_{x in N(a) and N(b)} (t(b, x) - 1 + c(a, x) - 1) ]:
+// t(a, b) apexes times the 4-cycles through (a, b), less the pairs whose apex
+// is one of the two other vertices of the 4-cycle.
+constexpr uint32_t kWedgeDegreeMax = 65535;  // c fits 16 bits
+enum WedgeUse : int { kWedgeSquare = 0, kWedgeHouse = 1 };
+struct WedgeArgs {
+  const uint64_t* rp;
+  const uint32_t* cols;
+  const uint64_t* up;
+  uint32_t n;
+  uint32_t v_begin, v_end;      // start vertices
+  uint32_t group;               // consecutive start vertices per wave (set by the launcher)
+  // LaunchSquareLight: heavy[0 .. *nheavy) receives the start vertices it leaves to
+  // LaunchWedgeTiles.  LaunchWedgeTiles: heavy == nullptr: every start vertex.
+  uint32_t* heavy;
+  unsigned long long* nheavy;
+  unsigned long long* next;     // work counter of LaunchWedgeTiles, zero
+  uint32_t ntiles;              // id tiles a start vertex is walked in (set by the launcher)
+  const uint32_t* t;            // house: triangles per CSR entry, both directions
+  // acc[0] += count; acc[1] += sum of |N+(a)|; square: acc[2] += wedges a - b - w;
+  // house: acc[2] += sum of d(a), acc[3] += sum_{b > a} t(a, b),
+  // acc[4] += sum of |N+(a)| (d(a) - 1), acc[5] += sum_{b > a} t(a, b) (d(a) - 2)
+  unsigned long long* acc;
+  BucketRef bk;
+};
+// 4-cycles of the start vertices with few wedges (one wave each) and acc[1],
+// acc[2] of all of them.
+void LaunchSquareLight(const WedgeArgs& a, hipStream_t stream);
+// Counts of `use` from heavy[] (or all start vertices): a workgroup per start
+// vertex and tile of ids keeps c in LDS.
+void LaunchWedgeTiles(const WedgeArgs& a, int use, hipStream_t stream);
+// *flag (zero before) becomes 1 unless every entry (v, u) has its mirror (u, v).
+void LaunchAsymmetric(const uint64_t* rp, const uint32_t* cols, uint64_t n, uint64_t nnz, uint32_t* flag,
+                      hipStream_t stream);
+
 // Exclusive scan: out[i] = sum(in[0..i)), out[n] = total.  `tmp` needs
 // ScanTempWords(n) u64 words.  out may alias in.
 size_t ScanTempWords(uint64_t n);

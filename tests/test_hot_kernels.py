@@ -146,3 +146,71 @@ def test_row_shapes(dev, d, stride):
         want = [oracle.light_count(g.row_ptrs, g.cols, q, 3, v_begin=a, v_end=b)[0] for a, b in zip(bounds, bounds[1:])]
         assert dev.count_buckets(dg, sme.Plan(q), bounds)[0].tolist() == want
     dg.release()
+
+
+def hub_and_sparse(n, d, m, seed):
+    """A vertex of degree d spread over [0, n) on top of G(n, m)."""
+    g = sme.gen_er(n, m, seed=seed)
+    src = np.repeat(np.arange(n), np.diff(g.row_ptrs.astype(np.int64)))
+    hub = n // 3
+    ends = np.unique(np.linspace(0, n - 1, d).astype(np.int64))
+    ends = ends[ends != hub]
+    a = np.concatenate([src, np.full(ends.size, hub), ends])
+    b = np.concatenate([g.cols.astype(np.int64), ends, np.full(ends.size, hub)])
+    key = np.unique(a * n + b)
+    rp = np.searchsorted(key, np.arange(n + 1) * n).astype(np.uint64)
+    return sme.Graph(rp, (key % n).astype(np.uint32))
+
+
+def one_way(g):
+    """The same lists without the mirror of every third entry."""
+    src = np.repeat(np.arange(g.n), np.diff(g.row_ptrs.astype(np.int64)))
+    keep = np.arange(g.nnz) % 3 != 0
+    rp = np.concatenate([[0], np.cumsum(np.bincount(src[keep], minlength=g.n))]).astype(np.uint64)
+    return sme.Graph(rp, g.cols[keep])
+
+
+# byte counters over a span (one pass, two passes), hash beyond two spans, 16,384-id and 65,536-id
+# tiles (one and two), start vertices with over 64 middles or 4,096 list entries, and a graph whose
+# entries have no mirrors (level engine)
+def wedge_graphs(small):
+    out = {"rmat7": sme.gen_rmat(7, 6, seed=3), "span": sme.gen_er(4500, 9000, seed=2),
+           "one_way": one_way(sme.gen_rmat(7, 6, seed=4)), "k66": clique(66)}
+    if small:
+        return out
+    return dict(out, rmat12=sme.gen_rmat(12, 16, seed=5), hash=sme.gen_er(16384, 60000, seed=6),
+                tile=hub_and_sparse(16385, 5000, 60000, 7), tiles=hub_and_sparse(65537, 40000, 100000, 8),
+                two_tiles=hub_and_sparse(70001, 3000, 300000, 9))
+
+
+@pytest.mark.parametrize("name", list(wedge_graphs(True)))
+@pytest.mark.parametrize("q", [1])
+def test_emu_wedges(emu, name, q):
+    g = wedge_graphs(True)[name]
+    for cl in (0, 3):
+        want = oracle.light_count(g.row_ptrs, g.cols, q, cl)
+        assert emu(g, q, cl=cl) == (want[0], want[1])
+    vb, ve = g.n // 5, g.n // 2
+    want = oracle.light_count(g.row_ptrs, g.cols, q, 3, v_begin=vb, v_end=ve)
+    assert emu(g, q, vb, ve) == (want[0], want[1])
+    bounds = [1, 2, g.n // 3, g.n // 3, g.n]
+    want = [oracle.light_count(g.row_ptrs, g.cols, q, 3, v_begin=a, v_end=b)[0] for a, b in zip(bounds, bounds[1:])]
+    assert emu(g, q, bounds=bounds)[2] == want
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", list(wedge_graphs(False)))
+@pytest.mark.parametrize("q", [1])
+def test_wedges(dev, name, q):
+    g = wedge_graphs(False)[name]
+    for cl in range(4):
+        want = oracle.light_count(g.row_ptrs, g.cols, q, cl)
+        assert on_gpu(dev, g, q, cl=cl) == (want[0], want[1])
+    vb, ve = g.n // 5, g.n // 2
+    want = oracle.light_count(g.row_ptrs, g.cols, q, 3, v_begin=vb, v_end=ve)
+    assert on_gpu(dev, g, q, vb, ve) == (want[0], want[1])
+    bounds = [1, 2, g.n // 3, g.n // 3, g.n]
+    dg = dev.upload(g)
+    got = dev.count_buckets(dg, sme.Plan(q), bounds)[0].tolist()
+    dg.release()
+    assert got == [oracle.light_count(g.row_ptrs, g.cols, q, 3, v_begin=a, v_end=b)[0] for a, b in zip(bounds, bounds[1:])]
