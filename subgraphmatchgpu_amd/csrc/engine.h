@@ -184,6 +184,9 @@ class DevGraph {
   bool check_symmetry = true;  // let Upload find out (off for a ranked copy)
   uint64_t max_degree = 0;     // largest |N(v)|
   uint64_t max_up_degree = 0;  // largest |N+(v)| (neighbours above v)
+  // house_work[v]: sum of |N+(u)| |N(u)| over u < v, the (edge, further
+  // neighbour) pairs that house counts from those start vertices look at
+  std::vector<uint64_t> house_work;
   // Built at upload for the clique bitmap path over all start vertices:
   // the vertices with kLocalSmall < |N+(v)| <= kLocalMax in decreasing
   // |N+(v)| (ties by id) with prefix sums of their rows, row words and

@@ -3,10 +3,9 @@
 // Passes over a degree-ranked graph without self-loops:
 //   1. triangles per edge: the clique row kernels with CliqueArgs::tc fill t
 //      for every upper entry (an entry of some N+(x));
-//   2. HouseMirrorKernel: one wave per vertex u gives each lower entry
-//      (u -> v, v < u) the t of its mirror (v -> u), adds up u's wedge load
-//      (the entries of each N(v) below u) and sums t(t-1) over u's upper
-//      entries;
+//   2. HouseMirrorKernel gives each lower entry (u -> v, v < u) the t of its
+//      mirror (v -> u), adds up u's wedge load (the entries of each N(v) below
+//      u) and sums t(t-1) over the upper entries;
 //   3. wedges: apexes with a load of at most kHouseHashMax are walked by one
 //      wave each into an LDS hash table (HouseWedgeHashKernel); heavier ones
 //      in groups, one dense u64 array over w per apex (HouseWedgeDenseKernel,
@@ -18,13 +17,13 @@
 // every (v1, v2, v3) path; this pass reaches the same count from per-edge
 // triangle counts and a degree-ordered 4-cycle walk.
 #include "kernels.h"
+#include "wave.h"
 
 namespace sme {
 
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kWave = 64;
 constexpr int kWaves = kThreads / kWave;
 constexpr uint64_t kMaxGrid = 16384;
 constexpr uint32_t kHashSlots = 2 * kHouseHashMax;  // at most half full
@@ -41,20 +40,8 @@ uint64_t Grid(uint64_t n, uint64_t per_block) {
   return g > kMaxGrid ? kMaxGrid : g;
 }
 
-__device__ __forceinline__ void Sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-__device__ __forceinline__ u64 Sum64(u64 v) {
-#pragma unroll
-  for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return v;
-}
-
 __device__ __forceinline__ void Flush(unsigned long long* acc, int j, u64 v, int lane) {
-  v = Sum64(v);
+  v = WaveSum(v);
   if (lane == 0 && v) atomicAdd(acc + j, v);
 }
 
@@ -77,28 +64,52 @@ __device__ __forceinline__ u64 Pairs(u64 p) {
 }
 
 // ---------------------------------------------------------------------------
+// 64 consecutive entries per wave; a lane finds its row u between those of the
+// wave's first and last entry.  Bound by the latency of the searches: 4.7 ms
+// with one wave per row (R-MAT scale 19, edge factor 32: half the rows hold a
+// few entries), 1.5 ms flat.
 __global__ __launch_bounds__(kThreads) void HouseMirrorKernel(HouseArgs a) {
   const int lane = threadIdx.x & (kWave - 1);
   const uint64_t wave = (blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x) / kWave;
   const uint64_t nwaves = static_cast<uint64_t>(gridDim.x) * blockDim.x / kWave;
+  // last row in [lo, hi] starting at or before entry e
+  auto row_of = [&](uint64_t e, uint64_t lo, uint64_t hi) {
+    while (lo < hi) {
+      const uint64_t mid = (lo + hi + 1) >> 1;
+      if (a.rp[mid] <= e)
+        lo = mid;
+      else
+        hi = mid - 1;
+    }
+    return lo;
+  };
+  BucketRef rows{};  // wedge loads: one "bucket" per row
+  rows.counts = a.load;
+  BucketAcc run{kNoBucket, 0};
   u64 sq = 0;
-  for (uint64_t u = wave; u < a.n; u += nwaves) {
-    const uint64_t b = a.rp[u], m = a.up[u], e = a.rp[u + 1];
-    u64 load = 0;
-    for (uint64_t k = b + lane; k < m; k += kWave) {
-      const uint32_t v = a.cols[k];
-      // u sits in N+(v); the entries of N(v) before it are v's neighbours below u
-      const uint64_t pos = Lower(a.cols, a.up[v], a.rp[v + 1], static_cast<uint32_t>(u));
-      a.t[k] = pos < a.rp[v + 1] && a.cols[pos] == u ? a.t[pos] : 0u;
-      load += pos - a.rp[v];
+  for (uint64_t e0 = wave * kWave; e0 < a.nnz; e0 += nwaves * kWave) {
+    const uint64_t e1 = e0 + kWave < a.nnz ? e0 + kWave : a.nnz;
+    const uint64_t r0 = row_of(e0, 0, a.n - 1);
+    const uint64_t r1 = row_of(e1 - 1, r0, a.n - 1);
+    const uint64_t k = e0 + lane;
+    u64 key = kNoBucket, load = 0;
+    if (k < e1) {
+      const uint64_t u = row_of(k, r0, r1);
+      if (k >= a.up[u]) {
+        const u64 x = a.t[k];
+        sq += x * (x ? x - 1 : 0);
+      } else {
+        const uint32_t v = a.cols[k];
+        // u sits in N+(v); the entries of N(v) before it are v's neighbours below u
+        const uint64_t ve = a.rp[v + 1], pos = Lower(a.cols, a.up[v], ve, static_cast<uint32_t>(u));
+        a.t[k] = pos < ve && a.cols[pos] == u ? a.t[pos] : 0u;
+        load = pos - a.rp[v];
+      }
+      key = u;
     }
-    for (uint64_t k = m + lane; k < e; k += kWave) {
-      const u64 x = a.t[k];
-      sq += x * (x ? x - 1 : 0);
-    }
-    load = Sum64(load);
-    if (lane == 0) a.load[u] = load;
+    if (a.load) BucketAccAdd(rows, &run, key, load);
   }
+  if (a.load) BucketFlush(rows, &run);
   Flush(a.acc, 1, sq, lane);
 }
 
@@ -137,7 +148,7 @@ __global__ __launch_bounds__(kThreads) void HouseWedgeHashKernel(HouseArgs a) {
   u64 sum = 0;
   for (uint64_t x = wave; x < a.napex; x += nwaves) {
     const uint32_t u = a.apex[x];
-    Sync();
+    WaveSync();
     for (uint64_t k = a.rp[u]; k < a.up[u]; ++k) {
       const uint32_t v = a.cols[k];
       const u64 tuv = a.t[k];
@@ -156,7 +167,7 @@ __global__ __launch_bounds__(kThreads) void HouseWedgeHashKernel(HouseArgs a) {
         }
       }
     }
-    Sync();
+    WaveSync();
     for (uint32_t j = lane; j < kHashSlots; j += kWave) {
       if (key[j] != kEmpty) {
         sum += Pairs(val[j]);
@@ -251,8 +262,9 @@ __global__ __launch_bounds__(kThreads) void HouseWedgeReduceKernel(HouseArgs a) 
 }  // namespace
 
 void LaunchHouseMirror(const HouseArgs& a, hipStream_t stream) {
-  if (a.n == 0) return;
-  hipLaunchKernelGGL(HouseMirrorKernel, dim3(Grid(a.n, kWaves)), dim3(kThreads), 0, stream, a);
+  if (a.nnz == 0) return;
+  const uint64_t need = Grid(a.nnz, kThreads);
+  hipLaunchKernelGGL(HouseMirrorKernel, dim3(need < 4096 ? need : 4096), dim3(kThreads), 0, stream, a);
 }
 
 void LaunchEdgePairs(const HouseArgs& a, hipStream_t stream) {

@@ -403,8 +403,9 @@ struct HouseArgs {
   const uint32_t* cols;
   const uint64_t* up;
   uint64_t n;
+  uint64_t nnz;
   uint32_t* t;                  // per CSR entry: triangles through its edge
-  unsigned long long* load;     // HouseMirrorKernel: wedges with apex u
+  unsigned long long* load;     // HouseMirrorKernel: wedges with apex u (zero before; nullptr: not wanted)
   unsigned long long* acc;      // acc[0] += sum (c - 1) s; acc[1] += sum_e t(e) (t(e) - 1)
   // wedge kernels: apex vertices (HouseWedgeHashKernel: load <= kHouseHashMax)
   const uint32_t* apex;
@@ -420,8 +421,8 @@ struct HouseArgs {
   uint32_t* touched;            // napex x n
   unsigned long long* ntouched; // napex
 };
-// Lower CSR entries (v < u) take t from their mirror in N+(v); load[u] and
-// acc[1] as above.  The upper entries' t must be complete.
+// Lower CSR entries (v < u) take t from their mirror in N+(v); load[u] (added
+// to) and acc[1] as above.  The upper entries' t must be complete.
 void LaunchHouseMirror(const HouseArgs& a, hipStream_t stream);
 // Over the upper entries of every vertex: acc[0] += t, acc[1] += t(t-1)/2
 // (the diamonds on that edge: two triangles sharing it).

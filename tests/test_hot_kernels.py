@@ -175,16 +175,16 @@ def one_way(g):
 # entries have no mirrors (level engine)
 def wedge_graphs(small):
     out = {"rmat7": sme.gen_rmat(7, 6, seed=3), "span": sme.gen_er(4500, 9000, seed=2),
-           "one_way": one_way(sme.gen_rmat(7, 6, seed=4)), "k66": clique(66)}
+           "one_way": one_way(sme.gen_rmat(7, 6, seed=4)), "k12": clique(12)}
     if small:
         return out
-    return dict(out, rmat12=sme.gen_rmat(12, 16, seed=5), hash=sme.gen_er(16384, 60000, seed=6),
-                tile=hub_and_sparse(16385, 5000, 60000, 7), tiles=hub_and_sparse(65537, 40000, 100000, 8),
+    return dict(out, k66=clique(66), rmat12=sme.gen_rmat(12, 16, seed=5), hash=sme.gen_er(16384, 60000, seed=6),
+                tile=hub_and_sparse(16385, 5000, 60000, 7), tiles=hub_and_sparse(65537, 12000, 100000, 8),
                 two_tiles=hub_and_sparse(70001, 3000, 300000, 9))
 
 
 @pytest.mark.parametrize("name", list(wedge_graphs(True)))
-@pytest.mark.parametrize("q", [1])
+@pytest.mark.parametrize("q", [1, 4])
 def test_emu_wedges(emu, name, q):
     g = wedge_graphs(True)[name]
     for cl in (0, 3):
@@ -200,7 +200,7 @@ def test_emu_wedges(emu, name, q):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("name", list(wedge_graphs(False)))
-@pytest.mark.parametrize("q", [1])
+@pytest.mark.parametrize("q", [1, 4])
 def test_wedges(dev, name, q):
     g = wedge_graphs(False)[name]
     for cl in range(4):
