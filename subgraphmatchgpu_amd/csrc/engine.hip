@@ -1757,39 +1757,56 @@ void LocalHouse(Context* ctx, const DevGraph* g, uint64_t* count, RunStats* st) 
   LaunchFill64(reinterpret_cast<uint64_t*>(load.get()), n, 0, s);
   EdgeTriangles(ctx, g, t.get(), load.get(), acc.get(), st);
   HouseArgs h = HouseBase(g, t.get(), load.get(), acc.get());
-  std::vector<unsigned long long> hl(n);
-  std::vector<uint64_t> hrp(n + 1), hup(n);
-  SME_HIP(hipMemcpyAsync(hl.data(), load.get(), n * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
-  SME_HIP(hipMemcpyAsync(hrp.data(), g->rp, (n + 1) * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
-  SME_HIP(hipMemcpyAsync(hup.data(), g->up, n * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
-  SME_HIP(hipStreamSynchronize(s));
-  st->d2h_syncs++;
-  std::vector<uint32_t> light, heavy;
-  double wedges = 0;
-  for (uint64_t u = 0; u < n; ++u) {
-    if (!hl[u]) continue;
-    wedges += static_cast<double>(hl[u]);
-    (hl[u] <= kHouseHashMax ? light : heavy).push_back(static_cast<uint32_t>(u));
+  // 3a. light apexes in an LDS hash, heavier ones over tiles of ids
+  Buf<unsigned long long> lists(ctx, 3);
+  LaunchFill64(reinterpret_cast<uint64_t*>(lists.get()), 3, 0, s);
+  std::vector<unsigned long long> hl;
+  std::vector<uint64_t> hrp, hup;
+  {
+    Buf<uint32_t> light(ctx, n), tiled(ctx, n);
+    h.light = light.get();
+    h.nlight = lists.get();
+    h.tiled = tiled.get();
+    h.ntiled = lists.get() + 1;
+    LaunchHouseApexes(h, s);
+    {
+      // per wedge: the entry w and its t (the number is not known here)
+      Timed tm(ctx, s, kSlotHouseWedge, 0, 0);
+      LaunchHouseWedgeHash(h, s);
+    }
+    WedgeArgs w{};
+    w.rp = g->rp;
+    w.cols = g->cols;
+    w.up = g->up;
+    w.n = static_cast<uint32_t>(n);
+    w.v_end = static_cast<uint32_t>(n);
+    w.heavy = tiled.get();
+    w.nheavy = lists.get() + 1;
+    w.next = lists.get() + 2;
+    w.t = t.get();
+    w.acc = acc.get();
+    {
+      Timed tm(ctx, s, kSlotHouseWedge, 0, 0);
+      LaunchWedgeTiles(w, kWedgeApex, s);
+    }
+    if (g->max_degree > kWedgeDegreeMax) {
+      hl.resize(n);
+      hrp.resize(n + 1);
+      hup.resize(n);
+      SME_HIP(hipMemcpyAsync(hl.data(), load.get(), n * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
+      SME_HIP(hipMemcpyAsync(hrp.data(), g->rp, (n + 1) * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
+      SME_HIP(hipMemcpyAsync(hup.data(), g->up, n * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
+      SME_HIP(hipStreamSynchronize(s));
+      st->d2h_syncs++;
+    }
   }
+  std::vector<uint32_t> heavy;
+  for (uint64_t u = 0; u < hl.size(); ++u)
+    if (hl[u] > kHouseHashMax && hup[u] - hrp[u] > kWedgeDegreeMax) heavy.push_back(static_cast<uint32_t>(u));
   std::sort(heavy.begin(), heavy.end(), [&](uint32_t a, uint32_t b) {
     return hl[a] != hl[b] ? hl[a] > hl[b] : a < b;
   });
-  // 3a. light apexes: one wave each, LDS hash
-  if (!light.empty()) {
-    Buf<uint32_t> d(ctx, light.size());
-    SME_HIP(hipMemcpyAsync(d.get(), light.data(), light.size() * sizeof(uint32_t), hipMemcpyHostToDevice, s));
-    h.apex = d.get();
-    h.napex = light.size();
-    double lw = 0;
-    for (uint32_t u : light) lw += static_cast<double>(hl[u]);
-    {
-      // per wedge: the entry w and its t
-      Timed tm(ctx, s, kSlotHouseWedge, 8.0 * lw, static_cast<uint64_t>(lw));
-      LaunchHouseWedgeHash(h, s);
-    }
-    SME_HIP(hipStreamSynchronize(s));
-  }
-  // 3b. heavy apexes: groups of dense per-apex arrays over w
+  // 3b. apexes whose c may not fit 16 bits: groups of dense per-apex arrays over w
   if (!heavy.empty()) {
     const uint64_t per_slot = 12 * n;  // u64 accumulator + u32 touched entry per w
     const uint64_t fit = static_cast<uint64_t>(0.5 * static_cast<double>(ctx->RunAvailable())) / per_slot;
@@ -1839,7 +1856,6 @@ void LocalHouse(Context* ctx, const DevGraph* g, uint64_t* count, RunStats* st) 
   SME_HIP(hipMemcpyAsync(pin, acc.get(), 2 * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
   SME_HIP(hipStreamSynchronize(s));
   st->d2h_syncs++;
-  (void)wedges;
   *count = pin[0] - 2 * pin[1];
 }
 

@@ -7,10 +7,12 @@
 //      mirror (v -> u), adds up u's wedge load (the entries of each N(v) below
 //      u) and sums t(t-1) over the upper entries;
 //   3. wedges: apexes with a load of at most kHouseHashMax are walked by one
-//      wave each into an LDS hash table (HouseWedgeHashKernel); heavier ones
-//      in groups, one dense u64 array over w per apex (HouseWedgeDenseKernel,
-//      one wave per lower neighbour v, one atomic per wedge), reduced and
-//      cleared by HouseWedgeReduceKernel.
+//      wave each into an LDS hash table (HouseWedgeHashKernel); heavier ones by
+//      a workgroup per tile of ids with 16-bit LDS counters (wedge.hip); those
+//      with more than kWedgeDegreeMax lower neighbours in groups, one dense u64
+//      array over w per apex (HouseWedgeDenseKernel, one wave per lower
+//      neighbour v, one device atomic per wedge), reduced and cleared by
+//      HouseWedgeReduceKernel.
 //
 // The reference counts the house by its LIGHT plan (match order 1, 2, 3, 0, 4;
 // src/query/optimizer/LazyTraversalPlanHardCode.h:59-117), which enumerates
@@ -129,6 +131,31 @@ __global__ __launch_bounds__(kThreads) void EdgePairsKernel(HouseArgs a) {
   Flush(a.acc, 1, pairs, lane);
 }
 
+// Appends the lanes' vertices for which `take` holds: one atomic per wave.
+__device__ __forceinline__ void Append(bool take, uint32_t u, uint32_t* list, unsigned long long* count, int lane) {
+  const u64 m = __ballot(take);
+  if (!m) return;
+  u64 at = 0;
+  if (lane == 0) at = atomicAdd(count, static_cast<u64>(__popcll(m)));
+  at = __shfl(at, 0);
+  if (take) list[at + __popcll(m & __lanemask_lt())] = u;
+}
+
+__global__ __launch_bounds__(kThreads) void HouseApexKernel(HouseArgs a) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
+  for (uint64_t b = blockIdx.x * static_cast<uint64_t>(blockDim.x) + (threadIdx.x - lane); b < a.n; b += stride) {
+    const uint64_t u = b + lane;
+    u64 load = 0, lower = 0;
+    if (u < a.n) {
+      load = a.load[u];
+      lower = a.up[u] - a.rp[u];
+    }
+    Append(load > 0 && load <= kHouseHashMax, static_cast<uint32_t>(u), a.light, a.nlight, lane);
+    Append(load > kHouseHashMax && lower <= kWedgeDegreeMax, static_cast<uint32_t>(u), a.tiled, a.ntiled, lane);
+  }
+}
+
 // One wave per apex u: every wedge u - v - w (v, w < u) goes into an LDS
 // hash table keyed by w (linear probing, at most half full since u's load,
 // and so its distinct w, is at most kHouseHashMax).
@@ -146,8 +173,9 @@ __global__ __launch_bounds__(kThreads) void HouseWedgeHashKernel(HouseArgs a) {
     val[j] = 0;
   }
   u64 sum = 0;
-  for (uint64_t x = wave; x < a.napex; x += nwaves) {
-    const uint32_t u = a.apex[x];
+  const u64 napex = *a.nlight;
+  for (uint64_t x = wave; x < napex; x += nwaves) {
+    const uint32_t u = a.light[x];
     WaveSync();
     for (uint64_t k = a.rp[u]; k < a.up[u]; ++k) {
       const uint32_t v = a.cols[k];
@@ -272,9 +300,16 @@ void LaunchEdgePairs(const HouseArgs& a, hipStream_t stream) {
   hipLaunchKernelGGL(EdgePairsKernel, dim3(Grid(a.n, kWaves)), dim3(kThreads), 0, stream, a);
 }
 
+void LaunchHouseApexes(const HouseArgs& a, hipStream_t stream) {
+  if (a.n == 0) return;
+  const uint64_t need = Grid(a.n, kThreads);
+  hipLaunchKernelGGL(HouseApexKernel, dim3(need < 2048 ? need : 2048), dim3(kThreads), 0, stream, a);
+}
+
 void LaunchHouseWedgeHash(const HouseArgs& a, hipStream_t stream) {
-  if (a.napex == 0) return;
-  hipLaunchKernelGGL(HouseWedgeHashKernel, dim3(Grid(a.napex, kWaves)), dim3(kThreads), 0, stream, a);
+  if (a.n == 0) return;
+  const uint64_t need = Grid(a.n, kWaves);  // (as many light apexes at most)
+  hipLaunchKernelGGL(HouseWedgeHashKernel, dim3(need < 4096 ? need : 4096), dim3(kThreads), 0, stream, a);
 }
 
 void LaunchHouseWedgeDense(const HouseArgs& a, hipStream_t stream) {

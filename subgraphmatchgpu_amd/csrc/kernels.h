@@ -407,7 +407,14 @@ struct HouseArgs {
   uint32_t* t;                  // per CSR entry: triangles through its edge
   unsigned long long* load;     // HouseMirrorKernel: wedges with apex u (zero before; nullptr: not wanted)
   unsigned long long* acc;      // acc[0] += sum (c - 1) s; acc[1] += sum_e t(e) (t(e) - 1)
-  // wedge kernels: apex vertices (HouseWedgeHashKernel: load <= kHouseHashMax)
+  // LaunchHouseApexes: light[0 .. *nlight) and tiled[0 .. *ntiled) receive the
+  // apexes with a load, up to kHouseHashMax and above; those of the latter with
+  // more than kWedgeDegreeMax lower neighbours are left out
+  uint32_t* light;
+  unsigned long long* nlight;
+  uint32_t* tiled;
+  unsigned long long* ntiled;
+  // HouseWedgeDenseKernel / HouseWedgeReduceKernel: apexes of one group
   const uint32_t* apex;
   uint64_t napex;
   // HouseWedgeDenseKernel / HouseWedgeReduceKernel: apex x accumulates in
@@ -427,6 +434,8 @@ void LaunchHouseMirror(const HouseArgs& a, hipStream_t stream);
 // Over the upper entries of every vertex: acc[0] += t, acc[1] += t(t-1)/2
 // (the diamonds on that edge: two triangles sharing it).
 void LaunchEdgePairs(const HouseArgs& a, hipStream_t stream);
+void LaunchHouseApexes(const HouseArgs& a, hipStream_t stream);
+// The wedges of the light apexes.
 void LaunchHouseWedgeHash(const HouseArgs& a, hipStream_t stream);
 void LaunchHouseWedgeDense(const HouseArgs& a, hipStream_t stream);
 void LaunchHouseWedgeReduce(const HouseArgs& a, hipStream_t stream);
@@ -463,7 +472,11 @@ void LaunchCliqueCount(const CliqueArgs& a, hipStream_t stream);
 // t(a, b) apexes times the 4-cycles through (a, b), less the pairs whose apex
 // is one of the two other vertices of the 4-cycle.
 constexpr uint32_t kWedgeDegreeMax = 65535;  // c fits 16 bits
-enum WedgeUse : int { kWedgeSquare = 0, kWedgeHouse = 1 };
+//
+// House over the whole graph from its apexes (HouseArgs): 4-cycles by their
+// highest vertex a, middles b < a, ends w < a,
+//   sum_w (c - 1) s = sum over wedges a - b - w of (c(a, w) - 1) (t(a, b) + t(b, w)).
+enum WedgeUse : int { kWedgeSquare = 0, kWedgeHouse = 1, kWedgeApex = 2 };
 struct WedgeArgs {
   const uint64_t* rp;
   const uint32_t* cols;
@@ -478,7 +491,7 @@ struct WedgeArgs {
   unsigned long long* next;     // work counter of LaunchWedgeTiles, zero
   uint32_t ntiles;              // id tiles a start vertex is walked in (set by the launcher)
   const uint32_t* t;            // house: triangles per CSR entry, both directions
-  // acc[0] += count; acc[1] += sum of |N+(a)|; square: acc[2] += wedges a - b - w;
+  // acc[0] += count (apex: that sum); acc[1] += sum of |N+(a)|; square: acc[2] += wedges a - b - w;
   // house: acc[2] += sum of d(a), acc[3] += sum_{b > a} t(a, b),
   // acc[4] += sum of |N+(a)| (d(a) - 1), acc[5] += sum_{b > a} t(a, b) (d(a) - 2)
   unsigned long long* acc;

@@ -259,8 +259,10 @@ __global__ __launch_bounds__(kThr) void WedgeTileKernel(WedgeArgs a) {
     __syncthreads();
     const u64 item = item_s;
     if (item >= nitems) break;
-    const u64 x = a.ntiles == 1 ? item : item / a.ntiles;
+    u64 x = a.ntiles == 1 ? item : item / a.ntiles;
     const uint32_t tile = a.ntiles == 1 ? 0 : static_cast<uint32_t>(item - x * a.ntiles);
+    // the apexes were appended in about increasing id: heaviest first
+    if (kUse == kWedgeApex) x = napex - 1 - x;
     const uint32_t v = a.heavy ? a.heavy[x] : a.v_begin + static_cast<uint32_t>(x);
     const uint64_t rb = a.rp[v], ub = a.up[v], re = a.rp[v + 1];
     // ends of this item: ids [lo, hi)
@@ -272,8 +274,11 @@ __global__ __launch_bounds__(kThr) void WedgeTileKernel(WedgeArgs a) {
     }
     if (kUse == kWedgeSquare && hi <= v + 1) continue;  // no end above v
     if (kUse == kWedgeSquare && lo <= v) lo = v + 1;
-    const uint64_t mb = kUse == kWedgeSquare ? ub : rb;  // middles
-    if (ub == re) continue;                              // no b > a
+    if (kUse == kWedgeApex && lo >= v) continue;         // no end below v
+    if (kUse == kWedgeApex && hi > v) hi = v;
+    // middles
+    const uint64_t mb = kUse == kWedgeSquare ? ub : rb, me = kUse == kWedgeApex ? ub : re;
+    if (kUse == kWedgeApex ? rb == ub : ub == re) continue;  // none, or no b > a
     const uint32_t words = (hi - lo + 1) / 2;
     for (uint32_t k = threadIdx.x; k < words; k += kThr) cnt[k] = 0;
     if (kUse == kWedgeHouse)
@@ -299,7 +304,7 @@ __global__ __launch_bounds__(kThr) void WedgeTileKernel(WedgeArgs a) {
         WalkLists(a.cols, lb, len, mid, s, lane, f);
       }
     };
-    walk(mb, re, [](uint64_t) { return 0u; },
+    walk(mb, me, [](uint64_t) { return 0u; },
          [&](uint32_t w, uint64_t, uint32_t) {
            const uint32_t k = w - lo;
            atomicAdd(cnt + (k >> 1), 1u << (16 * (k & 1)));
@@ -321,6 +326,13 @@ __global__ __launch_bounds__(kThr) void WedgeTileKernel(WedgeArgs a) {
         c2 += p + q;
         sum += (p ? p * (p - 1) / 2 : 0) + (q ? q * (q - 1) / 2 : 0);
       }
+    } else if (kUse == kWedgeApex) {
+      walk(rb, ub, [&](uint64_t k) { return a.t[k]; },
+           [&](uint32_t w, uint64_t e, uint32_t tab) {
+             const uint32_t k = w - lo;
+             const uint32_t c = (cnt[k >> 1] >> (16 * (k & 1))) & 0xffffu;
+             if (c > 1) sum += static_cast<u64>(c - 1) * (static_cast<u64>(tab) + a.t[e]);
+           });
     } else {
       // b > a: t(a, b) (c(a, w) - 1) per end w, less the pairs whose apex is w
       // or the middle opposite b
@@ -352,7 +364,7 @@ __global__ __launch_bounds__(kThr) void WedgeTileKernel(WedgeArgs a) {
   Flush(a.acc, 0, total, lane);
   if (kUse == kWedgeSquare) {
     Flush(a.acc, 2, c2, lane);
-  } else {
+  } else if (kUse == kWedgeHouse) {
     Flush(a.acc, 1, c1, lane);
     Flush(a.acc, 2, c2, lane);
     Flush(a.acc, 3, c3, lane);
@@ -429,8 +441,10 @@ void LaunchWedgeTiles(const WedgeArgs& a, int use, hipStream_t stream) {
   if (a.v_end <= a.v_begin) return;
   if (use == kWedgeSquare)
     LaunchTiles<kWedgeSquare>(a, stream);
-  else
+  else if (use == kWedgeHouse)
     LaunchTiles<kWedgeHouse>(a, stream);
+  else
+    LaunchTiles<kWedgeApex>(a, stream);
 }
 
 void LaunchAsymmetric(const uint64_t* rp, const uint32_t* cols, uint64_t n, uint64_t nnz, uint32_t* flag,
