@@ -1785,8 +1785,13 @@ void LocalHouse(Context* ctx, const DevGraph* g, uint64_t* count, RunStats* st) 
     w.next = lists.get() + 2;
     w.t = t.get();
     w.acc = acc.get();
+    // where the lists are cut into tiles, when that takes little of the memory
+    const uint64_t ncuts = (WedgeTiles(w.n) + 1ull) * n;
+    Buf<uint32_t> cuts(ctx, WedgeTiles(w.n) > 1 && 4 * ncuts <= ctx->RunAvailable() / 4 ? ncuts : 0);
     {
       Timed tm(ctx, s, kSlotHouseWedge, 0, 0);
+      if (cuts.get()) LaunchWedgeCuts(w, cuts.get(), s);
+      w.cuts = cuts.get();
       LaunchWedgeTiles(w, kWedgeApex, s);
     }
     if (g->max_degree > kWedgeDegreeMax) {

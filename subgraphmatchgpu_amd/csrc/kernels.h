@@ -490,6 +490,7 @@ struct WedgeArgs {
   unsigned long long* nheavy;
   unsigned long long* next;     // work counter of LaunchWedgeTiles, zero
   uint32_t ntiles;              // id tiles a start vertex is walked in (set by the launcher)
+  const uint32_t* cuts;         // LaunchWedgeCuts' table, or nullptr: lists are searched
   const uint32_t* t;            // house: triangles per CSR entry, both directions
   // acc[0] += count (apex: that sum); acc[1] += sum of |N+(a)|; square: acc[2] += wedges a - b - w;
   // house: acc[2] += sum of d(a), acc[3] += sum_{b > a} t(a, b),
@@ -503,6 +504,10 @@ void LaunchSquareLight(const WedgeArgs& a, hipStream_t stream);
 // Counts of `use` from heavy[] (or all start vertices): a workgroup per start
 // vertex and tile of ids keeps c in LDS.
 void LaunchWedgeTiles(const WedgeArgs& a, int use, hipStream_t stream);
+// Tiles of LaunchWedgeTiles; cuts[v * (tiles + 1) + k] = entries of N(v) below
+// tile k, k = 0 .. tiles.
+uint32_t WedgeTiles(uint32_t n);
+void LaunchWedgeCuts(const WedgeArgs& a, uint32_t* cuts, hipStream_t stream);
 // *flag (zero before) becomes 1 unless every entry (v, u) has its mirror (u, v).
 void LaunchAsymmetric(const uint64_t* rp, const uint32_t* cols, uint64_t n, uint64_t nnz, uint32_t* flag,
                       hipStream_t stream);

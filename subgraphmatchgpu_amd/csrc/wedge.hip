@@ -6,6 +6,8 @@
 // 13-119; the house likewise, one path per (v1, v2, v3)).  Here the wedges
 // a - b - w of a start vertex are counted per end w in LDS, so a wedge costs
 // one list entry and one LDS add instead of an intersection.
+#include <type_traits>
+
 #include "kernels.h"
 #include "wave.h"
 
@@ -44,33 +46,46 @@ __device__ __forceinline__ void Flush(unsigned long long* acc, int j, u64 v, int
   if (lane == 0 && v) atomicAdd(acc + j, v);
 }
 
+constexpr uint32_t kFlight = 4;                   // loads a lane keeps in flight
+constexpr uint32_t kWalkStep = kFlight * kWave;  // entries per step
+
 // Per-wave scratch of WalkLists.
 struct WalkLds {
-  uint64_t beg[kWave];
-  uint32_t start[kWave];
+  uint64_t from[kWave];  // k-th list: its first entry less its first item
   uint32_t mid[kWave];
-  uint32_t flag[kWave];
+  union {
+    uint8_t flag[kWalkStep];
+    uint32_t clear[kWave];
+  };
 };
-constexpr uint32_t kLongList = 48;  // lists from here on are streamed one by one
+static_assert(kWalkStep == 4 * kWave, "a lane clears one word of flags");
+constexpr uint32_t kLongList = kWalkStep;  // lists from here on are streamed one by one
 
-// Calls f(w, e, mid) for every entry e (w = cols[e]) of the lanes' lists
-// cols[lb, lb + len): long lists one after another, 64 consecutive entries per
-// load and four loads in flight, the short ones together as one flat list of
-// items.  f may use no wave operation.
-template <class F>
-__device__ __forceinline__ void WalkLists(const uint32_t* cols, uint64_t lb, uint32_t len, uint32_t mid, WalkLds& s,
-                                          int lane, F f) {
+// Calls f(w, t, mid) for every entry e (w = cols[e]; t = tri[e] with kT) of the
+// lanes' lists cols[lb, lb + len): long lists one after another, the others
+// together as one flat list of items, kWalkStep entries per step with all of a
+// step's loads issued before the first use.  f may use no wave operation.
+// (Streaming lists from 48 entries on one by one, and 64 items per step, left
+// one or two loads in flight: 59 against 44 ms for the tile kernel of the house
+// on R-MAT scale 19, 3.1 against 2.3 ms for the light 4-cycle kernel below.)
+template <bool kT, class F>
+__device__ __forceinline__ void WalkLists(const uint32_t* cols, const uint32_t* tri, uint64_t lb, uint32_t len,
+                                          uint32_t mid, WalkLds& s, int lane, F f) {
   for (u64 m = __ballot(len >= kLongList); m; m &= m - 1) {
     const uint32_t src = static_cast<uint32_t>(__builtin_ctzll(m));
     const uint64_t b = Lane64(lb, src);
     const uint32_t n = Lane32(len, src), md = Lane32(mid, src);
-    for (uint32_t i = static_cast<uint32_t>(lane); i < n; i += 4 * kWave) {
-      uint32_t w[4];
+    for (uint32_t i = static_cast<uint32_t>(lane); i < n; i += kWalkStep) {
+      uint32_t w[kFlight], t[kFlight];
 #pragma unroll
-      for (uint32_t h = 0; h < 4; ++h) w[h] = i + h * kWave < n ? cols[b + i + h * kWave] : 0u;
+      for (uint32_t h = 0; h < kFlight; ++h) {
+        const bool in = i + h * kWave < n;
+        w[h] = in ? cols[b + i + h * kWave] : 0u;
+        t[h] = kT && in ? tri[b + i + h * kWave] : 0u;
+      }
 #pragma unroll
-      for (uint32_t h = 0; h < 4; ++h)
-        if (i + h * kWave < n) f(w[h], b + i + h * kWave, md);
+      for (uint32_t h = 0; h < kFlight; ++h)
+        if (i + h * kWave < n) f(w[h], t[h], md);
     }
   }
   const uint32_t items = len < kLongList ? len : 0;
@@ -82,24 +97,34 @@ __device__ __forceinline__ void WalkLists(const uint32_t* cols, uint64_t lb, uin
   WaveSync();  // the previous walk's readers are done
   if (items) {
     const int at = static_cast<int>(__popcll(work & (upto >> 1)));
-    s.start[at] = start;
-    s.beg[at] = lb;
+    s.from[at] = lb - start;
     s.mid[at] = mid;
   }
-  uint32_t before = 0;
-  for (uint32_t t0 = 0; t0 < total; t0 += kWave) {
-    s.flag[lane] = 0;
+  uint32_t before = 0;  // lists that started before this step
+  for (uint32_t t0 = 0; t0 < total; t0 += kWalkStep) {
+    s.clear[lane] = 0;
     WaveSync();
-    if (items && start >= t0 && start - t0 < kWave) s.flag[start - t0] = 1;
+    if (items && start >= t0 && start - t0 < kWalkStep) s.flag[start - t0] = 1;
     WaveSync();
-    const u64 starts = __ballot(s.flag[lane] != 0);
-    const uint32_t own = before + static_cast<uint32_t>(__popcll(starts & upto)) - 1;
-    before += static_cast<uint32_t>(__popcll(starts));
-    const uint32_t it = t0 + static_cast<uint32_t>(lane);
-    if (it < total) {
-      const uint64_t e = s.beg[own] + (it - s.start[own]);
-      f(cols[e], e, s.mid[own]);
+    uint32_t w[kFlight], t[kFlight], md[kFlight];
+#pragma unroll
+    for (uint32_t h = 0; h < kFlight; ++h) {
+      w[h] = t[h] = md[h] = 0;
+      if (t0 + h * kWave >= total) continue;
+      const u64 starts = __ballot(s.flag[h * kWave + lane] != 0);
+      const uint32_t own = before + static_cast<uint32_t>(__popcll(starts & upto)) - 1;
+      before += static_cast<uint32_t>(__popcll(starts));
+      const uint32_t it = t0 + h * kWave + static_cast<uint32_t>(lane);
+      if (it < total) {
+        const uint64_t e = s.from[own] + it;
+        w[h] = cols[e];
+        if (kT) t[h] = tri[e];
+        md[h] = s.mid[own];
+      }
     }
+#pragma unroll
+    for (uint32_t h = 0; h < kFlight; ++h)
+      if (t0 + h * kWave + static_cast<uint32_t>(lane) < total) f(w[h], t[h], md[h]);
   }
 }
 
@@ -112,10 +137,11 @@ __device__ __forceinline__ void WalkLists(const uint32_t* cols, uint64_t lb, uin
 //
 // Bound by the latency of a start vertex's chain (its list, the middles' list
 // bounds, their entries, the LDS adds).  300 packed G(n, m) members (1.25e6
-// vertices, 3.3e7 entries): 3.1 ms, where the level engine wrote every wedge
+// vertices, 3.3e7 entries): 2.3 ms, where the level engine wrote every wedge
 // as a path and intersected two lists for it (52 ms).  Two passes over 4,096
 // ids cover the members (n <= 8,192) at 6 waves per SIMD; a start vertex above
 // kLightItems would hold its wave for over 64 steps and goes to the tiles.
+constexpr uint32_t kCutList = 48;       // lists up to here are walked whole and filtered
 constexpr uint32_t kLightItems = 4096;
 constexpr uint32_t kLightSpan = 4096;   // ids per pass of the byte counters
 constexpr uint32_t kLightSlots = 1024;  // hash slots, at most half full
@@ -155,7 +181,7 @@ __global__ __launch_bounds__(kThreads) void SquareLightKernel(WedgeArgs a) {
           lb = a.rp[v1];
           const uint64_t le = a.rp[v1 + 1];
           // v0 lies in N(v1): short lists are walked whole and filtered
-          if (le - lb >= kLongList) lb = Lower(a.cols, lb, le, v0);
+          if (le - lb >= kCutList) lb = Lower(a.cols, lb, le, v0);
           heavy = le - lb > kLightItems;
           len = heavy ? kLightItems : static_cast<uint32_t>(le - lb);
           last = a.cols[le - 1];
@@ -184,7 +210,7 @@ __global__ __launch_bounds__(kThreads) void SquareLightKernel(WedgeArgs a) {
           for (uint32_t k = lane; k < kLightSpan / 4; k += kWave) s.buf[k] = 0;
           WaveSync();
           uint32_t seen = 0, pairs = 0;
-          WalkLists(a.cols, lb, len, 0u, s.walk, lane, [&](uint32_t w, uint64_t, uint32_t) {
+          WalkLists<false>(a.cols, nullptr, lb, len, 0u, s.walk, lane, [&](uint32_t w, uint32_t, uint32_t) {
             const uint32_t k = w - lo;  // (w <= v0: wraps around)
             if (k >= kLightSpan) return;
             const uint32_t sh = 8 * (k & 3);
@@ -200,7 +226,7 @@ __global__ __launch_bounds__(kThreads) void SquareLightKernel(WedgeArgs a) {
         for (uint32_t k = lane; k < kLightSlots / 4; k += kWave) s.buf[kLightSlots + k] = 0;
         WaveSync();
         uint32_t seen = 0, pairs = 0;
-        WalkLists(a.cols, lb, len, 0u, s.walk, lane, [&](uint32_t w, uint64_t, uint32_t) {
+        WalkLists<false>(a.cols, nullptr, lb, len, 0u, s.walk, lane, [&](uint32_t w, uint32_t, uint32_t) {
           if (w <= v0) return;
           uint32_t h = (w * 0x9E3779B1u) >> (32 - kLightBits);
           while (true) {
@@ -231,11 +257,15 @@ __global__ __launch_bounds__(kThreads) void SquareLightKernel(WedgeArgs a) {
 // vertices differ by orders of magnitude; each ends when the counter passes
 // the last item.  Graphs of up to 16,384 vertices use 32 KB of counters and
 // four workgroups per CU; larger ones 128 KB and one of 1,024 threads, since a
-// list has to be cut (two searches) once per tile.
+// list has to be cut once per tile (tiles of 32,768 ids: 56 ms where these take
+// 38, searching).  The cuts of every list at the tiles' bounds are kept in a
+// table where there is room (one load instead of two searches: 38 -> 25 ms).
 //
-// Bound by the LDS adds and the list reads.  House from a third of R-MAT scale
-// 14's start vertices: 0.45 ms, where the level engine counted pairs for every
-// (v1, v2, v3) path (11.1 ms).
+// Bound by the wave instructions of the walks and the list reads.  House from a third of R-MAT scale
+// 14's start vertices: 0.38 ms, where the level engine counted pairs for every
+// (v1, v2, v3) path (11.1 ms).  House of R-MAT scale 19, edge factor 32, from
+// its apexes (6.7e9 wedges walked twice): 25 ms, where one 64-bit device atomic
+// per wedge into dense arrays and their reduction took 327 ms.
 template <int kUse, uint32_t kIds, int kThr>
 __global__ __launch_bounds__(kThr) void WedgeTileKernel(WedgeArgs a) {
   constexpr uint32_t kWv = kThr / kWave;
@@ -284,8 +314,11 @@ __global__ __launch_bounds__(kThr) void WedgeTileKernel(WedgeArgs a) {
     if (kUse == kWedgeHouse)
       for (uint32_t k = threadIdx.x; k < (hi - lo + 31) / 32; k += kThr) adj[k] = 0;
     __syncthreads();
-    // a wave takes `per` middles at a time, all waves about the same number
-    auto walk = [&](uint64_t b, uint64_t e, auto&& prep, auto&& f) {
+    // a wave takes `per` middles at a time, all waves about the same number; a
+    // second walk over the same middles finds the first ones' windows again
+    uint64_t lb_kept = 0;
+    uint32_t len_kept = 0;
+    auto walk = [&](auto with_t, uint64_t b, uint64_t e, auto&& prep, auto&& f) {
       const uint64_t share = (e - b + kWv - 1) / kWv;
       const uint32_t per = share < kWave ? static_cast<uint32_t>(share) : kWave;
       for (uint64_t k0 = b + static_cast<uint64_t>(wid) * per; k0 < e; k0 += static_cast<uint64_t>(kWv) * per) {
@@ -293,19 +326,37 @@ __global__ __launch_bounds__(kThr) void WedgeTileKernel(WedgeArgs a) {
         uint64_t lb = 0;
         uint32_t len = 0, mid = 0;
         if (static_cast<uint32_t>(lane) < per && k < e) {
-          const uint32_t m = a.cols[k];
-          lb = a.rp[m];
-          uint64_t le = a.rp[m + 1];
-          if (lo > 0) lb = Lower(a.cols, lb, le, lo);
-          if (hi < a.n) le = Lower(a.cols, lb, le, hi);
-          len = static_cast<uint32_t>(le - lb);
+          if (kUse == kWedgeApex && decltype(with_t)::value && k0 == b + static_cast<uint64_t>(wid) * per) {
+            lb = lb_kept;
+            len = len_kept;
+          } else {
+            const uint32_t m = a.cols[k];
+            lb = a.rp[m];
+            uint64_t le = a.rp[m + 1];
+            if (a.cuts) {
+              // the tile's share of N(m), then the end or start within it
+              const uint32_t* cut = a.cuts + static_cast<uint64_t>(m) * (a.ntiles + 1) + tile;
+              le = lb + cut[1];
+              lb += cut[0];
+              if (lo != tile * kIds) lb = Lower(a.cols, lb, le, lo);
+              if (hi != tile * kIds + kIds && hi != a.n) le = Lower(a.cols, lb, le, hi);
+            } else {
+              if (lo > 0) lb = Lower(a.cols, lb, le, lo);
+              if (hi < a.n) le = Lower(a.cols, lb, le, hi);
+            }
+            len = static_cast<uint32_t>(le - lb);
+          }
           mid = prep(k);
         }
-        WalkLists(a.cols, lb, len, mid, s, lane, f);
+        if (kUse == kWedgeApex && k0 == b + static_cast<uint64_t>(wid) * per) {
+          lb_kept = lb;
+          len_kept = len;
+        }
+        WalkLists<decltype(with_t)::value>(a.cols, a.t, lb, len, mid, s, lane, f);
       }
     };
-    walk(mb, me, [](uint64_t) { return 0u; },
-         [&](uint32_t w, uint64_t, uint32_t) {
+    walk(std::false_type{}, mb, me, [](uint64_t) { return 0u; },
+         [&](uint32_t w, uint32_t, uint32_t) {
            const uint32_t k = w - lo;
            atomicAdd(cnt + (k >> 1), 1u << (16 * (k & 1)));
          });
@@ -327,16 +378,16 @@ __global__ __launch_bounds__(kThr) void WedgeTileKernel(WedgeArgs a) {
         sum += (p ? p * (p - 1) / 2 : 0) + (q ? q * (q - 1) / 2 : 0);
       }
     } else if (kUse == kWedgeApex) {
-      walk(rb, ub, [&](uint64_t k) { return a.t[k]; },
-           [&](uint32_t w, uint64_t e, uint32_t tab) {
+      walk(std::true_type{}, rb, ub, [&](uint64_t k) { return a.t[k]; },
+           [&](uint32_t w, uint32_t tbw, uint32_t tab) {
              const uint32_t k = w - lo;
              const uint32_t c = (cnt[k >> 1] >> (16 * (k & 1))) & 0xffffu;
-             if (c > 1) sum += static_cast<u64>(c - 1) * (static_cast<u64>(tab) + a.t[e]);
+             sum += static_cast<u64>(c - 1) * (tab + tbw);
            });
     } else {
       // b > a: t(a, b) (c(a, w) - 1) per end w, less the pairs whose apex is w
       // or the middle opposite b
-      walk(ub, re,
+      walk(std::true_type{}, ub, re,
            [&](uint64_t k) {
              const uint32_t tab = a.t[k];
              if (tile == 0) {
@@ -345,12 +396,12 @@ __global__ __launch_bounds__(kThr) void WedgeTileKernel(WedgeArgs a) {
              }
              return tab;
            },
-           [&](uint32_t w, uint64_t e, uint32_t tab) {
+           [&](uint32_t w, uint32_t tbw, uint32_t tab) {
              if (w == v) return;
              const uint32_t k = w - lo;
              const uint32_t c = (cnt[k >> 1] >> (16 * (k & 1))) & 0xffffu;
              sum += static_cast<u64>(tab) * (c - 1);
-             if ((adj[k >> 5] >> (k & 31)) & 1u) sum -= static_cast<u64>(a.t[e]) + c - 2;
+             if ((adj[k >> 5] >> (k & 31)) & 1u) sum -= static_cast<u64>(tbw) + c - 2;
            });
     }
     total += sum;
@@ -406,18 +457,29 @@ __global__ __launch_bounds__(kThreads) void AsymmetricKernel(const uint64_t* rp,
   if (bad) atomicOr(flag, 1u);
 }
 
+// 16,384 ids: 32 KB of counters, four workgroups per CU; 65,536: 128 KB, one
+constexpr uint32_t kSmall = 16384, kLarge = 65536;
+
+__global__ __launch_bounds__(kThreads) void WedgeCutsKernel(WedgeArgs a, uint32_t* cuts) {
+  const uint64_t per = a.ntiles + 1, total = per * a.n;
+  const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
+  for (uint64_t i = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x; i < total; i += stride) {
+    const uint64_t v = i / per, b = a.rp[v], e = a.rp[v + 1], lo = (i - v * per) * kLarge;
+    cuts[i] = static_cast<uint32_t>((lo < a.n ? Lower(a.cols, b, e, static_cast<uint32_t>(lo)) : e) - b);
+  }
+}
+
 template <int kUse>
 void LaunchTiles(const WedgeArgs& a, hipStream_t stream) {
   WedgeArgs b = a;
   const uint64_t nv = a.v_end - a.v_begin;
-  // 16,384 ids: 32 KB of counters, four workgroups per CU; 65,536: 128 KB, one
-  constexpr uint32_t kSmall = 16384, kLarge = 65536;
   if (a.n <= kSmall) {
     b.ntiles = 1;
+    b.cuts = nullptr;
     const uint32_t grid = nv < 1024 ? static_cast<uint32_t>(nv) : 1024;
     hipLaunchKernelGGL((WedgeTileKernel<kUse, kSmall, 256>), dim3(grid), dim3(256), 0, stream, b);
   } else {
-    b.ntiles = (a.n + kLarge - 1) / kLarge;
+    b.ntiles = WedgeTiles(a.n);
     const uint64_t items = nv * b.ntiles;
     const uint32_t grid = items < 256 ? static_cast<uint32_t>(items) : 256;
     hipLaunchKernelGGL((WedgeTileKernel<kUse, kLarge, 1024>), dim3(grid), dim3(1024), 0, stream, b);
@@ -435,6 +497,15 @@ void LaunchSquareLight(const WedgeArgs& a, hipStream_t stream) {
   b.group = static_cast<uint32_t>(per < 1 ? 1 : per > 16 ? 16 : per);
   const uint64_t need = ((nv + b.group - 1) / b.group + kWaves - 1) / kWaves;
   hipLaunchKernelGGL(SquareLightKernel, dim3(need < 2048 ? need : 2048), dim3(kThreads), 0, stream, b);
+}
+
+uint32_t WedgeTiles(uint32_t n) { return n <= kSmall ? 1 : (n - 1) / kLarge + 1; }
+
+void LaunchWedgeCuts(const WedgeArgs& a, uint32_t* cuts, hipStream_t stream) {
+  WedgeArgs b = a;
+  b.ntiles = WedgeTiles(a.n);
+  const uint64_t need = ((b.ntiles + 1ull) * a.n + kThreads - 1) / kThreads;
+  hipLaunchKernelGGL(WedgeCutsKernel, dim3(need < 8192 ? need : 8192), dim3(kThreads), 0, stream, b, cuts);
 }
 
 void LaunchWedgeTiles(const WedgeArgs& a, int use, hipStream_t stream) {
