@@ -343,6 +343,22 @@ __device__ __forceinline__ uint64_t ItemVertex(const CliqueArgs& a, uint64_t t) 
   return lo;
 }
 
+// The same by the whole wave: 64 evenly spaced entries per round, so that the
+// chain of dependent loads is 3 long (60,000 vertices) instead of 16.
+__device__ __forceinline__ uint64_t ItemVertexWave(const CliqueArgs& a, uint64_t t, int lane) {
+  const uint64_t key = a.row_first[0] + t;
+  uint64_t lo = 0, n = a.nverts;  // the vertex lies in [lo, lo + n)
+  while (n > 1) {
+    const uint64_t step = (n + kWave - 1) / kWave;
+    const uint64_t at = lo + static_cast<uint64_t>(lane) * step;
+    const u64 m = __ballot(static_cast<uint64_t>(lane) * step < n && a.row_first[at] <= key);
+    const uint64_t skip = (__popcll(m) - 1) * step;  // lane 0 always holds
+    lo += skip;
+    n = n - skip < step ? n - skip : step;
+  }
+  return lo;
+}
+
 // One wave per row: word c of row i is the ballot of "u_j in N+(u_i)" over
 // j = 64c + lane (j > i).  Words are gathered one per lane and stored 64 at
 // a time.
@@ -787,39 +803,309 @@ __device__ __forceinline__ void FlushSums(unsigned long long* acc, int K, Clique
   if (K >= 6) Flush(acc, 6, cs->c6, lane);
 }
 
-// One wave per row i of a big vertex, rows in device memory.
-template <int K>
-__global__ __launch_bounds__(kThreads) void CliqueCountKernel(CliqueArgs a) {
-  constexpr int kBufs = K - 3;
-  __shared__ u64 lds_s[kWaves][kBufs][kWordsMax];
+// 4-cliques: a wave takes groups of kRowGroup consecutive rows, one search for
+// the group's first vertex, then a walk forward (a row is light next to the
+// search).
+__global__ __launch_bounds__(kThreads) void CliqueCount4Kernel(CliqueArgs a) {
+  __shared__ u64 lds_s[kWaves][kWordsMax];
   __shared__ uint32_t lds_q[kWaves][2 * kWave];
   const int lane = threadIdx.x & (kWave - 1);
   const int wid = threadIdx.x / kWave;
-  u64* s1 = lds_s[wid][0];
-  u64* s2 = lds_s[wid][kBufs > 1 ? 1 : 0];
-  u64* s3 = lds_s[wid][kBufs > 2 ? 2 : 0];
-  uint32_t* q = lds_q[wid];
   const uint64_t wave = (blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x) / kWave;
   const uint64_t nwaves = static_cast<uint64_t>(gridDim.x) * blockDim.x / kWave;
   CliqueSums cs;
-  // up to 4-cliques a row is light next to the search for its vertex: a
-  // wave takes groups of kRowGroup consecutive rows, one search for the
-  // group's first vertex, then a walk forward.  Deeper cliques' rows are
-  // heavy, and the first rows of the largest vertices heaviest; one row at
-  // a time keeps them spread over the waves.
-  constexpr uint64_t kRowGroup = K <= 4 ? 16 : 1;
+  constexpr uint64_t kRowGroup = 16;
   const uint64_t base = a.row_first[0];
   for (uint64_t t0 = wave * kRowGroup; t0 < a.nitems; t0 += nwaves * kRowGroup) {
     const uint64_t te = t0 + kRowGroup < a.nitems ? t0 + kRowGroup : a.nitems;
-    uint64_t x = ItemVertex(a, t0);
+    uint64_t x = ItemVertexWave(a, t0, lane);
     for (uint64_t t = t0; t < te; ++t) {
       while (a.row_first[x + 1] - base <= t) ++x;
       const uint32_t d = static_cast<uint32_t>(a.row_first[x + 1] - a.row_first[x]);
       const uint32_t i = static_cast<uint32_t>(t - (a.row_first[x] - base));
       const u64* rows = a.rows + (a.word_first[x] - a.word_first[0]);
-      const u64 vk = CountRow<K>(rows, d, i, s1, s2, s3, q, lane, &cs);
+      const u64 vk = CountRow<4>(rows, d, i, lds_s[wid], nullptr, nullptr, lds_q[wid], lane, &cs);
       if (a.bk.bounds) AddBucket(a.bk, a.verts[x], vk, lane);
     }
+  }
+  FlushSums(a.acc, 4, &cs, lane);
+}
+
+// 5- and 6-cliques.  The m members of row i span W words, most of whose bits
+// are not members.  Their rows are first packed to the members' columns: lane =
+// member j reads the words of row j, and for each set bit of row i (the same
+// for all lanes) one bit of the word moves to the next packed place.  What is
+// left to count is the triangles of a graph of m vertices held as m rows of
+// ceil(m / 32) words in LDS.  For 5-cliques lane = row j keeps its row in
+// registers and all lanes meet the same row l at a time (an LDS broadcast, no
+// bank conflicts): popcount(row_j & row_l) counts where row j has bit l.
+//
+// Bound by VALU issue (three quarters of the cycles in the long rows).  R-MAT
+// scale 19, edge factor 32, 5-clique: 160 ms when each row j below i was
+// intersected by a wave (W of 64 lanes busy) and its members probed rows in
+// device memory; 92 ms packed (26 ms rows of up to 128 members, 35 up to 256,
+// 30 up to 512).  Walking each lane's own bits instead of meeting rows by
+// broadcast took 173 ms: the random LDS rows conflict and the lanes' bit counts
+// differ.  6-cliques walk bits all the same: their inner sets differ by lane.
+
+// Words between packed rows of NW words: 16-byte aligned from 4 words on, and
+// an odd multiple of 4 so that 64 rows spread over 16 banks.
+constexpr uint32_t PackStride(int nw) { return nw < 4 ? nw : nw == 4 ? 4 : nw + 4; }
+
+// Packs the rows of members r = lane + 64 g (j = mem[r], r < m), g < G, taking
+// the words [w0, w1) of row i (s1), whose first set bit is packed bit `pos`.
+// pack must be zero.
+template <int G, int NW>
+__device__ __forceinline__ void PackRows(const u64* rows, uint32_t d, const u64* s1, uint32_t w0, uint32_t w1,
+                                         uint32_t pos, const uint16_t* mem, uint32_t m, uint32_t* pack, int lane) {
+  if (w0 >= w1) return;
+  const u64* rj[G];
+  u64 next[G];
+  uint32_t cur[G];
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    const uint32_t r = static_cast<uint32_t>(lane) + g * kWave;
+    rj[g] = r < m ? rows + mem[r] : nullptr;
+    next[g] = rj[g] ? rj[g][static_cast<uint64_t>(w0) * d] : 0;
+    cur[g] = 0;
+  }
+  auto flush = [&](uint32_t k) {
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      if (cur[g]) atomicOr(pack + (static_cast<uint32_t>(lane) + g * kWave) * PackStride(NW) + k, cur[g]);
+      cur[g] = 0;
+    }
+  };
+  for (uint32_t w = w0; w < w1; ++w) {
+    u64 x[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      x[g] = next[g];
+      if (w + 1 < w1 && rj[g]) next[g] = rj[g][static_cast<uint64_t>(w + 1) * d];
+    }
+    const u64 mask = First64(s1[w]);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      for (uint32_t mk = static_cast<uint32_t>(mask >> (32 * h)); mk; mk &= mk - 1) {
+        const uint32_t b = static_cast<uint32_t>(__builtin_ctz(mk));
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+          cur[g] |= ((static_cast<uint32_t>(x[g] >> (32 * h)) >> b) & 1u) << (pos & 31);
+        if ((++pos & 31) == 0) flush((pos >> 5) - 1);
+      }
+    }
+  }
+  if (pos & 31) flush(pos >> 5);
+}
+
+// The pairs and triangles of row r of a packed graph of m rows, meeting the
+// rows of the words w with w % parts == part.
+template <int NW>
+__device__ __forceinline__ u64 CountPacked5(const uint32_t* pack, uint32_t m, uint32_t r, uint32_t first,
+                                            uint32_t parts, uint32_t part, CliqueSums* cs) {
+  constexpr uint32_t S = PackStride(NW);
+  uint32_t c[NW];
+#pragma unroll
+  for (uint32_t k = 0; k < NW; ++k) c[k] = r < m ? pack[r * S + k] : 0u;
+  uint32_t pairs = 0;
+  u64 x5 = 0;
+#pragma unroll
+  for (uint32_t w = 0; w < NW; ++w) {
+    // (rows below `first`, the wave's first, have no bit in any of its rows)
+    if (w * 32 >= m || w < first / 32 || (parts > 1 && w % parts != part)) continue;
+    pairs += __builtin_popcount(c[w]);
+    const uint32_t* pl = pack + w * 32 * S;
+    const uint32_t n = m - w * 32 < 32 ? m - w * 32 : 32;
+    uint32_t x = 0;
+#pragma unroll 2
+    for (uint32_t b = 0; b < n; ++b, pl += S) {
+      uint32_t y = 0;
+#pragma unroll
+      for (uint32_t k = w; k < NW; ++k) y += __builtin_popcount(c[k] & pl[k]);
+      x += y & (0u - ((c[w] >> b) & 1u));  // (a multiply is quarter rate)
+    }
+    x5 += x;
+  }
+  cs->c4 += pairs;
+  cs->c5 += x5;
+  return x5;
+}
+
+// 6-cliques: row r's pairs and triangles, and the 4-cliques below it, each
+// lane walking the bits of its own row.
+template <int NW>
+__device__ __forceinline__ u64 CountPacked6(const uint32_t* pack, uint32_t m, uint32_t r, CliqueSums* cs) {
+  constexpr uint32_t S = PackStride(NW);
+  if (r >= m) return 0;
+  uint32_t c[NW];
+  uint32_t pairs = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < NW; ++k) {
+    c[k] = pack[r * S + k];
+    pairs += __builtin_popcount(c[k]);
+  }
+  u64 x5 = 0, x6 = 0;
+#pragma unroll
+  for (uint32_t w = 0; w < NW; ++w) {
+    for (uint32_t bits = c[w]; bits; bits &= bits - 1) {
+      const uint32_t* pl = pack + (w * 32 + __builtin_ctz(bits)) * S;
+      uint32_t t[NW];
+#pragma unroll
+      for (uint32_t k = 0; k < NW; ++k) {
+        t[k] = k >= w ? c[k] & pl[k] : 0u;
+        x5 += __builtin_popcount(t[k]);
+      }
+#pragma unroll
+      for (uint32_t k = 0; k < NW; ++k) {
+        for (uint32_t b2 = t[k]; b2; b2 &= b2 - 1) {
+          const uint32_t* pq = pack + (k * 32 + __builtin_ctz(b2)) * S;
+          uint32_t s6 = 0;
+#pragma unroll
+          for (uint32_t k2 = k; k2 < NW; ++k2) s6 += __builtin_popcount(t[k2] & pq[k2]);
+          x6 += s6;
+        }
+      }
+    }
+  }
+  cs->c4 += pairs;
+  cs->c5 += x5;
+  cs->c6 += x6;
+  return x6;
+}
+
+// One row of at most 32 NW members by one wave.
+template <int K, int NW>
+__device__ __forceinline__ u64 CountWave(const u64* rows, uint32_t d, uint32_t i, const u64* s1, const uint16_t* mem,
+                                         uint32_t m, uint32_t* pack, int lane, CliqueSums* cs) {
+  constexpr int G = NW > 2 ? NW / 2 : 1;
+  for (uint32_t k = lane; k < m * PackStride(NW); k += kWave) pack[k] = 0;
+  WaveSync();
+  PackRows<G, NW>(rows, d, s1, (i + 1) >> 6, (d + 63) / 64, 0, mem, m, pack, lane);
+  WaveSync();
+  u64 vk = 0;
+  for (uint32_t r = 0; r < m; r += kWave)
+    vk += K == 5 ? CountPacked5<NW>(pack, m, r + lane, r, 1, 0, cs) : CountPacked6<NW>(pack, m, r + lane, cs);
+  return vk;
+}
+
+// Row i into s1 (LDS), its members in order into mem (at most cap); returns
+// their number.  All lanes of the wave.
+__device__ __forceinline__ uint32_t LoadRow(const u64* rows, uint32_t d, uint32_t i, u64* s1, uint16_t* mem,
+                                            uint32_t cap, int lane) {
+  const uint32_t W = (d + 63) / 64, lo1 = (i + 1) >> 6;
+  const u64 below = lane ? (~0ull >> (64 - lane)) : 0ull;
+  WaveSync();  // readers of the previous row are done
+  for (uint32_t w = lo1 + lane; w < W; w += kWave) s1[w] = rows[static_cast<uint64_t>(w) * d + i];
+  WaveSync();
+  uint32_t m = 0;
+  for (uint32_t w = lo1; w < W; ++w) {
+    const u64 bits = First64(s1[w]);
+    const uint32_t at = m + static_cast<uint32_t>(__popcll(bits & below));
+    if (((bits >> lane) & 1) && at < cap) mem[at] = static_cast<uint16_t>(w * 64 + lane);
+    m += static_cast<uint32_t>(__popcll(bits));
+  }
+  WaveSync();
+  return m;
+}
+
+constexpr uint32_t kPackWave = 128;  // members a wave packs
+
+// One wave per row with at most kPackWave members.  Longer rows are left to
+// CliqueLongKernel in a.long_rows: up to 256 members from the front, the others
+// from the back.
+template <int K>
+__global__ __launch_bounds__(kThreads) void CliquePackKernel(CliqueArgs a) {
+  __shared__ u64 lds_s[kWaves][kWordsMax];
+  __shared__ __align__(16) uint32_t lds_pack[kWaves][PackStride(kPackWave / 32) * kPackWave];
+  __shared__ uint16_t lds_mem[kWaves][kPackWave];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wid = threadIdx.x / kWave;
+  u64* s1 = lds_s[wid];
+  uint32_t* pack = lds_pack[wid];
+  uint16_t* mem = lds_mem[wid];
+  const uint64_t wave = (blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x) / kWave;
+  const uint64_t nwaves = static_cast<uint64_t>(gridDim.x) * blockDim.x / kWave;
+  CliqueSums cs;
+  const uint64_t base = a.row_first[0];
+  constexpr uint64_t kRowGroup = 4;
+  for (uint64_t t0 = wave * kRowGroup; t0 < a.nitems; t0 += nwaves * kRowGroup) {
+    const uint64_t te = t0 + kRowGroup < a.nitems ? t0 + kRowGroup : a.nitems;
+    uint64_t x = ItemVertexWave(a, t0, lane);
+    for (uint64_t t = t0; t < te; ++t) {
+      while (a.row_first[x + 1] - base <= t) ++x;
+      const uint32_t d = static_cast<uint32_t>(a.row_first[x + 1] - a.row_first[x]);
+      const uint32_t i = static_cast<uint32_t>(t - (a.row_first[x] - base));
+      const u64* rows = a.rows + (a.word_first[x] - a.word_first[0]);
+      const uint32_t m = LoadRow(rows, d, i, s1, mem, kPackWave, lane);
+      if (m > kPackWave) {
+        if (lane == 0) {
+          const bool back = K != 5 || m > 256;
+          const u64 at = atomicAdd(a.nlong + (back ? 1 : 0), 1ull);
+          a.long_rows[back ? a.nitems - 1 - at : at] = static_cast<uint32_t>(t);
+        }
+        continue;
+      }
+      if (lane == 0) cs.c3 += m;
+      const u64 vk = m <= 32   ? CountWave<K, 1>(rows, d, i, s1, mem, m, pack, lane, &cs)
+                     : m <= 64 ? CountWave<K, 2>(rows, d, i, s1, mem, m, pack, lane, &cs)
+                               : CountWave<K, 4>(rows, d, i, s1, mem, m, pack, lane, &cs);
+      if (a.bk.bounds) AddBucket(a.bk, a.verts[x], vk, lane);
+    }
+  }
+  FlushSums(a.acc, K, &cs, lane);
+}
+
+// The long rows: 5-cliques of a row with at most 32 NW members by a workgroup,
+// each wave packing a share of the columns and meeting a share of the rows; the
+// others (longer, and all of 6-cliques, NW = 0) unpacked by its first wave.
+// kBack: the rows from the back of the list.
+template <int K, int NW, bool kBack>
+__global__ __launch_bounds__(kThreads) void CliqueLongKernel(CliqueArgs a) {
+  constexpr uint32_t kCap = NW ? 32 * NW : 1;
+  constexpr bool kUnpacked = kBack;
+  __shared__ u64 lds_s[kUnpacked ? K - 3 : 1][kWordsMax];
+  __shared__ uint32_t lds_q[kUnpacked ? 2 * kWave : 1];
+  __shared__ __align__(16) uint32_t pack[NW ? PackStride(NW) * kCap : 4];
+  __shared__ uint16_t mem[kCap];
+  __shared__ uint32_t members;
+  const int lane = threadIdx.x & (kWave - 1);
+  const uint32_t wid = threadIdx.x / kWave;
+  CliqueSums cs;
+  const uint64_t base = a.row_first[0];
+  const uint64_t nlong = a.nlong[kBack ? 1 : 0];
+  for (uint64_t y = blockIdx.x; y < nlong; y += gridDim.x) {
+    const uint64_t t = a.long_rows[kBack ? a.nitems - 1 - y : y];
+    const uint64_t x = ItemVertexWave(a, t, lane);
+    const uint32_t d = static_cast<uint32_t>(a.row_first[x + 1] - a.row_first[x]);
+    const uint32_t i = static_cast<uint32_t>(t - (a.row_first[x] - base));
+    const u64* rows = a.rows + (a.word_first[x] - a.word_first[0]);
+    __syncthreads();  // the previous row's readers are done
+    if (wid == 0) {
+      const uint32_t m = LoadRow(rows, d, i, lds_s[0], mem, kCap, lane);
+      if (lane == 0) members = m;
+    }
+    if (NW)
+      for (uint32_t k = threadIdx.x; k < PackStride(NW ? NW : 1) * kCap; k += kThreads) pack[k] = 0;
+    __syncthreads();
+    const uint32_t m = members;
+    u64 vk = 0;
+    if (kUnpacked && (m > kCap || !NW)) {
+      if (wid == 0)
+        vk = CountRow<K>(rows, d, i, lds_s[0], lds_s[kUnpacked ? 1 : 0], lds_s[kUnpacked && K > 5 ? 2 : 0], lds_q, lane,
+                         &cs);
+    } else if (NW) {
+      if (threadIdx.x == 0) cs.c3 += m;
+      const uint32_t W = (d + 63) / 64, lo1 = (i + 1) >> 6;
+      const uint32_t share = (W - lo1 + kWaves - 1) / kWaves;
+      const uint32_t w0 = lo1 + wid * share < W ? lo1 + wid * share : W, w1 = w0 + share < W ? w0 + share : W;
+      uint32_t pos = 0;
+      for (uint32_t w = lo1; w < w0; ++w) pos += static_cast<uint32_t>(__popcll(First64(lds_s[0][w])));
+      PackRows<NW ? (NW + 1) / 2 : 1, NW ? NW : 1>(rows, d, lds_s[0], w0, w1, pos, mem, m, pack, lane);
+      __syncthreads();
+      for (uint32_t r = 0; r < m; r += kWave)
+        vk += CountPacked5<NW ? NW : 1>(pack, m, r + lane, r, kWaves, wid, &cs);
+    }
+    if (a.bk.bounds) AddBucket(a.bk, a.verts[x], vk, lane);
   }
   FlushSums(a.acc, K, &cs, lane);
 }
@@ -875,10 +1161,19 @@ void LaunchCliqueRowsHash(const CliqueArgs& a, bool small_table, hipStream_t str
 void LaunchCliqueCount(const CliqueArgs& a, hipStream_t stream) {
   if (a.nitems == 0) return;
   const dim3 grid(Grid(a.nitems, kWaves)), block(kThreads);
+  const uint64_t rows = Grid(a.nitems, 1);
+  const dim3 longs(rows < 2048 ? rows : 2048);
   switch (a.k) {
-    case 4: hipLaunchKernelGGL(CliqueCountKernel<4>, grid, block, 0, stream, a); break;
-    case 5: hipLaunchKernelGGL(CliqueCountKernel<5>, grid, block, 0, stream, a); break;
-    case 6: hipLaunchKernelGGL(CliqueCountKernel<6>, grid, block, 0, stream, a); break;
+    case 4: hipLaunchKernelGGL(CliqueCount4Kernel, grid, block, 0, stream, a); break;
+    case 5:
+      hipLaunchKernelGGL(CliquePackKernel<5>, grid, block, 0, stream, a);
+      hipLaunchKernelGGL((CliqueLongKernel<5, 8, false>), longs, block, 0, stream, a);
+      hipLaunchKernelGGL((CliqueLongKernel<5, 16, true>), longs, block, 0, stream, a);
+      break;
+    case 6:
+      hipLaunchKernelGGL(CliquePackKernel<6>, grid, block, 0, stream, a);
+      hipLaunchKernelGGL((CliqueLongKernel<6, 0, true>), longs, block, 0, stream, a);
+      break;
   }
 }
 

@@ -1451,8 +1451,8 @@ void LocalCliqueRange(Context* ctx, const DevGraph* g, const EnginePlan* plan, u
   const int K = plan->nv;
   const uint64_t range = ve > vb ? ve - vb : 0;
   constexpr int kAcc = kCliqueMaxK + 1;
-  Buf<unsigned long long> acc(ctx, kAcc + 2);
-  LaunchFill64(reinterpret_cast<uint64_t*>(acc.get()), kAcc + 2, 0, s);
+  Buf<unsigned long long> acc(ctx, kAcc + 4);
+  LaunchFill64(reinterpret_cast<uint64_t*>(acc.get()), kAcc + 4, 0, s);
   // over all start vertices the upload-time lists serve; otherwise the small
   // kernel appends the range's larger vertices and they are sorted here
   const bool whole = vb == 0 && ve == g->n;
@@ -1471,6 +1471,7 @@ void LocalCliqueRange(Context* ctx, const DevGraph* g, const EnginePlan* plan, u
   a.nbig = acc.get() + kAcc;
   a.huge = huge.get();
   a.nhuge = acc.get() + kAcc + 1;
+  a.nlong = acc.get() + kAcc + 2;
   a.tc = tc;
   {
     Timed t(ctx, s, kSlotCliqueSmall, 20.0 * static_cast<double>(range), range);
@@ -1538,7 +1539,7 @@ void LocalCliqueRange(Context* ctx, const DevGraph* g, const EnginePlan* plan, u
   }
   if (nbig) {
     // batches of whole vertices whose rows fit what the run may use
-    uint64_t cap_words = static_cast<uint64_t>(0.9 * static_cast<double>(ctx->RunAvailable())) / 8;
+    uint64_t cap_words = static_cast<uint64_t>((K > 4 ? 0.7 : 0.9) * static_cast<double>(ctx->RunAvailable())) / 8;
     if (ctx->tuning.batch_bytes) cap_words = std::min<uint64_t>(cap_words, ctx->tuning.batch_bytes / 8);
     st->batches = 0;
     // the largest neighbourhoods come first: any whose rows alone exceed
@@ -1551,10 +1552,13 @@ void LocalCliqueRange(Context* ctx, const DevGraph* g, const EnginePlan* plan, u
     }
     for (uint64_t x0 = first_fit; x0 < nbig;) {
       uint64_t x1 = x0 + 1;
-      while (x1 < nbig && wf[x1 + 1] - wf[x0] <= cap_words) ++x1;
+      while (x1 < nbig && wf[x1 + 1] - wf[x0] <= cap_words && rf[x1 + 1] - rf[x0] <= kMaxBatchPaths) ++x1;
       const uint64_t words = wf[x1] - wf[x0];
       // triangles are counted as the rows are found: nothing to keep
       Buf<unsigned long long> rows(ctx, K > 3 ? words : 0);
+      // one row item per row (a row is at least two words)
+      Buf<uint32_t> long_rows(ctx, K > 4 ? rf[x1] - rf[x0] : 0);
+      a.long_rows = long_rows.get();
       a.verts = dverts + x0;
       a.nverts = x1 - x0;
       a.nitems = rf[x1] - rf[x0];
@@ -1616,6 +1620,7 @@ void LocalCliqueRange(Context* ctx, const DevGraph* g, const EnginePlan* plan, u
       if (K > 3) {
         // every row word read at least once
         Timed t(ctx, s, kSlotCliqueCount, 8.0 * static_cast<double>(words), a.nitems);
+        if (K > 4) LaunchFill64(reinterpret_cast<uint64_t*>(a.nlong), 2, 0, s);
         LaunchCliqueCount(a, s);
       }
       st->batches++;

@@ -377,6 +377,11 @@ struct CliqueArgs {
   // rows each
   const uint64_t* chunk_first;
   uint64_t nchunks;
+  // k >= 5: row items (nitems entries of room) that the first count kernel
+  // leaves to the others, at the front nlong[0] and at the back nlong[1] of
+  // them (zero before)
+  uint32_t* long_rows;
+  unsigned long long* nlong;
   // k == 3, nullable: tc[p] += the triangles through the edge stored at
   // cols[p] (p an index of some N+(x)), recorded by CliqueSmallKernel and
   // CliqueRowsKernel as they find each triangle (v, u_i, u_j)

@@ -214,3 +214,35 @@ def test_wedges(dev, name, q):
     got = dev.count_buckets(dg, sme.Plan(q), bounds)[0].tolist()
     dg.release()
     assert got == [oracle.light_count(g.row_ptrs, g.cols, q, 3, v_begin=a, v_end=b)[0] for a, b in zip(bounds, bounds[1:])]
+
+
+# row sizes at which the packed count changes: 32, 64, 128 members per wave, 512 per workgroup,
+# longer rows unpacked (vertex 0 of a clique of n has n - 1 upper neighbours, its first row n - 2)
+@pytest.mark.parametrize("q,n", [(7, 67), (7, 131), (11, 70)])
+def test_emu_packed_rows(emu, q, n):
+    g = union(clique(n) if n < 100 else sme.gen_er(n, n * n // 3, seed=n), sme.gen_er(70, 1200, seed=5))
+    want = oracle.light_count(g.row_ptrs, g.cols, q, 3)
+    assert emu(g, q) == (want[0], want[1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("q,n,p", [(7, 98, 1.0), (7, 131, 1.0), (7, 132, 0.9), (7, 300, 0.5), (7, 600, 0.97), (11, 131, 0.6),
+                                   (11, 200, 0.7), (7, 900, 0.2)])
+def test_packed_rows(dev, q, n, p):
+    m = int(p * n * (n - 1) / 2)
+    g = clique(n) if p == 1.0 else sme.gen_er(n, m, seed=n)
+    cut = max(0, n - 128) if p > 0.9 and n > 500 else 0  # (keeps the oracle's share small)
+    want = oracle.light_count(g.row_ptrs, g.cols, q, 3, v_begin=cut)
+    got = on_gpu(dev, g, q, cut)
+    assert got == (want[0], want[1])
+    # the level engine, which the oracle is too slow to stand in for on the dense ones
+    dg = dev.upload(g)
+    a = dev.count(dg, sme.Plan(q))
+    dev.set_tuning(super_chunks=4, clique_level_engine=1)
+    b = dev.count(dg, sme.Plan(q))
+    dev.set_tuning(super_chunks=4)
+    bounds = [0, 1, n // 3, n]
+    buckets = dev.count_buckets(dg, sme.Plan(q), bounds)[0]
+    dg.release()
+    assert (a.count, a.levels) == (b.count, b.levels)
+    assert int(buckets.sum()) == a.count
