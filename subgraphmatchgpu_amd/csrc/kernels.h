@@ -517,6 +517,34 @@ void LaunchWedgeCuts(const WedgeArgs& a, uint32_t* cuts, hipStream_t stream);
 void LaunchAsymmetric(const uint64_t* rp, const uint32_t* cols, uint64_t n, uint64_t nnz, uint32_t* flag,
                       hipStream_t stream);
 
+// ---------------------------------------------------------------------------
+// COMPUTE_PATH_COUNT and COMPUTE_COUNT of paths p over two or three adjacency
+// lists N(M[v]) (paths.hip): `own_v` is the list's vertex matched last,
+// shared_v the others, which runs of consecutive paths have in common.  Graphs
+// of at most kPathRunIds vertices.
+constexpr uint32_t kPathRunIds = 32768;
+constexpr uint32_t kOwnRatio = 16;
+struct PathRunArgs {
+  uint64_t npaths;
+  const uint64_t* rp;
+  const uint32_t* cols;
+  uint32_t n;
+  ColSet cs;
+  uint8_t nshared;
+  uint8_t shared_v[2];
+  uint8_t own_v;
+  uint8_t nlt, ngt;
+  uint8_t lt_v[kQ];
+  uint8_t gt_v[kQ];
+  uint8_t nne;
+  uint8_t ne_v[2];
+  uint64_t* out_len;              // per path (nullable)
+  unsigned long long* acc;        // the count (nullable), buckets with it
+  unsigned long long* acc_level;
+  BucketRef bk;
+};
+void LaunchPathRuns(const PathRunArgs& a, hipStream_t stream);
+
 // Exclusive scan: out[i] = sum(in[0..i)), out[n] = total.  `tmp` needs
 // ScanTempWords(n) u64 words.  out may alias in.
 size_t ScanTempWords(uint64_t n);

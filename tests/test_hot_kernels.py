@@ -246,3 +246,33 @@ def test_packed_rows(dev, q, n, p):
     dg.release()
     assert (a.count, a.levels) == (b.count, b.levels)
     assert int(buckets.sum()) == a.count
+
+
+# path runs: bitmaps of 8,192 ids, 32,768 ids and none; a hub whose list is over 16 times the shared one
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [8192, 8193, 32768, 32769])
+@pytest.mark.parametrize("q", [6, 8])
+def test_path_runs(dev, q, n):
+    tail = sme.gen_rmat(8, 12, seed=n)
+    g = union(hub_and_sparse(n - tail.n, 1500, 6 * n, n), tail)
+    assert g.n == n
+    want = oracle.light_count(g.row_ptrs, g.cols, q, 3)
+    assert want[0] and on_gpu(dev, g, q) == (want[0], want[1])
+    bounds = [0, 9, n // 2, n - tail.n, n]
+    dg = dev.upload(g)
+    got = dev.count_buckets(dg, sme.Plan(q), bounds)[0].tolist()
+    dg.release()
+    assert got == [oracle.light_count(g.row_ptrs, g.cols, q, 3, v_begin=a, v_end=b)[0] for a, b in zip(bounds, bounds[1:])]
+
+
+@pytest.mark.parametrize("q", [6, 8])
+def test_emu_path_runs(emu, q):
+    g = union(hub_and_sparse(400, 90, 700, 3), sme.gen_rmat(5, 8, seed=2))
+    for self_loop in (False, True):
+        if self_loop:  # the != conditions then count
+            src = np.repeat(np.arange(g.n), np.diff(g.row_ptrs.astype(np.int64)))
+            key = np.unique(np.concatenate([src * g.n + g.cols, np.arange(0, g.n, 7) * (g.n + 1)]))
+            g = sme.Graph(np.searchsorted(key, np.arange(g.n + 1) * g.n).astype(np.uint64),
+                          (key % g.n).astype(np.uint32))
+        want = oracle.light_count(g.row_ptrs, g.cols, q, 3)
+        assert emu(g, q) == (want[0], want[1])
