@@ -67,11 +67,6 @@ __device__ __forceinline__ void AddBucket(const BucketRef& b, uint32_t v, u64 pe
   if (lane == 0 && tot) atomicAdd(b.counts + BucketOf(b, v), tot);
 }
 
-__device__ __forceinline__ void Flush(unsigned long long* acc, int j, u64 v, int lane) {
-  v = WaveSum(v);
-  if (lane == 0 && v) atomicAdd(acc + j, v);
-}
-
 // ---------------------------------------------------------------------------
 // Start vertices with d <= 64.  A wave takes kSmallGroup consecutive start
 // vertices, packs as many whole ones as fit into 64 upper entries (lane =
@@ -97,7 +92,9 @@ constexpr uint32_t kSmallStream = 32;    // lists up to this length are streamed
 // up to here one start vertex per wave step: 4,096 waves of 4 vertices would
 // leave half the chip idle (R-MAT scale 14: 67 us against 130 us)
 constexpr uint64_t kSmallAlone = 16384;
-constexpr uint64_t kSmallGrid = 2048;    // workgroups: 8 per CU
+// workgroups: what the chip holds at once; fewer where each would get a few
+// vertices, since every one ends with an atomic on the same counters
+constexpr uint64_t kSmallGrid = 2048, kSmallGridFew = 1024;
 
 struct SmallLds {
   uint64_t beg[kWave];    // entry: N+(u_i) begins at cols[beg]
@@ -115,7 +112,6 @@ struct SmallLds {
 template <int K>
 __global__ __launch_bounds__(kThreads) void CliqueSmallKernel(CliqueArgs a) {
   __shared__ SmallLds lds_all[kWaves];
-  __shared__ u64 lds_sum[kCliqueMaxK + 1];
   const int lane = threadIdx.x & (kWave - 1);
   SmallLds& s = lds_all[threadIdx.x / kWave];
   const u64 upto = ~0ull >> (kWave - 1 - lane);  // lanes 0..lane
@@ -312,18 +308,12 @@ __global__ __launch_bounds__(kThreads) void CliqueSmallKernel(CliqueArgs a) {
     }
   }
   if (a.bk.bounds) BucketFlush(a.bk, &bacc);
-  // one atomic per workgroup and level
-  if (threadIdx.x <= static_cast<unsigned>(kCliqueMaxK)) lds_sum[threadIdx.x] = 0;
-  __syncthreads();
-  Flush(lds_sum, 1, c1, lane);
-  Flush(lds_sum, 2, c2, lane);
-  Flush(lds_sum, 3, c3, lane);
-  if (K >= 4) Flush(lds_sum, 4, c4, lane);
-  if (K >= 5) Flush(lds_sum, 5, c5, lane);
-  if (K >= 6) Flush(lds_sum, 6, c6, lane);
-  __syncthreads();
-  if (threadIdx.x >= 1 && threadIdx.x <= static_cast<unsigned>(K) && lds_sum[threadIdx.x])
-    atomicAdd(a.acc + threadIdx.x, lds_sum[threadIdx.x]);
+  BlockAdd<kThreads>(Into{a.acc + 1, c1},
+                     Into{a.acc + 2, c2},
+                     Into{a.acc + 3, c3},
+                     Into{K >= 4 ? a.acc + 4 : nullptr, c4},
+                     Into{K >= 5 ? a.acc + 5 : nullptr, c5},
+                     Into{K >= 6 ? a.acc + 6 : nullptr, c6});
 }
 
 // ---------------------------------------------------------------------------
@@ -400,7 +390,7 @@ __global__ __launch_bounds__(kThreads) void CliqueRowsKernel(CliqueArgs a) {
     if (lane == 0) c3 += bits;
     if (!a.rows && a.bk.bounds) AddBucket(a.bk, v, lane == 0 ? bits : 0u, lane);
   }
-  if (!a.rows) Flush(a.acc, 3, c3, lane);
+  if (!a.rows) BlockAdd<kThreads>(Into{a.acc + 3, c3});
 }
 
 // Chunk t of a batch: largest x with chunk_first[x] - chunk_first[0] <= t.
@@ -559,7 +549,7 @@ __global__ __launch_bounds__(kThreads) void CliqueRowsTableKernel(CliqueArgs a) 
       if (a.bk.bounds) AddBucket(a.bk, v, mine, lane);
     }
   }
-  if (kMode != kRowsBits) Flush(a.acc, 3, c3, lane);
+  if (kMode != kRowsBits) BlockAdd<kThreads>(Into{a.acc + 3, c3});
 }
 
 // One workgroup per chunk of 64 rows of one vertex v.  N+(v) goes into an LDS
@@ -676,7 +666,7 @@ __global__ __launch_bounds__(kThreads) void CliqueRowsHashKernel(CliqueArgs a) {
         if (lds_col[j]) atomicAdd(a.tc + nb + j, lds_col[j]);
     }
   }
-  if (!a.rows) Flush(a.acc, 3, c3, lane);
+  if (!a.rows) BlockAdd<kThreads>(Into{a.acc + 3, c3});
 }
 
 // |s & row_j| over the words of row j that can be non-zero (bits above j).
@@ -796,11 +786,11 @@ __device__ __forceinline__ u64 CountRow(const u64* rows, uint32_t d, uint32_t i,
   return vk;
 }
 
-__device__ __forceinline__ void FlushSums(unsigned long long* acc, int K, CliqueSums* cs, int lane) {
-  Flush(acc, 3, cs->c3, lane);
-  Flush(acc, 4, cs->c4, lane);
-  if (K >= 5) Flush(acc, 5, cs->c5, lane);
-  if (K >= 6) Flush(acc, 6, cs->c6, lane);
+__device__ __forceinline__ void FlushSums(unsigned long long* acc, int K, const CliqueSums& cs) {
+  BlockAdd<kThreads>(Into{acc + 3, cs.c3},
+                     Into{acc + 4, cs.c4},
+                     Into{K >= 5 ? acc + 5 : nullptr, cs.c5},
+                     Into{K >= 6 ? acc + 6 : nullptr, cs.c6});
 }
 
 // 4-cliques: a wave takes groups of kRowGroup consecutive rows, one search for
@@ -828,7 +818,7 @@ __global__ __launch_bounds__(kThreads) void CliqueCount4Kernel(CliqueArgs a) {
       if (a.bk.bounds) AddBucket(a.bk, a.verts[x], vk, lane);
     }
   }
-  FlushSums(a.acc, 4, &cs, lane);
+  FlushSums(a.acc, 4, cs);
 }
 
 // 5- and 6-cliques.  The m members of row i span W words, most of whose bits
@@ -1052,7 +1042,7 @@ __global__ __launch_bounds__(kThreads) void CliquePackKernel(CliqueArgs a) {
       if (a.bk.bounds) AddBucket(a.bk, a.verts[x], vk, lane);
     }
   }
-  FlushSums(a.acc, K, &cs, lane);
+  FlushSums(a.acc, K, cs);
 }
 
 // The long rows: 5-cliques of a row with at most 32 NW members by a workgroup,
@@ -1107,7 +1097,7 @@ __global__ __launch_bounds__(kThreads) void CliqueLongKernel(CliqueArgs a) {
     }
     if (a.bk.bounds) AddBucket(a.bk, a.verts[x], vk, lane);
   }
-  FlushSums(a.acc, K, &cs, lane);
+  FlushSums(a.acc, K, cs);
 }
 
 }  // namespace
@@ -1119,7 +1109,8 @@ void LaunchCliqueSmall(const CliqueArgs& a, hipStream_t stream) {
   CliqueArgs b = a;
   b.group = nv > kSmallAlone ? kSmallGroup : 1;
   const uint64_t need = Grid((nv + b.group - 1) / b.group, kWaves);
-  const dim3 grid(need < kSmallGrid ? need : kSmallGrid), block(kThreads);
+  const uint64_t most = nv > 4 * kSmallAlone ? kSmallGrid : kSmallGridFew;
+  const dim3 grid(need < most ? need : most), block(kThreads);
   switch (a.k) {
     case 3: hipLaunchKernelGGL(CliqueSmallKernel<3>, grid, block, 0, stream, b); break;
     case 4: hipLaunchKernelGGL(CliqueSmallKernel<4>, grid, block, 0, stream, b); break;

@@ -42,11 +42,6 @@ uint64_t Grid(uint64_t n, uint64_t per_block) {
   return g > kMaxGrid ? kMaxGrid : g;
 }
 
-__device__ __forceinline__ void Flush(unsigned long long* acc, int j, u64 v, int lane) {
-  v = WaveSum(v);
-  if (lane == 0 && v) atomicAdd(acc + j, v);
-}
-
 // First index in [lo, hi) with a[i] >= key.
 __device__ __forceinline__ uint64_t Lower(const uint32_t* a, uint64_t lo, uint64_t hi, uint32_t key) {
   while (lo < hi) {
@@ -112,7 +107,7 @@ __global__ __launch_bounds__(kThreads) void HouseMirrorKernel(HouseArgs a) {
     if (a.load) BucketAccAdd(rows, &run, key, load);
   }
   if (a.load) BucketFlush(rows, &run);
-  Flush(a.acc, 1, sq, lane);
+  BlockAdd<kThreads>(Into{a.acc + 1, sq});
 }
 
 __global__ __launch_bounds__(kThreads) void EdgePairsKernel(HouseArgs a) {
@@ -127,8 +122,7 @@ __global__ __launch_bounds__(kThreads) void EdgePairsKernel(HouseArgs a) {
       pairs += x * (x ? x - 1 : 0) / 2;
     }
   }
-  Flush(a.acc, 0, tri, lane);
-  Flush(a.acc, 1, pairs, lane);
+  BlockAdd<kThreads>(Into{a.acc, tri}, Into{a.acc + 1, pairs});
 }
 
 // Appends the lanes' vertices for which `take` holds: one atomic per wave.
@@ -204,7 +198,7 @@ __global__ __launch_bounds__(kThreads) void HouseWedgeHashKernel(HouseArgs a) {
       }
     }
   }
-  Flush(a.acc, 0, sum, lane);
+  BlockAdd<kThreads>(Into{a.acc, sum});
 }
 
 // Apex of dense item t: largest x with item_first[x] <= t.
@@ -261,7 +255,6 @@ __global__ __launch_bounds__(kThreads) void HouseWedgeDenseKernel(HouseArgs a) {
 
 // blockIdx.y = apex x: sums (c - 1) s over its w and clears them.
 __global__ __launch_bounds__(kThreads) void HouseWedgeReduceKernel(HouseArgs a) {
-  const int lane = threadIdx.x & (kWave - 1);
   const uint64_t x = blockIdx.y;
   u64* slot = a.slots + x * a.n;
   const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
@@ -284,7 +277,7 @@ __global__ __launch_bounds__(kThreads) void HouseWedgeReduceKernel(HouseArgs a) 
       slot[w] = 0;
     }
   }
-  Flush(a.acc, 0, sum, lane);
+  BlockAdd<kThreads>(Into{a.acc, sum});
 }
 
 }  // namespace

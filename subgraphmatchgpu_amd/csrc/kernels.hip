@@ -285,11 +285,7 @@ __global__ __launch_bounds__(kThreads) void CountPathsKernel(CountPathArgs a) {
     }
   }
   if (a.bk.bounds) BucketFlush(a.bk, &bacc);
-  local = WaveSum(local);
-  if ((threadIdx.x & (kWave - 1)) == 0 && local) {
-    if (a.acc) atomicAdd(a.acc, local);
-    if (a.acc_level) atomicAdd(a.acc_level, local);
-  }
+  BlockAdd<kThreads>(Into{a.acc, local}, Into{a.acc_level, local});
 }
 
 // chunk_seg[c] = segment of item 64c, written by the owning segment.
@@ -644,11 +640,7 @@ __global__ __launch_bounds__(kThreads) void VerifyKernel(ItemArgs a) {
   }
   if (kMode != kModeMask && a.bk.bounds) BucketFlush(a.bk, &bacc);
   if (kMode != kModeMask) {
-    local = WaveSum(local);
-    if (lane == 0 && local) {
-      atomicAdd(a.acc, local);
-      atomicAdd(a.acc_level, local);
-    }
+    BlockAdd<kThreads>(Into{a.acc, local}, Into{a.acc_level, local});
   }
 }
 
@@ -767,15 +759,7 @@ __global__ __launch_bounds__(kThreads) void PrepCountKernel(PrepCountArgs a) {
     }
   }
   if (a.it.bk.bounds) BucketFlush(a.it.bk, &bacc);
-  local = WaveSum(local);
-  nlane = WaveSum(nlane);
-  if (lane == 0) {
-    if (local) {
-      atomicAdd(a.it.acc, local);
-      atomicAdd(a.it.acc_level, local);
-    }
-    if (nlane && a.lane_items) atomicAdd(a.lane_items, nlane);
-  }
+  BlockAdd<kThreads>(Into{a.it.acc, local}, Into{a.it.acc_level, local}, Into{a.lane_items, nlane});
 }
 
 __device__ __forceinline__ uint64_t RankOf(const RankRef& r, uint64_t t) {
@@ -876,8 +860,7 @@ __global__ __launch_bounds__(kThreads) void ExclusionKernel(ExclusionArgs a) {
     a.excl_in[p] = bits;
     local += n - drop;
   }
-  local = WaveSum(local);
-  if ((threadIdx.x & (kWave - 1)) == 0 && local) atomicAdd(a.acc_level, local);
+  BlockAdd<kThreads>(Into{a.acc_level, local});
 }
 
 __global__ __launch_bounds__(kThreads) void BuildHubBitsKernel(const uint64_t* rp, const uint32_t* cols,
@@ -1034,7 +1017,6 @@ __global__ __launch_bounds__(kThreads) void PathWorkgroupKernel(ItemArgs a, cons
                                                                 const unsigned long long* wg_count,
                                                                 unsigned long long* items) {
   __shared__ uint32_t stage[kWgStage];
-  const int lane = threadIdx.x & (kWave - 1);
   const uint64_t np = *wg_count;
   u64 local = 0, walked = 0;
   BucketAcc bacc{kNoBucket, 0};
@@ -1091,14 +1073,7 @@ __global__ __launch_bounds__(kThreads) void PathWorkgroupKernel(ItemArgs a, cons
     if (a.bk.bounds) BucketAccAdd(a.bk, &bacc, BucketOf(a.bk, Gather(a.cs, a.bk.start_v, p)), v);
   }
   if (a.bk.bounds) BucketFlush(a.bk, &bacc);
-  local = WaveSum(local);
-  if (lane == 0) {
-    if (local) {
-      atomicAdd(a.acc, local);
-      atomicAdd(a.acc_level, local);
-    }
-    if (items && walked) atomicAdd(items, walked);
-  }
+  BlockAdd<kThreads>(Into{a.acc, local}, Into{a.acc_level, local}, Into{items, walked});
 }
 
 // --------------------------------------------------------------------------
@@ -1329,17 +1304,7 @@ __global__ __launch_bounds__(kThreads) void GroupCountKernel(GroupCountArgs a) {
     }
   }
   if (a.bk.bounds) BucketFlush(a.bk, &bacc);
-  local = WaveSum(local);
-  lower = WaveSum(lower);
-  walked = WaveSum(walked);
-  if (lane == 0) {
-    if (local) {
-      atomicAdd(a.acc, local);
-      atomicAdd(a.acc_level, local);
-    }
-    if (a.walked && walked) atomicAdd(a.walked, walked);
-    if (a.lower && lower) atomicAdd(a.lower, lower);
-  }
+  BlockAdd<kThreads>(Into{a.acc, local}, Into{a.acc_level, local}, Into{a.walked, walked}, Into{a.lower, lower});
 }
 
 __global__ __launch_bounds__(kThreads) void UpperStartKernel(const uint64_t* rp, const uint32_t* cols,
@@ -1398,7 +1363,7 @@ void LaunchPrepTwo(const PrepTwoArgs& a, hipStream_t stream) {
 
 void LaunchCountPaths(const CountPathArgs& a, hipStream_t stream) {
   if (a.npaths == 0) return;
-  hipLaunchKernelGGL(CountPathsKernel, dim3(GridFor(a.npaths, kThreads)), dim3(kThreads), 0, stream, a);
+  hipLaunchKernelGGL(CountPathsKernel, dim3(GridFor(a.npaths, kThreads, 2048)), dim3(kThreads), 0, stream, a);
 }
 
 void LaunchChunkPartition(const uint64_t* offs, uint64_t nseg, uint64_t nchunks, uint32_t* chunk_seg,

@@ -183,11 +183,7 @@ __global__ __launch_bounds__(kThreads) void PathRunKernel(PathRunArgs a) {
     }
   }
   if (a.bk.bounds && a.acc) BucketFlush(a.bk, &bacc);
-  total = WaveSum(total);
-  if (lane == 0 && total) {
-    if (a.acc) atomicAdd(a.acc, total);
-    atomicAdd(a.acc_level, total);
-  }
+  BlockAdd<kThreads>(Into{a.acc, total}, Into{a.acc_level, total});
 }
 
 }  // namespace
@@ -197,9 +193,9 @@ void LaunchPathRuns(const PathRunArgs& a, hipStream_t stream) {
   const uint64_t need = (a.npaths + kThreads - 1) / kThreads;
   // 1 KB bitmaps let 32 waves share a CU, 4 KB ones 20
   if (a.n <= 8192)
-    hipLaunchKernelGGL(PathRunKernel<256>, dim3(need < 8192 ? need : 8192), dim3(kThreads), 0, stream, a);
+    hipLaunchKernelGGL(PathRunKernel<256>, dim3(need < 4096 ? need : 4096), dim3(kThreads), 0, stream, a);
   else
-    hipLaunchKernelGGL(PathRunKernel<kPathRunIds / 32>, dim3(need < 8192 ? need : 8192), dim3(kThreads), 0, stream, a);
+    hipLaunchKernelGGL(PathRunKernel<kPathRunIds / 32>, dim3(need < 4096 ? need : 4096), dim3(kThreads), 0, stream, a);
 }
 
 }  // namespace sme

@@ -37,6 +37,40 @@ __device__ __forceinline__ uint32_t WavePrefix(uint32_t v, int lane, uint32_t* t
   return s - v;
 }
 
+// A sum and where it goes (nullptr, the same for all threads: nowhere).
+struct Into {
+  unsigned long long* p;
+  unsigned long long v;
+};
+
+// Adds each sum's v over the workgroup of kThr threads to its *p.  Every
+// thread must reach it.  One atomic instruction per workgroup, thread n for
+// sum n: the counters share a line, and device atomics to it complete about 6
+// ns apart (3.5e6 paths counted by 55,000 waves: 0.67 ms of 0.70 were spent
+// there; 2,048 workgroups with three instructions each: 37 us).
+template <int kThr, class... T>
+__device__ __forceinline__ void BlockAdd(T... sums) {
+  constexpr int N = sizeof...(T);
+  __shared__ unsigned long long part[N][kThr / kWave];
+  const Into in[N] = {sums...};
+  __syncthreads();  // an earlier call's readers are done
+#pragma unroll
+  for (int n = 0; n < N; ++n) {
+    const unsigned long long v = WaveSum(in[n].v);
+    if ((threadIdx.x & (kWave - 1)) == 0) part[n][threadIdx.x / kWave] = v;
+  }
+  __syncthreads();
+  if (threadIdx.x < N) {
+    unsigned long long* p = nullptr;
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+      if (static_cast<int>(threadIdx.x) == n) p = in[n].p;
+    unsigned long long v = 0;
+    for (int w = 0; w < kThr / kWave; ++w) v += part[threadIdx.x][w];
+    if (p && v) atomicAdd(p, v);
+  }
+}
+
 constexpr unsigned long long kNoBucket = ~0ull;
 
 // Bucket of start vertex v: largest k with bounds[k] <= v.

@@ -41,11 +41,6 @@ __device__ __forceinline__ uint64_t Lower(const uint32_t* a, uint64_t lo, uint64
   return lo;
 }
 
-__device__ __forceinline__ void Flush(unsigned long long* acc, int j, u64 v, int lane) {
-  v = WaveSum(v);
-  if (lane == 0 && v) atomicAdd(acc + j, v);
-}
-
 constexpr uint32_t kFlight = 4;                   // loads a lane keeps in flight
 constexpr uint32_t kWalkStep = kFlight * kWave;  // entries per step
 
@@ -246,9 +241,7 @@ __global__ __launch_bounds__(kThreads) void SquareLightKernel(WedgeArgs a) {
     }
   }
   if (a.bk.bounds) BucketFlush(a.bk, &bacc);
-  Flush(a.acc, 0, total, lane);
-  Flush(a.acc, 1, nup, lane);
-  Flush(a.acc, 2, nwedge, lane);
+  BlockAdd<kThreads>(Into{a.acc, total}, Into{a.acc + 1, nup}, Into{a.acc + 2, nwedge});
 }
 
 // ---------------------------------------------------------------------------
@@ -412,15 +405,15 @@ __global__ __launch_bounds__(kThr) void WedgeTileKernel(WedgeArgs a) {
       if (threadIdx.x == 0 && sum_s) atomicAdd(a.bk.counts + BucketOf(a.bk, v), sum_s);
     }
   }
-  Flush(a.acc, 0, total, lane);
+  BlockAdd<kThr>(Into{a.acc, total});
   if (kUse == kWedgeSquare) {
-    Flush(a.acc, 2, c2, lane);
+    BlockAdd<kThr>(Into{a.acc + 2, c2});
   } else if (kUse == kWedgeHouse) {
-    Flush(a.acc, 1, c1, lane);
-    Flush(a.acc, 2, c2, lane);
-    Flush(a.acc, 3, c3, lane);
-    Flush(a.acc, 4, c4, lane);
-    Flush(a.acc, 5, c5, lane);
+    BlockAdd<kThr>(Into{a.acc + 1, c1},
+                   Into{a.acc + 2, c2},
+                   Into{a.acc + 3, c3},
+                   Into{a.acc + 4, c4},
+                   Into{a.acc + 5, c5});
   }
 }
 
