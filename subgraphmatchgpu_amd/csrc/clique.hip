@@ -314,6 +314,21 @@ __global__ __launch_bounds__(kThreads) void CliqueSmallKernel(CliqueArgs a) {
                      Into{K >= 4 ? a.acc + 4 : nullptr, c4},
                      Into{K >= 5 ? a.acc + 5 : nullptr, c5},
                      Into{K >= 6 ? a.acc + 6 : nullptr, c6});
+  if (!a.publish) return;
+  // the sums above were added by threads of wave 0, as is the ticket
+  __shared__ bool last;
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "agent");
+  if (threadIdx.x == 0) last = atomicAdd(a.done, 1ull) == gridDim.x - 1;
+  __syncthreads();
+  if (!last) return;
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "agent");
+  if (threadIdx.x <= static_cast<unsigned>(kCliqueMaxK)) {
+    a.publish[threadIdx.x] = atomicAdd(a.acc + threadIdx.x, 0ull);
+    a.acc[threadIdx.x] = 0;
+  }
+  if (threadIdx.x == 0) *a.done = 0;
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "");  // (these are all of wave 0)
+  if (threadIdx.x == 0) *const_cast<volatile unsigned long long*>(a.publish + kCliqueMaxK + 1) = a.call;
 }
 
 // ---------------------------------------------------------------------------

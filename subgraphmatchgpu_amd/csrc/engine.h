@@ -89,6 +89,20 @@ class Context {
   uint64_t held = 0;
   uint64_t held_peak = 0;
   uint64_t* pinned() { return pinned_; }
+  // kCounters device u64, zero between runs: a run that uses them leaves them
+  // zero, a failed one has them cleared (ClearCounters)
+  static constexpr int kCounters = 16;
+  unsigned long long* counters() { return counters_; }
+  // where in pinned() kernels write results themselves; nothing else is copied
+  // there (a stale value could pass for a call number)
+  static constexpr int kPublish = 496;
+  void ClearCounters();
+  // Waits until the device has written `call` to pinned()[at] (within the part
+  // from kPublish on), or the stream
+  // is idle: a short launch is seen by its write several us before the runtime
+  // reports the stream idle.
+  void WaitFor(int at, uint64_t call);
+  uint64_t next_call() { return ++calls_; }
 
   // hub adjacency bitmaps for graphs uploaded from now on: vertices of
   // degree >= hub_min_degree, highest degree first, at most hub_max_bytes
@@ -163,6 +177,8 @@ class Context {
   DevicePool own_pool_;
   DevicePool* pool_ = &own_pool_;
   uint64_t* pinned_ = nullptr;
+  unsigned long long* counters_ = nullptr;
+  uint64_t calls_ = 0;
 };
 
 class DevGraph {

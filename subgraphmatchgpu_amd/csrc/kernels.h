@@ -358,6 +358,12 @@ struct CliqueArgs {
   // big / huge are null: the caller holds these lists already).
   uint32_t v_begin, v_end;
   uint32_t group;                // start vertices per wave step (set by the launcher)
+  // nullable: the last workgroup to end writes acc[0 .. kCliqueMaxK] to publish
+  // (host memory the device sees), clears them and *done (zero before), and
+  // then writes `call` behind them
+  unsigned long long* publish;
+  unsigned long long* done;
+  unsigned long long call;
   uint32_t* big;
   uint32_t* big_d;
   unsigned long long* nbig;

@@ -276,3 +276,17 @@ def test_emu_path_runs(emu, q):
                           (key % g.n).astype(np.uint32))
         want = oracle.light_count(g.row_ptrs, g.cols, q, 3)
         assert emu(g, q) == (want[0], want[1])
+
+
+@pytest.mark.gpu
+def test_small_calls_in_a_row(dev):
+    """Calls whose kernel hands its sums to the host itself, among others that copy theirs, keep apart."""
+    gs = [sme.gen_er(n, 3 * n, seed=n) for n in (5, 64, 300, 1000)] + [small_graphs(0)]
+    up = [(g, dev.upload(g)) for g in gs]
+    want = {(i, q): oracle.light_count(g.row_ptrs, g.cols, q, 3) for i, (g, _) in enumerate(up) for q in (0, 1, 3, 7)}
+    for k in range(200):
+        i, q = k % len(up), (0, 3, 1, 0, 7)[k % 4]
+        r = dev.count(up[i][1], sme.Plan(q))
+        assert (r.count, r.levels) == (want[i, q][0], want[i, q][1]), (k, i, q)
+    for _, dg in up:
+        dg.release()
