@@ -808,34 +808,6 @@ __device__ __forceinline__ void FlushSums(unsigned long long* acc, int K, const 
                      Into{K >= 6 ? acc + 6 : nullptr, cs.c6});
 }
 
-// 4-cliques: a wave takes groups of kRowGroup consecutive rows, one search for
-// the group's first vertex, then a walk forward (a row is light next to the
-// search).
-__global__ __launch_bounds__(kThreads) void CliqueCount4Kernel(CliqueArgs a) {
-  __shared__ u64 lds_s[kWaves][kWordsMax];
-  __shared__ uint32_t lds_q[kWaves][2 * kWave];
-  const int lane = threadIdx.x & (kWave - 1);
-  const int wid = threadIdx.x / kWave;
-  const uint64_t wave = (blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x) / kWave;
-  const uint64_t nwaves = static_cast<uint64_t>(gridDim.x) * blockDim.x / kWave;
-  CliqueSums cs;
-  constexpr uint64_t kRowGroup = 16;
-  const uint64_t base = a.row_first[0];
-  for (uint64_t t0 = wave * kRowGroup; t0 < a.nitems; t0 += nwaves * kRowGroup) {
-    const uint64_t te = t0 + kRowGroup < a.nitems ? t0 + kRowGroup : a.nitems;
-    uint64_t x = ItemVertexWave(a, t0, lane);
-    for (uint64_t t = t0; t < te; ++t) {
-      while (a.row_first[x + 1] - base <= t) ++x;
-      const uint32_t d = static_cast<uint32_t>(a.row_first[x + 1] - a.row_first[x]);
-      const uint32_t i = static_cast<uint32_t>(t - (a.row_first[x] - base));
-      const u64* rows = a.rows + (a.word_first[x] - a.word_first[0]);
-      const u64 vk = CountRow<4>(rows, d, i, lds_s[wid], nullptr, nullptr, lds_q[wid], lane, &cs);
-      if (a.bk.bounds) AddBucket(a.bk, a.verts[x], vk, lane);
-    }
-  }
-  FlushSums(a.acc, 4, cs);
-}
-
 // 5- and 6-cliques.  The m members of row i span W words, most of whose bits
 // are not members.  Their rows are first packed to the members' columns: lane =
 // member j reads the words of row j, and for each set bit of row i (the same
@@ -855,7 +827,7 @@ __global__ __launch_bounds__(kThreads) void CliqueCount4Kernel(CliqueArgs a) {
 
 // Words between packed rows of NW words: 16-byte aligned from 4 words on, and
 // an odd multiple of 4 so that 64 rows spread over 16 banks.
-constexpr uint32_t PackStride(int nw) { return nw < 4 ? nw : nw == 4 ? 4 : nw + 4; }
+constexpr uint32_t PackStride(int nw) { return nw < 4 ? nw : nw % 8 == 4 ? nw : nw + 4; }
 
 // Packs the rows of members r = lane + 64 g (j = mem[r], r < m), g < G, taking
 // the words [w0, w1) of row i (s1), whose first set bit is packed bit `pos`.
@@ -991,6 +963,69 @@ __device__ __forceinline__ u64 CountWave(const u64* rows, uint32_t d, uint32_t i
   for (uint32_t r = 0; r < m; r += kWave)
     vk += K == 5 ? CountPacked5<NW>(pack, m, r + lane, r, 1, 0, cs) : CountPacked6<NW>(pack, m, r + lane, cs);
   return vk;
+}
+
+// 4-cliques of the vertices with d > kDenseMax: a wave takes groups of
+// kRowGroup consecutive rows, one search for the group's first vertex, then a
+// walk forward (a row is light next to the search).
+__global__ __launch_bounds__(kThreads) void CliqueCount4Kernel(CliqueArgs a) {
+  __shared__ u64 lds_s[kWaves][kWordsMax];
+  __shared__ uint32_t lds_q[kWaves][2 * kWave];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wid = threadIdx.x / kWave;
+  const uint64_t wave = (blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x) / kWave;
+  const uint64_t nwaves = static_cast<uint64_t>(gridDim.x) * blockDim.x / kWave;
+  CliqueSums cs;
+  constexpr uint64_t kRowGroup = 16;
+  const uint64_t base = a.row_first[0];
+  for (uint64_t t0 = wave * kRowGroup; t0 < a.nitems; t0 += nwaves * kRowGroup) {
+    const uint64_t te = t0 + kRowGroup < a.nitems ? t0 + kRowGroup : a.nitems;
+    uint64_t x = ItemVertexWave(a, t0, lane);
+    for (uint64_t t = t0; t < te; ++t) {
+      while (a.row_first[x + 1] - base <= t) ++x;
+      const uint32_t d = static_cast<uint32_t>(a.row_first[x + 1] - a.row_first[x]);
+      const uint32_t i = static_cast<uint32_t>(t - (a.row_first[x] - base));
+      const u64* rows = a.rows + (a.word_first[x] - a.word_first[0]);
+      const u64 vk = CountRow<4>(rows, d, i, lds_s[wid], nullptr, nullptr, lds_q[wid], lane, &cs);
+      if (a.bk.bounds) AddBucket(a.bk, a.verts[x], vk, lane);
+    }
+  }
+  FlushSums(a.acc, 4, cs);
+}
+
+// 4-cliques of the vertices with 32 (NW - 4) < d <= 32 NW: the pairs and
+// triangles of the graph on N+(v), whose d rows one workgroup reads once, in
+// order, into LDS.
+//
+// Bound by VALU issue.  R-MAT scale 20 (60,395 vertices): 1.0 ms with the few above kDenseMax; one wave
+// per row, probing its members' rows in device memory, took 3.2.  Meeting every
+// row, member or not, costs d^2 / 128 steps of a wave against one per 64
+// members: above kDenseMax the members are few enough that probing them wins.
+template <int NW>
+__global__ __launch_bounds__(kThreads) void CliqueDenseKernel(CliqueArgs a) {
+  constexpr uint32_t S = PackStride(NW);
+  __shared__ __align__(16) uint32_t pack[32 * NW * S];
+  const int lane = threadIdx.x & (kWave - 1);
+  const uint32_t wid = threadIdx.x / kWave;
+  CliqueSums cs;
+  for (uint64_t x = blockIdx.x; x < a.nverts; x += gridDim.x) {
+    const uint32_t d = static_cast<uint32_t>(a.row_first[x + 1] - a.row_first[x]);
+    const uint32_t W = (d + 63) / 64;
+    const u64* rows = a.rows + (a.word_first[x] - a.word_first[0]);
+    __syncthreads();  // the previous vertex's readers are done
+    for (uint32_t w = 0; w < NW / 2; ++w)
+      for (uint32_t i = threadIdx.x; i < d; i += kThreads) {
+        const u64 y = w < W ? rows[static_cast<uint64_t>(w) * d + i] : 0;
+        pack[i * S + 2 * w] = static_cast<uint32_t>(y);
+        pack[i * S + 2 * w + 1] = static_cast<uint32_t>(y >> 32);
+      }
+    __syncthreads();
+    u64 vk = 0;
+    for (uint32_t r = 0; r < d; r += kWave) vk += CountPacked5<NW>(pack, d, r + lane, r, kWaves, wid, &cs);
+    if (a.bk.bounds) AddBucket(a.bk, a.verts[x], vk, lane);
+  }
+  // (pairs of the graph on N+(v) are triangles, its triangles 4-cliques)
+  BlockAdd<kThreads>(Into{a.acc + 3, cs.c4}, Into{a.acc + 4, cs.c5});
 }
 
 // Row i into s1 (LDS), its members in order into mem (at most cap); returns
@@ -1162,6 +1197,17 @@ void LaunchCliqueRowsHash(const CliqueArgs& a, bool small_table, hipStream_t str
     hipLaunchKernelGGL(CliqueRowsHashKernel<10>, grid, block, 0, stream, a);
   else
     hipLaunchKernelGGL(CliqueRowsHashKernel<13>, grid, block, 0, stream, a);
+}
+
+void LaunchCliqueDense(const CliqueArgs& a, int words, hipStream_t stream) {
+  if (a.nverts == 0) return;
+  const dim3 grid(Grid(a.nverts, 1)), block(kThreads);
+  switch (words) {
+    case 4: hipLaunchKernelGGL(CliqueDenseKernel<4>, grid, block, 0, stream, a); break;
+    case 8: hipLaunchKernelGGL(CliqueDenseKernel<8>, grid, block, 0, stream, a); break;
+    case 12: hipLaunchKernelGGL(CliqueDenseKernel<12>, grid, block, 0, stream, a); break;
+    case 16: hipLaunchKernelGGL(CliqueDenseKernel<16>, grid, block, 0, stream, a); break;
+  }
 }
 
 void LaunchCliqueCount(const CliqueArgs& a, hipStream_t stream) {

@@ -1730,7 +1730,26 @@ void LocalCliqueRange(Context* ctx, const DevGraph* g, const EnginePlan* plan, u
         // every row word read at least once
         Timed t(ctx, s, kSlotCliqueCount, 8.0 * static_cast<double>(words), a.nitems);
         if (K > 4) LaunchFill64(reinterpret_cast<uint64_t*>(a.nlong), 2, 0, s);
-        LaunchCliqueCount(a, s);
+        CliqueArgs b = a;
+        // 4-cliques: up to kDenseMax by whole vertices, in classes of d
+        uint64_t rest = x1;
+        for (int words = 4; K == 4 && words <= static_cast<int>(kDenseMax / 32); words += 4) {
+          const uint32_t over = 32u * static_cast<uint32_t>(words);
+          const uint64_t from = std::partition_point(hd_sorted.begin() + x0, hd_sorted.begin() + rest,
+                                                     [over](uint32_t d) { return d > over; }) -
+                                hd_sorted.begin();
+          b.verts = dverts + from;
+          b.nverts = rest - from;
+          b.row_first = drf + from;
+          b.word_first = dwf + from;
+          b.rows = rows.get() + (wf[from] - wf[x0]);
+          LaunchCliqueDense(b, words, s);
+          rest = from;
+        }
+        b = a;
+        b.nverts = rest - x0;
+        b.nitems = rf[rest] - rf[x0];
+        LaunchCliqueCount(b, s);
       }
       st->batches++;
       x0 = x1;

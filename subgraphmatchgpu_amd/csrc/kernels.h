@@ -467,6 +467,10 @@ constexpr uint32_t kRowsHashMax = 4096;
 constexpr uint32_t kRowsHashSmall = 512;
 void LaunchCliqueRowsHash(const CliqueArgs& a, bool small_table, hipStream_t stream);
 void LaunchCliqueCount(const CliqueArgs& a, hipStream_t stream);
+// 4-cliques of vertices with 32 (words - 4) < d <= 32 words, words 4, 8, 12 or
+// 16 (verts, nverts, row_first, word_first and rows of those vertices).
+constexpr uint32_t kDenseMax = 512;
+void LaunchCliqueDense(const CliqueArgs& a, int words, hipStream_t stream);
 
 // ---------------------------------------------------------------------------
 // Wedges counted per start vertex (wedge.hip).  On a symmetric graph without

@@ -290,3 +290,24 @@ def test_small_calls_in_a_row(dev):
         assert (r.count, r.levels) == (want[i, q][0], want[i, q][1]), (k, i, q)
     for _, dg in up:
         dg.release()
+
+
+# upper neighbourhoods at the classes of the dense 4-clique count: 128, 256, 384 and 512 rows, beyond
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [65, 127, 128, 129, 256, 257, 384, 385, 512, 513])
+def test_dense_rows(dev, d):
+    rng = np.random.default_rng(d)
+    inner = sme.gen_er(d, min(d * (d - 1) // 2, 14 * d), seed=d)
+    first = clique(2)  # vertex 0 below all of them
+    src = np.repeat(np.arange(d), np.diff(inner.row_ptrs.astype(np.int64))) + 1
+    key = np.unique(np.concatenate([src * (d + 1) + inner.cols + 1, np.arange(1, d + 1),
+                                    np.arange(1, d + 1) * (d + 1)]))
+    g = sme.Graph(np.searchsorted(key, np.arange(d + 2) * (d + 1)).astype(np.uint64), (key % (d + 1)).astype(np.uint32))
+    g = union(g, first, sme.gen_er(150, 6000 + int(rng.integers(50)), seed=d))
+    want = oracle.light_count(g.row_ptrs, g.cols, 3, 3)
+    assert on_gpu(dev, g, 3) == (want[0], want[1])
+    bounds = [0, 1, d // 2, g.n]
+    dg = dev.upload(g)
+    got = dev.count_buckets(dg, sme.Plan(3), bounds)[0].tolist()
+    dg.release()
+    assert got == [oracle.light_count(g.row_ptrs, g.cols, 3, 3, v_begin=a, v_end=b)[0] for a, b in zip(bounds, bounds[1:])]
