@@ -84,7 +84,7 @@ __device__ __forceinline__ void AddBucket(const BucketRef& b, uint32_t v, u64 pe
 // wave per start vertex, searching one row after another with most lanes
 // idle, took 10.2 ms on 1,000 packed G(n, m) members (5.4e7 entries, 13 per
 // vertex) and 3.7 ms on R-MAT scale 20 (degree-ranked, 6 per vertex); the
-// flat items take 3.1 and 1.4 ms.  Groups of 8 or 16 start vertices were
+// flat items take 2.4 and 1.1 ms.  Groups of 8 or 16 start vertices were
 // slower (1.6, 1.7 ms on R-MAT: the heavy groups end last), and so was
 // choosing the mode on rem * steps < len (67 against 87 us, R-MAT scale 14).
 constexpr uint32_t kSmallGroup = 4;  // start vertices per wave step
@@ -109,8 +109,11 @@ struct SmallLds {
   uint32_t cnt[kWave];    // entry: triangles (per-edge counts or buckets)
 };
 
+// (8 waves per SIMD: at the 67 registers of free choice a CU holds 7 of the 8
+// workgroups it is given, and the last ones run alone: 3.1 against 2.4 ms on the
+// packed members, 1.37 against 1.12 on R-MAT scale 20.)
 template <int K>
-__global__ __launch_bounds__(kThreads) void CliqueSmallKernel(CliqueArgs a) {
+__global__ __launch_bounds__(kThreads, 8) void CliqueSmallKernel(CliqueArgs a) {
   __shared__ SmallLds lds_all[kWaves];
   const int lane = threadIdx.x & (kWave - 1);
   SmallLds& s = lds_all[threadIdx.x / kWave];
@@ -458,6 +461,7 @@ __global__ __launch_bounds__(kThreads) void CliqueRowsTableKernel(CliqueArgs a) 
   const int lane = threadIdx.x & (kWave - 1);
   const uint32_t wid = threadIdx.x / kWave;
   u64* row = lds_row[kMode == kRowsBits ? wid : 0];
+  uint32_t* row32 = reinterpret_cast<uint32_t*>(row);
   u64 c3 = 0;
   for (uint64_t x = blockIdx.x; x < a.nverts; x += gridDim.x) {
     const uint32_t v = a.verts[x];
@@ -518,16 +522,17 @@ __global__ __launch_bounds__(kThreads) void CliqueRowsTableKernel(CliqueArgs a) 
           // every entry lies above u_i, so above base
           const uint32_t o0 = x0 - base, o1 = x1 - base;
           const u64 t0 = o0 < range ? tab[o0 >> 5] : 0, t1 = o1 < range ? tab[o1 >> 5] : 0;
-  #pragma unroll
+#pragma unroll
           for (int h = 0; h < 2; ++h) {
             const uint32_t o = h ? o1 : o0;
             const u64 t = h ? t1 : t0;
-            if (!((t >> (o & 31)) & 1)) continue;
+            const uint32_t members = static_cast<uint32_t>(t);  // (shifts take o & 31)
+            if (!((members >> (o & 31)) & 1u)) continue;
             ++bits;
             if (kMode == kRowsCount) continue;
             const uint32_t j = static_cast<uint32_t>(t >> 32) +
-                               static_cast<uint32_t>(__popcll(t & ((1ull << (o & 31)) - 1)));
-            if (kMode == kRowsBits) atomicOr(row + (j >> 6), 1ull << (j & 63));
+                               static_cast<uint32_t>(__builtin_popcount(members & ((1u << (o & 31)) - 1u)));
+            if (kMode == kRowsBits) atomicOr(row32 + (j >> 5), 1u << (j & 31));
             if (kMode == kRowsEdges) {
               atomicAdd(a.tc + lb + e + h * kWave, 1u);  // edge (u_i, u_j)
               atomicAdd(lds_col + (j >> 1), 1u << (16 * (j & 1)));  // edge (v, u_j)

@@ -132,7 +132,7 @@ __device__ __forceinline__ void WalkLists(const uint32_t* cols, const uint32_t* 
 //
 // Bound by the latency of a start vertex's chain (its list, the middles' list
 // bounds, their entries, the LDS adds).  300 packed G(n, m) members (1.25e6
-// vertices, 3.3e7 entries): 2.3 ms, where the level engine wrote every wedge
+// vertices, 3.3e7 entries): 1.8 ms, where the level engine wrote every wedge
 // as a path and intersected two lists for it (52 ms).  Two passes over 4,096
 // ids cover the members (n <= 8,192) at 6 waves per SIMD; a start vertex above
 // kLightItems would hold its wave for over 64 steps and goes to the tiles.
@@ -149,7 +149,7 @@ struct LightLds {
 };
 static_assert(kLightSpan <= kLightSlots * 4, "byte counters fit the keys' place");
 
-__global__ __launch_bounds__(kThreads) void SquareLightKernel(WedgeArgs a) {
+__global__ __launch_bounds__(kThreads, 6) void SquareLightKernel(WedgeArgs a) {
   __shared__ LightLds lds_all[kWaves];
   const int lane = threadIdx.x & (kWave - 1);
   LightLds& s = lds_all[threadIdx.x / kWave];
@@ -489,7 +489,8 @@ void LaunchSquareLight(const WedgeArgs& a, hipStream_t stream) {
   const uint64_t per = nv / 8192;
   b.group = static_cast<uint32_t>(per < 1 ? 1 : per > 16 ? 16 : per);
   const uint64_t need = ((nv + b.group - 1) / b.group + kWaves - 1) / kWaves;
-  hipLaunchKernelGGL(SquareLightKernel, dim3(need < 2048 ? need : 2048), dim3(kThreads), 0, stream, b);
+  // whole rounds of the six workgroups per CU that their LDS allows (2,048: 2.25 ms, 1,536: 1.92, 6,144: 1.82)
+  hipLaunchKernelGGL(SquareLightKernel, dim3(need < 6144 ? need : 6144), dim3(kThreads), 0, stream, b);
 }
 
 uint32_t WedgeTiles(uint32_t n) { return n <= kSmall ? 1 : (n - 1) / kLarge + 1; }
