@@ -198,6 +198,7 @@ class DevGraph {
   bool self_loops = false;
   bool symmetric = false;      // every entry (v, u) has its mirror (u, v)
   bool check_symmetry = true;  // let Upload find out (off for a ranked copy)
+  bool by_degree = false;      // ids are in increasing degree (a ranked copy)
   uint64_t max_degree = 0;     // largest |N(v)|
   uint64_t max_up_degree = 0;  // largest |N+(v)| (neighbours above v)
   // house_work[v]: sum of |N+(u)| |N(u)| over u < v, the (edge, further
@@ -214,6 +215,7 @@ class DevGraph {
     uint64_t* drf = nullptr;
     uint64_t* dwf = nullptr;
     uint64_t* dcf = nullptr;
+    uint32_t first = UINT32_MAX;  // smallest id of verts
     bool wide = false;  // some of verts' N+(v) spans kRowsTableRange ids or more
   } upper;
   int device = -1;

@@ -392,6 +392,7 @@ struct CliqueArgs {
   // cols[p] (p an index of some N+(x)), recorded by CliqueSmallKernel and
   // CliqueRowsKernel as they find each triangle (v, u_i, u_j)
   uint32_t* tc;
+  uint32_t middles;              // see LaunchCliqueMiddles
 };
 // ---------------------------------------------------------------------------
 // House (5-cycle with one chord closing a triangle) counted from edge
@@ -459,6 +460,12 @@ void LaunchCliqueRows(const CliqueArgs& a, hipStream_t stream);
 constexpr uint32_t kRowsTableMax = 4096;
 constexpr uint32_t kRowsTableRange = 65536;
 void LaunchCliqueRowsTable(const CliqueArgs& a, uint32_t dmax, hipStream_t stream);
+// With a.middles the table kernel leaves the middle edges (u, w) of its
+// triangles to this one, for every u with |N+(u)| <= kMiddleMax whose N+(u)
+// spans fewer than kRowsTableRange ids; u in [v_begin, v_end), which must hold
+// every upper neighbour of the table's vertices.  Symmetric graphs.
+constexpr uint32_t kMiddleMax = 1024;
+void LaunchCliqueMiddles(const CliqueArgs& a, hipStream_t stream);
 // Rows of vertices with d <= kRowsHashMax: a workgroup per chunk of 64 rows
 // keeps N+(v) as a hash (value -> local index) in LDS and streams each row
 // vertex's upper list, 64 consecutive entries per load; `small_table`: every

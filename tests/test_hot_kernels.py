@@ -311,3 +311,30 @@ def test_dense_rows(dev, d):
     got = dev.count_buckets(dg, sme.Plan(3), bounds)[0].tolist()
     dg.release()
     assert got == [oracle.light_count(g.row_ptrs, g.cols, 3, 3, v_begin=a, v_end=b)[0] for a, b in zip(bounds, bounds[1:])]
+
+
+def test_emu_middle_edges(emu):
+    """Per-edge counts on the degree-ranked copy: rows from the table, middle edges per u."""
+    g = union(sme.gen_er(150, 7000, seed=3), clique(70), sme.gen_rmat(6, 6, seed=2))
+    want = oracle.light_count(g.row_ptrs, g.cols, 2, 3)
+    assert emu(g, 2, RANK=1) == (want[0], want[1])
+    assert emu(g, 4, RANK=1, NOLEVELS=1)[0] == oracle.light_count(g.row_ptrs, g.cols, 4, 3)[0]
+
+
+# spans and lengths at which u's list leaves the middle pass (1,024 entries, 65,536 ids)
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,stride", [(300, 1), (300, 230), (1100, 1), (80, 900)])
+def test_middle_edges(d, stride):
+    g = union(fan(d * stride + 2, d, stride, 30 * d, d), sme.gen_er(400, 24000, seed=d), clique(90))
+    ranked = sme.Device(0, budget_bytes=2 << 30)
+    ranked.set_rank_order(True)
+    dg = ranked.upload(g)
+    for q in (2, 4):
+        want = oracle.light_count(g.row_ptrs, g.cols, q, 3)
+        print(f"case q={q} d={d} stride={stride}", flush=True)
+        if q == 2:
+            r = ranked.count(dg, sme.Plan(q))
+            assert (r.count, r.levels) == (want[0], want[1])
+        else:
+            assert ranked.count_only(dg, sme.Plan(q)).count == want[0]
+    ranked.close()
