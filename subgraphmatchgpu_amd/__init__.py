@@ -464,10 +464,11 @@ class Device:
         candidates are counted by a whole workgroup each (0: off);
         clique_level_engine -- 1: clique plans run through the level engine
         instead of bitmap counting over each start vertex's upper
-        neighbourhood (0, the default); census_level_engine -- 1: a house
-        count over all start vertices without level outputs runs through the
-        level engine instead of per-edge triangle counts and a 4-cycle wedge
-        walk (0, the default)."""
+        neighbourhood (0, the default); census_level_engine -- 1: 4-cycle
+        and house counts run through the level engine instead of wedge and
+        per-edge triangle counts (0, the default; clique_level_engine 1 also
+        turns these off, but for a house count over all start vertices
+        without level outputs)."""
         t = _Tuning(lane_path_max, item_grid, super_chunks, batch_bytes, stream_ratio, group_max,
                     wg_path_min, clique_level_engine, census_level_engine)
         _check(library().sme_set_tuning(self._h, ctypes.byref(t)), self._h)

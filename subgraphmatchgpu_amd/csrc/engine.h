@@ -139,8 +139,9 @@ class Context {
   //                  neighbourhood (clique.hip); 1: through the level engine
   //   census_level_engine  0 (default): a house count over all start vertices
   //                  without level outputs comes from per-edge triangle
-  //                  counts and a 4-cycle wedge walk (house.hip); 1: the
-  //                  level engine
+  //                  counts and a 4-cycle wedge walk (house.hip), and 4-cycle
+  //                  and house counts over ranges and buckets from wedges per
+  //                  start vertex (wedge.hip); 1: the level engine
   struct Tuning {
     uint64_t lane_path_max = 0;
     uint32_t item_grid = 0;

@@ -640,7 +640,7 @@ __global__ __launch_bounds__(kThreads) void VerifyKernel(ItemArgs a) {
   }
   if (kMode != kModeMask && a.bk.bounds) BucketFlush(a.bk, &bacc);
   if (kMode != kModeMask) {
-    BlockAdd<kThreads>(Into{a.acc, local}, Into{a.acc_level, local});
+    WaveAdd(Into{a.acc, local}, Into{a.acc_level, local});
   }
 }
 
@@ -759,7 +759,7 @@ __global__ __launch_bounds__(kThreads) void PrepCountKernel(PrepCountArgs a) {
     }
   }
   if (a.it.bk.bounds) BucketFlush(a.it.bk, &bacc);
-  BlockAdd<kThreads>(Into{a.it.acc, local}, Into{a.it.acc_level, local}, Into{a.lane_items, nlane});
+  WaveAdd(Into{a.it.acc, local}, Into{a.it.acc_level, local}, Into{a.lane_items, nlane});
 }
 
 __device__ __forceinline__ uint64_t RankOf(const RankRef& r, uint64_t t) {
@@ -1304,7 +1304,7 @@ __global__ __launch_bounds__(kThreads) void GroupCountKernel(GroupCountArgs a) {
     }
   }
   if (a.bk.bounds) BucketFlush(a.bk, &bacc);
-  BlockAdd<kThreads>(Into{a.acc, local}, Into{a.acc_level, local}, Into{a.walked, walked}, Into{a.lower, lower});
+  WaveAdd(Into{a.acc, local}, Into{a.acc_level, local}, Into{a.walked, walked}, Into{a.lower, lower});
 }
 
 __global__ __launch_bounds__(kThreads) void UpperStartKernel(const uint64_t* rp, const uint32_t* cols,

@@ -71,6 +71,27 @@ __device__ __forceinline__ void BlockAdd(T... sums) {
   }
 }
 
+// The same by each wave alone, for kernels whose waves end at very different
+// times: a wave that waits for its workgroup keeps its place from the next one
+// (the pair counts of the solar square on R-MAT scale 12: 25.0 against 23.7 ms).
+template <class... T>
+__device__ __forceinline__ void WaveAdd(T... sums) {
+  constexpr int N = sizeof...(T);
+  const Into in[N] = {sums...};
+  const int lane = threadIdx.x & (kWave - 1);
+  unsigned long long* p = nullptr;
+  unsigned long long mine = 0;
+#pragma unroll
+  for (int n = 0; n < N; ++n) {
+    const unsigned long long v = WaveSum(in[n].v);
+    if (lane == n) {
+      p = in[n].p;
+      mine = v;
+    }
+  }
+  if (p && mine) atomicAdd(p, mine);
+}
+
 constexpr unsigned long long kNoBucket = ~0ull;
 
 // Bucket of start vertex v: largest k with bounds[k] <= v.
