@@ -149,17 +149,18 @@ KERNEL_NAMES = {
     "intersect_group": "intersect_group (GroupCountKernel)",
     "intersect_lane": "intersect_lane (PrepCountKernel)",
     "clique_small": "clique_small (CliqueSmallKernel)",
-    "clique_rows": "clique_rows (CliqueRowsHashKernel<10> + <13>; CliqueRowsKernel above 4,096)",
-    "clique_count": "clique_count (CliqueCountKernel)",
+    "clique_rows": "clique_rows (CliqueRowsTableKernel; CliqueMiddleKernel for per-edge counts; CliqueRowsHashKernel "
+                   "where a neighbourhood spans 65,536 ids or more, CliqueRowsKernel above 4,096)",
+    "clique_count": "clique_count (CliqueDenseKernel, CliqueCount4Kernel; CliquePackKernel, CliqueLongKernel)",
     "house_mirror": "house_mirror (HouseMirrorKernel / EdgePairsKernel)",
-    "house_wedge": "house_wedge (HouseWedgeHashKernel / HouseWedgeDenseKernel)",
+    "house_wedge": "house_wedge (HouseWedgeHashKernel, WedgeTileKernel, HouseWedgeDenseKernel; SquareLightKernel)",
 }
 # Revision of the intersect kernel's memory behaviour; a committed traffic
 # figure is used only when it was measured on the same revision.
-KERNEL_REV = "clique-bitmaps-hash-rows-word-major-ldscol-pipelined"
+KERNEL_REV = "clique-rows-table-middles"
 
 
-def summarize_pmc(fetch_csv, write_csv, calib_bytes, kernel="CliqueRowsHashKernel", per_launch=1):
+def summarize_pmc(fetch_csv, write_csv, calib_bytes, kernel="CliqueRowsTableKernel", per_launch=1):
     """HBM bytes per launch of `kernel` from two rocprofv3 --pmc runs
     (FETCH_SIZE, then WRITE_SIZE, KiB per dispatch), each scaled by what the
     same counter read for the calibration copy of calib_bytes (the largest
@@ -231,11 +232,11 @@ def main():
                     help="rmat20: no degree-ranked copy (clique counts then walk the original ids)")
     ap.add_argument("--summarize-pmc", nargs="+", metavar="ARG",
                     help="FETCH_CSV WRITE_CSV CALIB_MIB [KERNEL]: print HBM traffic per launch of KERNEL "
-                         "(default GroupCountKernel) from two rocprofv3 --pmc runs")
+                         "(default CliqueRowsTableKernel) from two rocprofv3 --pmc runs")
     args = ap.parse_args()
     if args.summarize_pmc:
         f, w, mib = args.summarize_pmc[:3]
-        kernel = args.summarize_pmc[3] if len(args.summarize_pmc) > 3 else "CliqueRowsHashKernel"
+        kernel = args.summarize_pmc[3] if len(args.summarize_pmc) > 3 else "CliqueRowsTableKernel"
         per = int(args.summarize_pmc[4]) if len(args.summarize_pmc) > 4 else 1
         print(json.dumps(summarize_pmc(f, w, int(mib) << 20, kernel, per)))
         return
