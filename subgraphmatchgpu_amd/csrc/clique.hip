@@ -1189,17 +1189,15 @@ __global__ __launch_bounds__(kThreads) void CliquePackKernel(CliqueArgs a) {
   FlushSums(a.acc, K, cs);
 }
 
-// The long rows: 5-cliques of a row with at most 32 NW members by a workgroup,
-// each wave packing a share of the columns and meeting a share of the rows; the
-// others (longer, and all of 6-cliques, NW = 0) unpacked by its first wave.
-// kBack: the rows from the back of the list.
-template <int K, int NW, bool kBack>
+// 5-cliques of the long rows with at most 32 NW members, one workgroup each,
+// every wave packing a share of the columns and meeting a share of the rows.
+// kBack: the rows from the back of the list (longer ones among them are left to
+// CliqueUnpackedKernel).
+template <int NW, bool kBack>
 __global__ __launch_bounds__(kThreads) void CliqueLongKernel(CliqueArgs a) {
-  constexpr uint32_t kCap = NW ? 32 * NW : 1;
-  constexpr bool kUnpacked = kBack;
-  __shared__ u64 lds_s[kUnpacked ? K - 3 : 1][kWordsMax];
-  __shared__ uint32_t lds_q[kUnpacked ? 2 * kWave : 1];
-  __shared__ __align__(16) uint32_t pack[NW ? PackStride(NW) * kCap : 4];
+  constexpr uint32_t kCap = 32 * NW;
+  __shared__ u64 s1[kWordsMax];
+  __shared__ __align__(16) uint32_t pack[PackStride(NW) * kCap];
   __shared__ uint16_t mem[kCap];
   __shared__ uint32_t members;
   const int lane = threadIdx.x & (kWave - 1);
@@ -1215,30 +1213,57 @@ __global__ __launch_bounds__(kThreads) void CliqueLongKernel(CliqueArgs a) {
     const u64* rows = a.rows + (a.word_first[x] - a.word_first[0]);
     __syncthreads();  // the previous row's readers are done
     if (wid == 0) {
-      const uint32_t m = LoadRow(rows, d, i, lds_s[0], mem, kCap, lane);
+      const uint32_t m = LoadRow(rows, d, i, s1, mem, kCap, lane);
       if (lane == 0) members = m;
     }
-    if (NW)
-      for (uint32_t k = threadIdx.x; k < PackStride(NW ? NW : 1) * kCap; k += kThreads) pack[k] = 0;
+    for (uint32_t k = threadIdx.x; k < PackStride(NW) * kCap; k += kThreads) pack[k] = 0;
     __syncthreads();
     const uint32_t m = members;
+    if (m > kCap) continue;
+    if (threadIdx.x == 0) cs.c3 += m;
+    const uint32_t W = (d + 63) / 64, lo1 = (i + 1) >> 6;
+    const uint32_t share = (W - lo1 + kWaves - 1) / kWaves;
+    const uint32_t w0 = lo1 + wid * share < W ? lo1 + wid * share : W, w1 = w0 + share < W ? w0 + share : W;
+    uint32_t pos = 0;
+    for (uint32_t w = lo1; w < w0; ++w) pos += static_cast<uint32_t>(__popcll(First64(s1[w])));
+    PackRows<(NW + 1) / 2, NW>(rows, d, s1, w0, w1, pos, mem, m, pack, lane);
+    __syncthreads();
     u64 vk = 0;
-    if (kUnpacked && (m > kCap || !NW)) {
-      if (wid == 0)
-        vk = CountRow<K>(rows, d, i, lds_s[0], lds_s[kUnpacked ? 1 : 0], lds_s[kUnpacked && K > 5 ? 2 : 0], lds_q, lane,
-                         &cs);
-    } else if (NW) {
-      if (threadIdx.x == 0) cs.c3 += m;
-      const uint32_t W = (d + 63) / 64, lo1 = (i + 1) >> 6;
-      const uint32_t share = (W - lo1 + kWaves - 1) / kWaves;
-      const uint32_t w0 = lo1 + wid * share < W ? lo1 + wid * share : W, w1 = w0 + share < W ? w0 + share : W;
-      uint32_t pos = 0;
-      for (uint32_t w = lo1; w < w0; ++w) pos += static_cast<uint32_t>(__popcll(First64(lds_s[0][w])));
-      PackRows<NW ? (NW + 1) / 2 : 1, NW ? NW : 1>(rows, d, lds_s[0], w0, w1, pos, mem, m, pack, lane);
-      __syncthreads();
-      for (uint32_t r = 0; r < m; r += kWave)
-        vk += CountPacked5<NW ? NW : 1>(pack, m, r + lane, r, kWaves, wid, &cs);
+    for (uint32_t r = 0; r < m; r += kWave) vk += CountPacked5<NW>(pack, m, r + lane, r, kWaves, wid, &cs);
+    if (a.bk.bounds) AddBucket(a.bk, a.verts[x], vk, lane);
+  }
+  FlushSums(a.acc, 5, cs);
+}
+
+// The rows at the back of the list that are not packed, one wave each: 5-clique
+// rows with more than kPackLong members, and all long rows of 6-cliques.
+constexpr uint32_t kPackLong = 512;
+
+template <int K>
+__global__ __launch_bounds__(kThreads) void CliqueUnpackedKernel(CliqueArgs a) {
+  constexpr int kBufs = K - 3;
+  __shared__ u64 lds_s[kWaves][kBufs][kWordsMax];
+  __shared__ uint32_t lds_q[kWaves][2 * kWave];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wid = threadIdx.x / kWave;
+  const uint64_t wave = (blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x) / kWave;
+  const uint64_t nwaves = static_cast<uint64_t>(gridDim.x) * blockDim.x / kWave;
+  CliqueSums cs;
+  const uint64_t base = a.row_first[0];
+  const uint64_t nlong = a.nlong[1];
+  for (uint64_t y = wave; y < nlong; y += nwaves) {
+    const uint64_t t = a.long_rows[a.nitems - 1 - y];
+    const uint64_t x = ItemVertexWave(a, t, lane);
+    const uint32_t d = static_cast<uint32_t>(a.row_first[x + 1] - a.row_first[x]);
+    const uint32_t i = static_cast<uint32_t>(t - (a.row_first[x] - base));
+    const u64* rows = a.rows + (a.word_first[x] - a.word_first[0]);
+    if (K == 5) {
+      u64 m = 0;
+      for (uint32_t w = lane; w < (d + 63) / 64; w += kWave) m += __popcll(rows[static_cast<uint64_t>(w) * d + i]);
+      if (First64(WaveSum(m)) <= kPackLong) continue;
     }
+    const u64 vk = CountRow<K>(rows, d, i, lds_s[wid][0], lds_s[wid][kBufs > 1 ? 1 : 0], lds_s[wid][kBufs > 2 ? 2 : 0],
+                               lds_q[wid], lane, &cs);
     if (a.bk.bounds) AddBucket(a.bk, a.verts[x], vk, lane);
   }
   FlushSums(a.acc, K, cs);
@@ -1318,12 +1343,13 @@ void LaunchCliqueCount(const CliqueArgs& a, hipStream_t stream) {
     case 4: hipLaunchKernelGGL(CliqueCount4Kernel, grid, block, 0, stream, a); break;
     case 5:
       hipLaunchKernelGGL(CliquePackKernel<5>, grid, block, 0, stream, a);
-      hipLaunchKernelGGL((CliqueLongKernel<5, 8, false>), longs, block, 0, stream, a);
-      hipLaunchKernelGGL((CliqueLongKernel<5, 16, true>), longs, block, 0, stream, a);
+      hipLaunchKernelGGL((CliqueLongKernel<8, false>), longs, block, 0, stream, a);
+      hipLaunchKernelGGL((CliqueLongKernel<16, true>), longs, block, 0, stream, a);
+      hipLaunchKernelGGL(CliqueUnpackedKernel<5>, grid, block, 0, stream, a);
       break;
     case 6:
       hipLaunchKernelGGL(CliquePackKernel<6>, grid, block, 0, stream, a);
-      hipLaunchKernelGGL((CliqueLongKernel<6, 0, true>), longs, block, 0, stream, a);
+      hipLaunchKernelGGL(CliqueUnpackedKernel<6>, grid, block, 0, stream, a);
       break;
   }
 }
