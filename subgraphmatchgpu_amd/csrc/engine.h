@@ -93,9 +93,10 @@ class Context {
   // zero, a failed one has them cleared (ClearCounters)
   static constexpr int kCounters = 16;
   unsigned long long* counters() { return counters_; }
-  // where in pinned() kernels write results themselves; nothing else is copied
-  // there (a stale value could pass for a call number)
+  // where in pinned() kernels write results themselves: zero at open, and
+  // nothing else is copied there (a stale value could pass for a call number)
   static constexpr int kPublish = 496;
+  static constexpr size_t kPinnedBytes = 4096;
   void ClearCounters();
   // Waits until the device has written `call` to pinned()[at] (within the part
   // from kPublish on), or the stream

@@ -77,10 +77,12 @@ Status Context::OpenShared(int device, DevicePool* shared, std::string* err) {
     *err = "hipStreamCreate failed";
     return kErrHip;
   }
-  if (hipHostMalloc(reinterpret_cast<void**>(&pinned_), 4096, hipHostMallocDefault) != hipSuccess) {
+  if (hipHostMalloc(reinterpret_cast<void**>(&pinned_), kPinnedBytes, hipHostMallocDefault) != hipSuccess) {
     *err = "hipHostMalloc failed";
     return kErrHip;
   }
+  // the page may come from an earlier context, whose call numbers began at 1 too
+  std::memset(pinned_, 0, kPinnedBytes);
   if (hipMalloc(reinterpret_cast<void**>(&counters_), kCounters * sizeof(uint64_t)) != hipSuccess) {
     *err = "hipMalloc failed";
     return kErrHip;
