@@ -99,9 +99,9 @@ class Context {
   static constexpr size_t kPinnedBytes = 4096;
   void ClearCounters();
   // Waits until the device has written `call` to pinned()[at] (within the part
-  // from kPublish on), or the stream
-  // is idle: a short launch is seen by its write several us before the runtime
-  // reports the stream idle.
+  // from kPublish on): a short launch is seen by its write several us before
+  // the runtime reports the stream idle.  Fails if the stream is idle and the
+  // number is not there (a launch that did not happen).
   void WaitFor(int at, uint64_t call);
   uint64_t next_call() { return ++calls_; }
 

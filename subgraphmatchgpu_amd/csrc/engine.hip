@@ -110,6 +110,9 @@ void Context::WaitFor(int at, uint64_t call) {
     if ((spin & 63) == 63 && std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(100)) break;
   }
   SME_HIP(hipStreamSynchronize(stream_));
+  // the words before it are an earlier call's unless this one came
+  if (*seen != call)
+    Fail(kErrHip, std::string("the counting kernel wrote no result: ") + hipGetErrorString(hipGetLastError()));
 }
 
 void* Context::Alloc(size_t bytes) {

@@ -2,6 +2,7 @@
 // holds before the call may not pass for this call's result.  The linker sends
 // hipHostMalloc and the kernel's launcher here first (--wrap).
 //   publish_test stale    the page comes filled with 1, 2, 3, ...
+//   publish_test dropped  some launches do not happen
 #include <hip/hip_runtime.h>
 
 #include <cstdio>
@@ -13,6 +14,7 @@
 namespace {
 unsigned long long g_fill = 0;      // value of every word of a new pinned page
 bool g_stale = false;               // a launch found its call's number already published
+bool g_drop = false;                // launches do not happen
 }  // namespace
 
 hipError_t RealHostMalloc(void** p, size_t n, unsigned flags) asm("__real__Z13hipHostMallocPPvmj");
@@ -27,7 +29,7 @@ void RealSmall(const sme::CliqueArgs& a, hipStream_t s) asm("__real__ZN3sme17Lau
 void WrapSmall(const sme::CliqueArgs& a, hipStream_t s) asm("__wrap__ZN3sme17LaunchCliqueSmallERKNS_10CliqueArgsEP9EmuStream");
 void WrapSmall(const sme::CliqueArgs& a, hipStream_t s) {
   if (a.publish && a.publish[sme::kCliqueMaxK + 1] == a.call) g_stale = true;
-  RealSmall(a, s);
+  if (!g_drop) RealSmall(a, s);
 }
 
 namespace {
@@ -77,11 +79,30 @@ int Stale() {
   return 0;
 }
 
+// A call without its kernel is an error, and the calls after it are right.
+int Dropped() {
+  sme_ctx* ctx = nullptr;
+  if (sme_open(0, 1 << 20, &ctx) != SME_OK) return 2;
+  for (uint64_t n = 7; n < 19; ++n) {
+    g_drop = n % 4 < 2;
+    uint64_t got = 0;
+    const int rc = Count(ctx, n, &got);
+    if (rc != (g_drop ? SME_ERR_HIP : SME_OK) || (!g_drop && got != n)) {
+      std::fprintf(stderr, "n %llu, launch %d: rc %d count %llu\n", static_cast<unsigned long long>(n), !g_drop, rc,
+                   static_cast<unsigned long long>(got));
+      return 1;
+    }
+  }
+  sme_close(ctx);
+  return 0;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const char* what = argc > 1 ? argv[1] : "";
   if (!std::strcmp(what, "stale")) return Stale();
-  std::fprintf(stderr, "usage: %s stale\n", argv[0]);
+  if (!std::strcmp(what, "dropped")) return Dropped();
+  std::fprintf(stderr, "usage: %s stale|dropped\n", argv[0]);
   return 2;
 }

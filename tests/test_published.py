@@ -19,9 +19,11 @@ def publish_test():
     return os.path.join(EMU_DIR, "publish_test")
 
 
-def test_new_page_holds_no_call_number(publish_test):
-    """Pinned pages that come filled with 1, 2, ..: before its launch no call is published."""
-    r = subprocess.run([publish_test, "stale"], capture_output=True, text=True, timeout=120,
+@pytest.mark.parametrize("what", ["stale", "dropped"])
+def test_published_sums_are_the_calls(publish_test, what):
+    """stale: pinned pages that come filled with 1, 2, ..: before its launch no call is published;
+    dropped: a call whose launch did not happen fails, the calls after it are right."""
+    r = subprocess.run([publish_test, what], capture_output=True, text=True, timeout=120,
                        env=dict(os.environ, ASAN_OPTIONS="detect_leaks=0"))
     assert r.returncode == 0, r.stderr[-2000:]
 
