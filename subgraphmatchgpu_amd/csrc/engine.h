@@ -96,6 +96,7 @@ class Context {
   // where in pinned() kernels write results themselves: zero at open, and
   // nothing else is copied there (a stale value could pass for a call number)
   static constexpr int kPublish = 496;
+  static constexpr int kFlag = 495;  // an upload's
   static constexpr size_t kPinnedBytes = 4096;
   void ClearCounters();
   // Waits until the device has written `call` to pinned()[at] (within the part

@@ -301,20 +301,13 @@ Status DevGraph::Upload(Context* ctx, const uint64_t* row_ptrs, const uint32_t* 
   }
   LaunchUpperStart(rp, cols, nv, up, ctx->stream());
   // (an isomorphic copy is as symmetric as its original)
-  bool checked = false;
-  if (check_symmetry && !loops) {
-    if (uint32_t* flag = static_cast<uint32_t*>(ctx->Alloc(sizeof(uint64_t)))) {
-      LaunchFill32(flag, 1, 0, ctx->stream());
-      LaunchAsymmetric(rp, cols, nv, ne, flag, ctx->stream());
-      uint32_t* pin = reinterpret_cast<uint32_t*>(ctx->pinned());
-      const hipError_t e = hipMemcpyAsync(pin, flag, sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream());
-      ctx->Free(flag, sizeof(uint64_t));
-      SME_HIP(e);
-      checked = true;
-    }
+  volatile uint64_t* flag = ctx->pinned() + Context::kFlag;
+  if (check_symmetry) {
+    *flag = 0;
+    LaunchAsymmetric(rp, cols, nv, ne, ctx->pinned() + Context::kFlag, ctx->stream());
   }
   SME_HIP(hipStreamSynchronize(ctx->stream()));
-  if (checked) symmetric = *reinterpret_cast<uint32_t*>(ctx->pinned()) == 0;
+  if (check_symmetry) symmetric = *flag == 0;
   if (ctx->rank_order && nv) {
     std::vector<uint64_t> rrp;
     std::vector<uint32_t> rcols, new_id;

@@ -530,8 +530,9 @@ void LaunchWedgeTiles(const WedgeArgs& a, int use, hipStream_t stream);
 // tile k, k = 0 .. tiles.
 uint32_t WedgeTiles(uint32_t n);
 void LaunchWedgeCuts(const WedgeArgs& a, uint32_t* cuts, hipStream_t stream);
-// *flag (zero before) becomes 1 unless every entry (v, u) has its mirror (u, v).
-void LaunchAsymmetric(const uint64_t* rp, const uint32_t* cols, uint64_t n, uint64_t nnz, uint32_t* flag,
+// *flag (zero before; host memory the device sees) becomes 1 unless every entry
+// (v, u) has its mirror (u, v).
+void LaunchAsymmetric(const uint64_t* rp, const uint32_t* cols, uint64_t n, uint64_t nnz, uint64_t* flag,
                       hipStream_t stream);
 
 // ---------------------------------------------------------------------------

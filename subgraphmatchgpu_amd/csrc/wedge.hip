@@ -331,7 +331,7 @@ __global__ __launch_bounds__(kThr) void WedgeTileKernel(WedgeArgs a) {
 // 64 consecutive entries per wave; a lane finds its row between those of the
 // wave's first and last entry.
 __global__ __launch_bounds__(kThreads) void AsymmetricKernel(const uint64_t* rp, const uint32_t* cols, uint64_t n,
-                                                             uint64_t nnz, uint32_t* flag) {
+                                                             uint64_t nnz, uint64_t* flag) {
   const int lane = threadIdx.x & (kWave - 1);
   const uint64_t wave = (blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x) / kWave;
   const uint64_t nwaves = static_cast<uint64_t>(gridDim.x) * blockDim.x / kWave;
@@ -357,7 +357,7 @@ __global__ __launch_bounds__(kThreads) void AsymmetricKernel(const uint64_t* rp,
     const uint64_t p = Lower(cols, rp[u], rp[u + 1], v);
     bad = bad || p >= rp[u + 1] || cols[p] != v;
   }
-  if (bad) atomicOr(flag, 1u);
+  if (__ballot(bad) && lane == 0) *flag = 1;
 }
 
 // 16,384 ids: 32 KB of counters, four workgroups per CU; 65,536: 128 KB, one
@@ -422,7 +422,7 @@ void LaunchWedgeTiles(const WedgeArgs& a, int use, hipStream_t stream) {
     LaunchTiles<kWedgeApex>(a, stream);
 }
 
-void LaunchAsymmetric(const uint64_t* rp, const uint32_t* cols, uint64_t n, uint64_t nnz, uint32_t* flag,
+void LaunchAsymmetric(const uint64_t* rp, const uint32_t* cols, uint64_t n, uint64_t nnz, uint64_t* flag,
                       hipStream_t stream) {
   if (nnz == 0) return;
   const uint64_t need = (nnz + kThreads - 1) / kThreads;
