@@ -239,8 +239,8 @@ int sme_plan_vertices(const sme_plan* p);
  *                  is computed from per-edge triangle counts and a
  *                  degree-ordered 4-cycle walk: houses = sum_e t(e) p(e) -
  *                  2 sum_e t(e)(t(e)-1), t(e) and p(e) the triangles and
- *                  4-cycles through edge e (graphs without self-loops, every
- *                  degree below 2^19); a 4-cycle count (Q1, ordering on)
+ *                  4-cycles through edge e (symmetric graphs without
+ *                  self-loops, every degree below 2^19); a 4-cycle count (Q1, ordering on)
  *                  over any start range, with level outputs and per bucket,
  *                  comes from the wedges of each start vertex (symmetric
  *                  graphs without self-loops, every |N+(v)| at most 65,535;

@@ -1839,7 +1839,8 @@ void LocalClique(Context* ctx, const DevGraph* g, const EnginePlan* plan, uint32
 // bit kHouseShift and a sum of at most that many pairs of triangle counts
 // (each below the largest degree) below it, so the largest degree must stay
 // under 2^19; the per-edge triangle pass needs every upper neighbourhood
-// within the clique bitmap path's limit.
+// within the clique bitmap path's limit, and counts belong to edges only where
+// every entry has its mirror.
 // Device bytes the per-edge triangle pass needs at least: the counts, the
 // start-vertex lists of one part and the bit rows of the largest upper
 // neighbourhood.
@@ -1851,7 +1852,7 @@ uint64_t CensusBytes(const DevGraph* g) {
 bool LocalHouseApplies(const Context* ctx, const DevGraph* g, const EnginePlan* plan) {
   // plus the wedge loads and one dense accumulator with its touched list
   return !ctx->tuning.census_level_engine && plan->query_type == 4 && plan->enable_ordering &&
-         !g->self_loops && g->max_degree < (1ull << 19) && g->max_up_degree <= kLocalMax &&
+         g->symmetric && !g->self_loops && g->max_degree < (1ull << 19) && g->max_up_degree <= kLocalMax &&
          CensusBytes(g) + 20 * g->n <= ctx->RunAvailable();
 }
 
@@ -2134,7 +2135,7 @@ void LocalHouseRange(Context* ctx, const DevGraph* g, const EnginePlan* plan, ui
 // isomorphic copy.
 bool LocalDiamondApplies(const Context* ctx, const DevGraph* g, const EnginePlan* plan) {
   return !ctx->tuning.census_level_engine && plan->algo == kAlgoLight && plan->query_type == 2 &&
-         plan->enable_ordering && !g->self_loops && g->max_up_degree <= kLocalMax &&
+         plan->enable_ordering && g->symmetric && !g->self_loops && g->max_up_degree <= kLocalMax &&
          CensusBytes(g) <= ctx->RunAvailable();
 }
 
