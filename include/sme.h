@@ -109,7 +109,8 @@ int sme_graph_hubs(const sme_graph* g, uint64_t* nhub);
  * vertices runs on the copy when the answer cannot differ: a clique plan
  * (Q0, Q3, Q7, Q11), whose count and per-level outputs are all invariant
  * under relabeling, or any plan when level_counts is NULL (a count is
- * invariant).  Listing each instance from its lowest-degree vertex bounds
+ * invariant; of a graph that lists an edge in one direction only, just that
+ * of a plan without ordering).  Listing each instance from its lowest-degree vertex bounds
  * the lists walked (Chiba-Nishizeki orientation).  Start-range, bucketed
  * and match-list calls use the original ids.  Off by default.  No
  * counterpart in the reference, which lists from the lowest id

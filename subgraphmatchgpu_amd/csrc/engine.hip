@@ -2225,9 +2225,11 @@ Status RunPlan(Context* ctx, const DevGraph* g, const EnginePlan* plan, uint32_t
   // A count over all start vertices is the same on any isomorphic copy of
   // the graph, and so are a clique plan's level outputs; the degree-ranked
   // copy walks far shorter lists (each instance is reached from its
-  // lowest-degree vertex first).
-  const bool use_ranked =
-      ranked_ids || (g->ranked && v_begin == 0 && v_end == g->n && (plan->clique || !level_counts));
+  // lowest-degree vertex first).  Not so where an entry lacks its mirror and
+  // the plan orders ids: which end of the edge lists it then matters.
+  const bool invariant = g->symmetric || !plan->enable_ordering;
+  const bool use_ranked = ranked_ids || (g->ranked && invariant && v_begin == 0 && v_end == g->n &&
+                                         (plan->clique || !level_counts));
   const DevGraph* rg = use_ranked ? g->ranked : g;
   const auto t0 = std::chrono::steady_clock::now();
   try {

@@ -365,3 +365,29 @@ def test_one_way_edges(dev, scale, ef, seed):
         assert (r.count, r.levels) == (want[0], want[1]), q
         assert dev.count_only(dg, sme.Plan(q)).count == want[0], q
     dg.release()
+
+
+@pytest.mark.parametrize("scale,ef,seed", ONE_WAY[:2])
+def test_emu_one_way_edges_keep_their_ids(emu, scale, ef, seed):
+    """The ids decide which of a one-way graph's edges a count follows: not on the ranked copy."""
+    g = one_way(sme.gen_rmat(scale, ef, seed=seed))
+    for q in (0, 3, 7):
+        want = oracle.light_count(g.row_ptrs, g.cols, q, 3)
+        assert emu(g, q, RANK=1) == (want[0], want[1])
+    for q in (1, 2, 4, 6, 8):
+        assert emu(g, q, RANK=1, NOLEVELS=1)[0] == oracle.light_count(g.row_ptrs, g.cols, q, 3)[0]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scale,ef,seed", ONE_WAY)
+def test_one_way_edges_keep_their_ids(scale, ef, seed):
+    g = one_way(sme.gen_rmat(scale, ef, seed=seed))
+    d = sme.Device(0, budget_bytes=1 << 30)
+    d.set_rank_order(True)
+    dg = d.upload(g)
+    for q in range(9):
+        want = oracle.light_count(g.row_ptrs, g.cols, q, 3)
+        r = d.count(dg, sme.Plan(q))
+        assert (r.count, r.levels) == (want[0], want[1]), q
+        assert d.count_only(dg, sme.Plan(q)).count == want[0], q
+    d.close()
