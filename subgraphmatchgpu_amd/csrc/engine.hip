@@ -1652,24 +1652,29 @@ void LocalCliqueRange(Context* ctx, const DevGraph* g, const EnginePlan* plan, u
   }
   if (nbig) {
     // batches of whole vertices whose rows fit what the run may use
-    uint64_t cap_words = static_cast<uint64_t>((K > 4 ? 0.7 : 0.9) * static_cast<double>(ctx->RunAvailable())) / 8;
+    const uint64_t avail = ctx->RunAvailable();
+    uint64_t cap_words = static_cast<uint64_t>(0.9 * static_cast<double>(avail)) / 8;
     if (ctx->tuning.batch_bytes) cap_words = std::min<uint64_t>(cap_words, ctx->tuning.batch_bytes / 8);
+    // (the list of long rows of 5- and 6-cliques lies beside them)
+    auto fits = [&](uint64_t words, uint64_t rows) {
+      return words <= cap_words && rows <= kMaxBatchPaths &&
+             (K <= 4 || DevicePool::Rounded(8 * words) + DevicePool::Rounded(4 * rows) <= avail);
+    };
     st->batches = 0;
     // the largest neighbourhoods come first: any whose rows alone exceed
     // the cap join the level engine's start vertices below
     uint64_t first_fit = 0;
-    while (first_fit < nbig && wf[first_fit + 1] - wf[first_fit] > cap_words) ++first_fit;
+    while (first_fit < nbig && !fits(wf[first_fit + 1] - wf[first_fit], hd_sorted[first_fit])) ++first_fit;
     if (first_fit) {
       if (tc) Fail(kErrOom, "bit rows of one start vertex exceed the memory the run may use");
       hh.insert(hh.end(), verts.begin(), verts.begin() + static_cast<int64_t>(first_fit));
     }
     for (uint64_t x0 = first_fit; x0 < nbig;) {
       uint64_t x1 = x0 + 1;
-      while (x1 < nbig && wf[x1 + 1] - wf[x0] <= cap_words && rf[x1 + 1] - rf[x0] <= kMaxBatchPaths) ++x1;
+      while (x1 < nbig && fits(wf[x1 + 1] - wf[x0], rf[x1 + 1] - rf[x0])) ++x1;
       const uint64_t words = wf[x1] - wf[x0];
       // triangles are counted as the rows are found: nothing to keep
       Buf<unsigned long long> rows(ctx, K > 3 ? words : 0);
-      // one row item per row (a row is at least two words)
       Buf<uint32_t> long_rows(ctx, K > 4 ? rf[x1] - rf[x0] : 0);
       a.long_rows = long_rows.get();
       a.verts = dverts + x0;

@@ -391,3 +391,16 @@ def test_one_way_edges_keep_their_ids(scale, ef, seed):
         assert (r.count, r.levels) == (want[0], want[1]), q
         assert d.count_only(dg, sme.Plan(q)).count == want[0], q
     d.close()
+
+
+def test_emu_rows_of_nine_tenths_of_the_memory(emu, tmp_path):
+    """5-clique: vertex 0's rows (500 x 8 words) take four fifths of a 40 KB budget, which they may:
+    one batch of rows and no run of the level engine."""
+    g = fan(502, 500, 1, 3000, 8)
+    want = oracle.light_count(g.row_ptrs, g.cols, 7, 3)
+    assert emu(g, 7, budget=40_000) == (want[0], want[1])
+    path = str(tmp_path / "g.bin")
+    sme.write_bin(path, g)
+    r = subprocess.run([os.path.join(EMU_DIR, "emu_driver"), path, "6", "7", "3", "1", "0", str(g.n), "40000"],
+                       capture_output=True, text=True, env=dict(os.environ, ASAN_OPTIONS="detect_leaks=0"), timeout=600)
+    assert r.stdout.split()[2] == "batches=1"
