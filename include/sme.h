@@ -249,7 +249,8 @@ int sme_plan_vertices(const sme_plan* p);
  *                  over a start range, with level outputs or per bucket,
  *                  likewise from wedges and per-edge triangle counts (every
  *                  degree at most 65,535, the counts within a quarter of the
- *                  memory, and not for a range with under 1/128 of the work);
+ *                  memory, not for a range with under 1/128 of the work, and
+ *                  not where wedges are few for the ids they are spread over);
  *                  1: through the level engine.  Counts and level outputs are identical.
  * Settings apply to every later call on the context; results never depend
  * on them. */

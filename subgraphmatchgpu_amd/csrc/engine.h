@@ -207,6 +207,7 @@ class DevGraph {
   // house_work[v]: sum of |N+(u)| |N(u)| over u < v, the (edge, further
   // neighbour) pairs that house counts from those start vertices look at
   std::vector<uint64_t> house_work;
+  double list_mean = 0;  // mean |N(u)| over the entries u
   // Built at upload for the clique bitmap path over all start vertices:
   // the vertices with kLocalSmall < |N+(v)| <= kLocalMax in decreasing
   // |N+(v)| (ties by id) with prefix sums of their rows, row words and

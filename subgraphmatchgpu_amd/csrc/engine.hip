@@ -6,6 +6,7 @@
 #include <algorithm>
 #include <atomic>
 #include <chrono>
+#include <cmath>
 #include <memory>
 #include <new>
 #include <cstring>
@@ -202,6 +203,7 @@ Status DevGraph::Upload(Context* ctx, const uint64_t* row_ptrs, const uint32_t* 
     max_degree = std::max<uint64_t>(max_degree, e - b);
     max_up_degree = std::max<uint64_t>(max_up_degree, dp);
     house_work[v + 1] = house_work[v] + dp * static_cast<uint64_t>(e - b);
+    list_mean += static_cast<double>(e - b) * static_cast<double>(e - b);
     if (dp > kLocalMax) {
       upper.huge.push_back(static_cast<uint32_t>(v));
     } else if (dp > kLocalSmall) {
@@ -211,6 +213,7 @@ Status DevGraph::Upload(Context* ctx, const uint64_t* row_ptrs, const uint32_t* 
       upper.d.push_back(static_cast<uint32_t>(dp));
     }
   }
+  if (nnz) list_mean /= static_cast<double>(nnz);
   {
     const uint64_t nb = upper.verts.size();
     std::vector<uint32_t> order(nb);
@@ -2092,15 +2095,40 @@ bool HouseLevels(const EnginePlan* plan) {
 // first.  That pass (0.3 ms on R-MAT scale 14) and the walk together beat the
 // level engine unless the range holds only a small share of the work: a third
 // of the start vertices takes 0.82 ms against 12.6, so the engine's time equals
-// the pass's at about a 128th of the work.  The
+// the pass's at about a 128th of the work.  Nor does the walk where a start
+// vertex has little to walk in each tile of ids (HouseTilesPay).  The
 // bytes are held to a quarter of the run's memory, so that a run with little
 // memory stays with the level engine's batches.
+//
+// A tile costs a workgroup its counters and a chain of waits whatever it holds:
+// 24 ns a tile over the whole chip (15 n / 65,536 where one tile holds all ids:
+// no list is cut then).  The engine's time goes with the (edge, further
+// neighbour) pairs: from 0.26 ns each (G(n, m) of degree 8) to 1.1 (R-MAT scale
+// 17, mean list 326), within a factor of two of 0.085 list_mean^0.45.
+//                           tiles   engine     walk      pairs ns / tiles ns
+//   G(300,000, 1.2e6)         5      2.9 ms    35.7 ms   0.07
+//   G(1,048,576, 4.2e6)      16      9.8      401        0.02
+//   G(1,048,576, 1.26e7)     16    169        565        0.28
+//   G(1,048,576, 2.5e7)      16   1073        676        1.5
+//   G(100,000, 8e5)           2      5.4        5.4      0.87
+//   R-MAT 19, factor 1        8     81         56        1.1
+//   R-MAT 20, factor 1       16    246        225        0.80
+//   R-MAT 21, factor 1       32    about 800  901        0.57
+bool HouseTilesPay(const DevGraph* g, uint32_t vb, uint32_t ve) {
+  const uint32_t tiles = WedgeTiles(static_cast<uint32_t>(g->n));
+  if (g->n <= kWedgeSmallIds) return true;
+  const double tile_ns = tiles > 1 ? 24.0 : 15.0 / 65536 * static_cast<double>(g->n);
+  const double pair_ns = 0.085 * std::pow(std::max(1.0, g->list_mean), 0.45);
+  return pair_ns * static_cast<double>(g->house_work[ve] - g->house_work[vb]) >=
+         0.8 * tile_ns * static_cast<double>(ve - vb) * tiles;
+}
+
 bool HouseRangeApplies(const Context* ctx, const DevGraph* g, const EnginePlan* plan, uint32_t vb, uint32_t ve,
                        bool levels) {
   return plan->query_type == 4 && WedgeApplies(ctx, g, plan) && (!levels || HouseLevels(plan)) &&
          g->max_degree <= kWedgeDegreeMax && g->max_up_degree <= kLocalMax &&
          CensusBytes(g) <= ctx->RunAvailable() / 4 && ve > vb &&
-         (g->house_work[ve] - g->house_work[vb]) * 128 >= g->house_work[g->n];
+         (g->house_work[ve] - g->house_work[vb]) * 128 >= g->house_work[g->n] && HouseTilesPay(g, vb, ve);
 }
 
 void LocalHouseRange(Context* ctx, const DevGraph* g, const EnginePlan* plan, uint32_t vb, uint32_t ve,

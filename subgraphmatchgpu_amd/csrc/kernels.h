@@ -526,6 +526,7 @@ void LaunchSquareLight(const WedgeArgs& a, hipStream_t stream);
 // Counts of `use` from heavy[] (or all start vertices): a workgroup per start
 // vertex and tile of ids keeps c in LDS.
 void LaunchWedgeTiles(const WedgeArgs& a, int use, hipStream_t stream);
+constexpr uint32_t kWedgeSmallIds = 16384;  // up to here one tile of a small workgroup
 // Tiles of LaunchWedgeTiles; cuts[v * (tiles + 1) + k] = entries of N(v) below
 // tile k, k = 0 .. tiles.
 uint32_t WedgeTiles(uint32_t n);

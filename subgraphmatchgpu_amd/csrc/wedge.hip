@@ -361,7 +361,7 @@ __global__ __launch_bounds__(kThreads) void AsymmetricKernel(const uint64_t* rp,
 }
 
 // 16,384 ids: 32 KB of counters, four workgroups per CU; 65,536: 128 KB, one
-constexpr uint32_t kSmall = 16384, kLarge = 65536;
+constexpr uint32_t kSmall = kWedgeSmallIds, kLarge = 65536;
 
 __global__ __launch_bounds__(kThreads) void WedgeCutsKernel(WedgeArgs a, uint32_t* cuts) {
   const uint64_t per = a.ntiles + 1, total = per * a.n;

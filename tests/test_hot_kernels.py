@@ -404,3 +404,34 @@ def test_emu_rows_of_nine_tenths_of_the_memory(emu, tmp_path):
     r = subprocess.run([os.path.join(EMU_DIR, "emu_driver"), path, "6", "7", "3", "1", "0", str(g.n), "40000"],
                        capture_output=True, text=True, env=dict(os.environ, ASAN_OPTIONS="detect_leaks=0"), timeout=600)
     assert r.stdout.split()[2] == "batches=1"
+
+
+def slots_used(d, call):
+    """Kernel slots that a call times."""
+    d.profile(True)
+    d.profile_reset()
+    call()
+    used = {k for k, v in d.profile_read().items() if v["launches"]}
+    d.profile(False)
+    return used
+
+
+# a house over start vertices with a few neighbours each, spread over several tiles of ids (and, for
+# the largest degree, enough of them): the level engine; over a hub alone: the tiles
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,d,m,tiles", [(70001, 1000, 140000, False), (60000, 1000, 120000, False),
+                                         (300000, 3000, 600000, False), (70001, 3000, 1100000, True)])
+def test_house_over_sparse_ids(dev, n, d, m, tiles):
+    g = hub_and_sparse(n, d, m, n)
+    dg = dev.upload(g)
+    plan, hub = sme.Plan(4), n // 3
+    got = {}
+    assert ("house_wedge" in slots_used(dev, lambda: got.update(r=dev.count(dg, plan)))) == tiles
+    dev.set_tuning(super_chunks=4, census_level_engine=1)
+    want = dev.count(dg, plan)
+    dev.set_tuning(super_chunks=4)
+    assert (got["r"].count, got["r"].levels) == (want.count, want.levels)
+    assert "house_wedge" in slots_used(dev, lambda: got.update(h=dev.count(dg, plan, hub - 2, hub + 1)))
+    want = oracle.light_count(g.row_ptrs, g.cols, 4, 3, v_begin=hub - 2, v_end=hub + 1)
+    assert (got["h"].count, got["h"].levels) == (want[0], want[1])
+    dg.release()
