@@ -244,13 +244,14 @@ int sme_plan_vertices(const sme_plan* p);
  *                  self-loops, every degree below 2^19); a 4-cycle count (Q1, ordering on)
  *                  over any start range, with level outputs and per bucket,
  *                  comes from the wedges of each start vertex (symmetric
- *                  graphs without self-loops, every |N+(v)| at most 65,535;
+ *                  graphs without self-loops, every |N+(v)| at most 65,535, not
+ *                  where wedges are few for the ids they are spread over;
  *                  clique_level_engine 1 turns this off too); a house count
  *                  over a start range, with level outputs or per bucket,
  *                  likewise from wedges and per-edge triangle counts (every
  *                  degree at most 65,535, the counts within a quarter of the
- *                  memory, not for a range with under 1/128 of the work, and
- *                  not where wedges are few for the ids they are spread over);
+ *                  memory, likewise, and not for a range with under 1/128 of
+ *                  the work);
  *                  1: through the level engine.  Counts and level outputs are identical.
  * Settings apply to every later call on the context; results never depend
  * on them. */

@@ -2050,7 +2050,19 @@ WedgeArgs WedgeBase(const DevGraph* g, uint32_t vb, uint32_t ve, const BucketRef
   return w;
 }
 
-void LocalSquare(Context* ctx, const DevGraph* g, const EnginePlan* plan, uint32_t vb, uint32_t ve,
+// The light kernel finds the start vertices that need tiles, so only then is
+// their number known.  A tile costs 35 ns over the whole chip, its share of the
+// walk included.  The level engine's time per (edge, further neighbour) pair
+// grows with the lists (0.007 ns times their mean), to about 0.28 ns.  Where the
+// tiles would take longer their kernel does nothing and the level engine counts.
+//                     list_mean   items   pairs   engine   light and tiles
+//   G(2^20, 1.26e7)      25       2.6e6   3.2e8    51 ms    92 ms
+//   G(2^22, 5.0e7)       25       4.2e7   1.3e9   229     1388
+//   G(2^20, 2.5e7)       49       9.4e6   1.2e9   341      320
+//   G(300,000, 3.6e6)    25       2.4e5   9.0e7    14        8.9
+//   R-MAT 21, factor 1  276       1.1e6   8.7e8   123       56
+// false: that is what is left to do (nothing is counted).
+bool LocalSquare(Context* ctx, const DevGraph* g, const EnginePlan* plan, uint32_t vb, uint32_t ve,
                  const BucketRef& bk, uint64_t* count, uint64_t* levels, RunStats* st) {
   hipStream_t s = ctx->stream();
   *st = RunStats{};
@@ -2061,15 +2073,25 @@ void LocalSquare(Context* ctx, const DevGraph* g, const EnginePlan* plan, uint32
   WedgeArgs w = WedgeBase(g, vb, ve, bk, acc.get());
   w.heavy = heavy.get();
   w.nheavy = acc.get() + kWedgeAcc;
+  const uint64_t tiles = WedgeTiles(w.n);
+  // (4,096 tiles take no longer than the level engine's launches)
+  if (tiles > 1) {
+    const double pairs = static_cast<double>(g->house_work[ve] - g->house_work[vb]);
+    w.max_items = std::max<uint64_t>(4096, static_cast<uint64_t>(pairs * std::min(0.28, 0.007 * g->list_mean) / 35));
+  }
   {
     Timed t(ctx, s, kSlotHouseWedge, 24.0 * (ve - vb), ve - vb);
     LaunchSquareLight(w, s);
     LaunchWedgeTiles(w, kWedgeSquare, s);
   }
   uint64_t* pin = ctx->pinned();
-  SME_HIP(hipMemcpyAsync(pin, acc.get(), kWedgeAcc * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
+  SME_HIP(hipMemcpyAsync(pin, acc.get(), (kWedgeAcc + 1) * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
   SME_HIP(hipStreamSynchronize(s));
   st->d2h_syncs++;
+  if (w.max_items && pin[kWedgeAcc] * tiles > w.max_items) {
+    if (bk.bounds) LaunchFill64(reinterpret_cast<uint64_t*>(bk.counts), bk.nbuckets, 0, s);
+    return false;
+  }
   *count = pin[0];
   if (levels)
     for (int L = 0; L < plan->nops; ++L) {
@@ -2077,6 +2099,7 @@ void LocalSquare(Context* ctx, const DevGraph* g, const EnginePlan* plan, uint32
       const bool set = o.kind == kCompute || o.kind == kMaterialize;
       levels[L] = set && o.u == 0 ? ve - vb : set && o.u == 1 ? pin[1] : set && o.u == 2 ? pin[2] : pin[0];
     }
+  return true;
 }
 
 // The house plan whose level outputs LocalHouseRange knows (M1 C2 C3 M2 C0 M3
@@ -2279,8 +2302,8 @@ Status RunPlan(Context* ctx, const DevGraph* g, const EnginePlan* plan, uint32_t
     } else if (full && LocalDiamondApplies(ctx, dg, plan) &&
                InMemory([&] { LocalDiamond(ctx, dg, plan, count, level_counts, &st); })) {
       on_ranked = dg != g;
-    } else if (SquareApplies(ctx, rg, plan, v_end - v_begin)) {
-      LocalSquare(ctx, rg, plan, v_begin, v_end, BucketRef{}, count, level_counts, &st);
+    } else if (SquareApplies(ctx, rg, plan, v_end - v_begin) &&
+               LocalSquare(ctx, rg, plan, v_begin, v_end, BucketRef{}, count, level_counts, &st)) {
     } else if (HouseRangeApplies(ctx, rg, plan, v_begin, v_end, level_counts != nullptr) && InMemory([&] {
                  LocalHouseRange(ctx, rg, plan, v_begin, v_end, BucketRef{}, count, level_counts, &st);
                })) {
@@ -2380,8 +2403,8 @@ Status RunPlanBuckets(Context* ctx, const DevGraph* g, const EnginePlan* plan, c
     bk.counts = dcounts.get();
     bk.table = table.get();
     bk.base = bounds[0];
-    if (SquareApplies(ctx, g, plan, range)) {
-      LocalSquare(ctx, g, plan, bounds[0], bounds[nbuckets], bk, count, level_counts, &st);
+    if (SquareApplies(ctx, g, plan, range) &&
+        LocalSquare(ctx, g, plan, bounds[0], bounds[nbuckets], bk, count, level_counts, &st)) {
     } else if (HouseRangeApplies(ctx, g, plan, bounds[0], bounds[nbuckets], level_counts != nullptr) && InMemory([&] {
                  LocalHouseRange(ctx, g, plan, bounds[0], bounds[nbuckets], bk, count, level_counts, &st);
                })) {

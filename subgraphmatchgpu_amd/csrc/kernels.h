@@ -511,6 +511,7 @@ struct WedgeArgs {
   uint32_t* heavy;
   unsigned long long* nheavy;
   unsigned long long* next;     // work counter of LaunchWedgeTiles, zero
+  uint64_t max_items;           // square: with more items (start vertices times tiles) nothing is counted; 0: no limit
   uint32_t ntiles;              // id tiles a start vertex is walked in (set by the launcher)
   const uint32_t* cuts;         // LaunchWedgeCuts' table, or nullptr: lists are searched
   const uint32_t* t;            // house: triangles per CSR entry, both directions

@@ -182,6 +182,7 @@ __global__ __launch_bounds__(kThr) void WedgeTileKernel(WedgeArgs a) {
   WalkLds& s = walk_all[wid];
   const u64 napex = a.heavy ? *a.nheavy : a.v_end - a.v_begin;
   const u64 nitems = napex * a.ntiles;
+  if (kUse == kWedgeSquare && a.max_items && nitems > a.max_items) return;  // (the same for all workgroups)
   u64 total = 0, c1 = 0, c2 = 0, c3 = 0, c4 = 0, c5 = 0;
   while (true) {
     __syncthreads();  // the previous item's readers of item_s, sum_s and the counters are done

@@ -435,3 +435,24 @@ def test_house_over_sparse_ids(dev, n, d, m, tiles):
     want = oracle.light_count(g.row_ptrs, g.cols, 4, 3, v_begin=hub - 2, v_end=hub + 1)
     assert (got["h"].count, got["h"].levels) == (want[0], want[1])
     dg.release()
+
+
+@pytest.mark.gpu
+def test_square_over_sparse_ids(dev):
+    """Many start vertices just above the light kernel's limits, 13 tiles of ids: the level engine
+    takes over what the light kernel has begun; a few of them keep the tiles."""
+    g = sme.gen_er(800_000, 9_600_000, seed=4)
+    dg = dev.upload(g)
+    plan = sme.Plan(1)
+    for vb, ve, tiles in ((0, g.n, False), (0, 1000, False), (0, 200, True), (500_000, 500_100, True)):
+        got = {}
+        bounds = [vb, vb + 3, (vb + ve) // 2, ve]
+        used = slots_used(dev, lambda: got.update(r=dev.count(dg, plan, vb, ve)))
+        assert used == {"house_wedge"} if tiles else "house_wedge" in used and len(used) > 1
+        buckets = dev.count_buckets(dg, plan, bounds)
+        dev.set_tuning(super_chunks=4, census_level_engine=1)
+        want, each = dev.count(dg, plan, vb, ve), dev.count_buckets(dg, plan, bounds)
+        dev.set_tuning(super_chunks=4)
+        assert (got["r"].count, got["r"].levels) == (want.count, want.levels)
+        assert (buckets[0].tolist(), buckets[1].count, buckets[1].levels) == (each[0].tolist(), want.count, want.levels)
+    dg.release()
