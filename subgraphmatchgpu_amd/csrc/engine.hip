@@ -1910,20 +1910,51 @@ void LocalHouse(Context* ctx, const DevGraph* g, uint64_t* count, RunStats* st) 
   EdgeTriangles(ctx, g, t.get(), load.get(), acc.get(), st);
   HouseArgs h = HouseBase(g, t.get(), load.get(), acc.get());
   // 3a. light apexes in an LDS hash, heavier ones over tiles of ids
-  Buf<unsigned long long> lists(ctx, 3);
-  LaunchFill64(reinterpret_cast<uint64_t*>(lists.get()), 3, 0, s);
+  constexpr int kLists = 5;  // light and tiled apexes, the loads of either, the tile kernel's work counter
+  Buf<unsigned long long> lists(ctx, kLists);
+  LaunchFill64(reinterpret_cast<uint64_t*>(lists.get()), kLists, 0, s);
   std::vector<unsigned long long> hl;
   std::vector<uint64_t> hrp, hup;
+  uint64_t* pin = ctx->pinned();
+  const uint64_t per_slot = 12 * n;  // dense arrays (3b): u64 accumulator + u32 touched entry per w
+  auto slots_for = [&](uint64_t apexes) {
+    const uint64_t fit = static_cast<uint64_t>(0.5 * static_cast<double>(ctx->RunAvailable())) / per_slot;
+    return std::max<uint64_t>(1, std::min<uint64_t>({256, apexes, fit}));
+  };
+  bool dense = false;
   {
     Buf<uint32_t> light(ctx, n), tiled(ctx, n);
     h.light = light.get();
     h.nlight = lists.get();
     h.tiled = tiled.get();
     h.ntiled = lists.get() + 1;
+    h.loads = lists.get() + 2;
     LaunchHouseApexes(h, s);
+    // A tile of ids takes 17.5 ns over the whole chip whatever it holds, and an
+    // apex is given all of them: on large sparse graphs the dense arrays, whose
+    // groups take 58 us and whose wedges up to 0.24 ns each, are the cheaper.
+    //                    apexes   wedges  tiles   tiled   dense (whole count)
+    //   G(2^20, 2.5e7)   5.5e5    7.2e8     16    161 ms  265 ms
+    //   G(2^21, 2.5e7)   1.5e5    8.7e7     32    121      99
+    //   G(2^22, 5.0e7)   2.9e5    1.7e8     64    418     204
+    // Up to 19 tiles the arrays never are: an apex's tiles take 333 ns, its
+    // wedges (over 512) and its share of a group 349.
+    const uint64_t tiles = WedgeTiles(static_cast<uint32_t>(n));
+    uint64_t wedges[2] = {0, 0};
+    if (tiles > 19 || ctx->profiling) {
+      SME_HIP(hipMemcpyAsync(pin, lists.get(), 4 * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
+      SME_HIP(hipStreamSynchronize(s));
+      st->d2h_syncs++;
+      const double apexes = static_cast<double>(pin[1]);
+      wedges[0] = pin[2];
+      wedges[1] = pin[3];
+      dense = tiles > 19 && 17.5 * apexes * static_cast<double>(tiles) >
+                                0.24 * static_cast<double>(wedges[1]) +
+                                    58e3 * apexes / static_cast<double>(slots_for(pin[1]));
+    }
     {
-      // per wedge: the entry w and its t (the number is not known here)
-      Timed tm(ctx, s, kSlotHouseWedge, 0, 0);
+      // per wedge: the entry w and its t
+      Timed tm(ctx, s, kSlotHouseWedge, 8.0 * static_cast<double>(wedges[0]), wedges[0]);
       LaunchHouseWedgeHash(h, s);
     }
     WedgeArgs w{};
@@ -1934,19 +1965,20 @@ void LocalHouse(Context* ctx, const DevGraph* g, uint64_t* count, RunStats* st) 
     w.v_end = static_cast<uint32_t>(n);
     w.heavy = tiled.get();
     w.nheavy = lists.get() + 1;
-    w.next = lists.get() + 2;
+    w.next = lists.get() + 4;
     w.t = t.get();
     w.acc = acc.get();
     // where the lists are cut into tiles, when that takes little of the memory
-    const uint64_t ncuts = (WedgeTiles(w.n) + 1ull) * n;
-    Buf<uint32_t> cuts(ctx, WedgeTiles(w.n) > 1 && 4 * ncuts <= ctx->RunAvailable() / 4 ? ncuts : 0);
-    {
-      Timed tm(ctx, s, kSlotHouseWedge, 0, 0);
+    const uint64_t ncuts = (tiles + 1) * n;
+    Buf<uint32_t> cuts(ctx, !dense && tiles > 1 && 4 * ncuts <= ctx->RunAvailable() / 4 ? ncuts : 0);
+    if (!dense) {
+      // (walked twice)
+      Timed tm(ctx, s, kSlotHouseWedge, 12.0 * static_cast<double>(wedges[1]), wedges[1]);
       if (cuts.get()) LaunchWedgeCuts(w, cuts.get(), s);
       w.cuts = cuts.get();
       LaunchWedgeTiles(w, kWedgeApex, s);
     }
-    if (g->max_degree > kWedgeDegreeMax) {
+    if (dense || g->max_degree > kWedgeDegreeMax) {
       hl.resize(n);
       hrp.resize(n + 1);
       hup.resize(n);
@@ -1959,15 +1991,14 @@ void LocalHouse(Context* ctx, const DevGraph* g, uint64_t* count, RunStats* st) 
   }
   std::vector<uint32_t> heavy;
   for (uint64_t u = 0; u < hl.size(); ++u)
-    if (hl[u] > kHouseHashMax && hup[u] - hrp[u] > kWedgeDegreeMax) heavy.push_back(static_cast<uint32_t>(u));
+    if (hl[u] > kHouseHashMax && (dense || hup[u] - hrp[u] > kWedgeDegreeMax)) heavy.push_back(static_cast<uint32_t>(u));
   std::sort(heavy.begin(), heavy.end(), [&](uint32_t a, uint32_t b) {
     return hl[a] != hl[b] ? hl[a] > hl[b] : a < b;
   });
-  // 3b. apexes whose c may not fit 16 bits: groups of dense per-apex arrays over w
+  // 3b. apexes whose c may not fit 16 bits, or all but the light ones: groups of
+  // dense per-apex arrays over w
   if (!heavy.empty()) {
-    const uint64_t per_slot = 12 * n;  // u64 accumulator + u32 touched entry per w
-    const uint64_t fit = static_cast<uint64_t>(0.5 * static_cast<double>(ctx->RunAvailable())) / per_slot;
-    const uint64_t S = std::max<uint64_t>(1, std::min<uint64_t>({256, heavy.size(), fit}));
+    const uint64_t S = slots_for(heavy.size());
     Buf<unsigned long long> slots(ctx, S * n);
     Buf<uint32_t> touched(ctx, S * n);
     Buf<unsigned long long> ntouched(ctx, S);
@@ -2009,7 +2040,6 @@ void LocalHouse(Context* ctx, const DevGraph* g, uint64_t* count, RunStats* st) 
       st->batches++;
     }
   }
-  uint64_t* pin = ctx->pinned();
   SME_HIP(hipMemcpyAsync(pin, acc.get(), 2 * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
   SME_HIP(hipStreamSynchronize(s));
   st->d2h_syncs++;

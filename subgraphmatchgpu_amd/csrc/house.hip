@@ -138,6 +138,7 @@ __device__ __forceinline__ void Append(bool take, uint32_t u, uint32_t* list, un
 __global__ __launch_bounds__(kThreads) void HouseApexKernel(HouseArgs a) {
   const int lane = threadIdx.x & (kWave - 1);
   const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
+  u64 light = 0, tiled = 0;
   for (uint64_t b = blockIdx.x * static_cast<uint64_t>(blockDim.x) + (threadIdx.x - lane); b < a.n; b += stride) {
     const uint64_t u = b + lane;
     u64 load = 0, lower = 0;
@@ -145,9 +146,13 @@ __global__ __launch_bounds__(kThreads) void HouseApexKernel(HouseArgs a) {
       load = a.load[u];
       lower = a.up[u] - a.rp[u];
     }
-    Append(load > 0 && load <= kHouseHashMax, static_cast<uint32_t>(u), a.light, a.nlight, lane);
-    Append(load > kHouseHashMax && lower <= kWedgeDegreeMax, static_cast<uint32_t>(u), a.tiled, a.ntiled, lane);
+    const bool hash = load > 0 && load <= kHouseHashMax, tile = load > kHouseHashMax && lower <= kWedgeDegreeMax;
+    Append(hash, static_cast<uint32_t>(u), a.light, a.nlight, lane);
+    Append(tile, static_cast<uint32_t>(u), a.tiled, a.ntiled, lane);
+    light += hash ? load : 0;
+    tiled += tile ? load : 0;
   }
+  BlockAdd<kThreads>(Into{a.loads, light}, Into{a.loads + 1, tiled});
 }
 
 // One wave per apex u: every wedge u - v - w (v, w < u) goes into an LDS

@@ -421,11 +421,13 @@ struct HouseArgs {
   unsigned long long* acc;      // acc[0] += sum (c - 1) s; acc[1] += sum_e t(e) (t(e) - 1)
   // LaunchHouseApexes: light[0 .. *nlight) and tiled[0 .. *ntiled) receive the
   // apexes with a load, up to kHouseHashMax and above; those of the latter with
-  // more than kWedgeDegreeMax lower neighbours are left out
+  // more than kWedgeDegreeMax lower neighbours are left out.  loads[0] and
+  // loads[1] += the loads of either list
   uint32_t* light;
   unsigned long long* nlight;
   uint32_t* tiled;
   unsigned long long* ntiled;
+  unsigned long long* loads;
   // HouseWedgeDenseKernel / HouseWedgeReduceKernel: apexes of one group
   const uint32_t* apex;
   uint64_t napex;

@@ -456,3 +456,17 @@ def test_square_over_sparse_ids(dev):
         assert (got["r"].count, got["r"].levels) == (want.count, want.levels)
         assert (buckets[0].tolist(), buckets[1].count, buckets[1].levels) == (each[0].tolist(), want.count, want.levels)
     dg.release()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,m,groups", [(1_700_000, 20_400_000, True), (1_200_000, 14_400_000, False)])
+def test_house_apexes_over_sparse_ids(n, m, groups):
+    """26 tiles of ids and apexes just above the hash's limit: dense arrays, in groups; 19: the tiles."""
+    g = sme.gen_er(n, m, seed=6)
+    d = sme.Device(0, budget_bytes=16 << 30)
+    dg = d.upload(g)
+    r = d.count_only(dg, sme.Plan(4))
+    assert (r.batches > 1) == groups
+    d.set_tuning(super_chunks=4, census_level_engine=1)
+    assert r.count == d.count_only(dg, sme.Plan(4)).count
+    d.close()
