@@ -543,7 +543,7 @@ void LaunchAsymmetric(const uint64_t* rp, const uint32_t* cols, uint64_t n, uint
 // COMPUTE_PATH_COUNT and COMPUTE_COUNT of paths p over two or three adjacency
 // lists N(M[v]) (paths.hip): `own_v` is the list's vertex matched last,
 // shared_v the others, which runs of consecutive paths have in common.  Graphs
-// of at most kPathRunIds vertices.
+// of at most kPathRunIds vertices, without repeated entries.
 constexpr uint32_t kPathRunIds = 32768;
 constexpr uint32_t kOwnRatio = 16;
 struct PathRunArgs {
@@ -560,6 +560,7 @@ struct PathRunArgs {
   uint8_t gt_v[kQ];
   uint8_t nne;
   uint8_t ne_v[2];
+  uint32_t group;                 // paths a wave takes at a time (set by the launcher)
   uint64_t* out_len;              // per path (nullable)
   unsigned long long* acc;        // the count (nullable), buckets with it
   unsigned long long* acc_level;

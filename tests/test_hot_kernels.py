@@ -470,3 +470,46 @@ def test_house_apexes_over_sparse_ids(n, m, groups):
     d.set_tuning(super_chunks=4, census_level_engine=1)
     assert r.count == d.count_only(dg, sme.Plan(4)).count
     d.close()
+
+
+def hubs_over(n, hubs, share, m, seed):
+    """The last `hubs` vertices joined to a share of all, on top of m random edges: long lists that
+    many runs of one or two short ones share."""
+    rng = np.random.default_rng(seed)
+    a, b = [rng.integers(0, n, m)], [rng.integers(0, n, m)]
+    for h in range(hubs):
+        ends = rng.choice(n, size=int(share * n), replace=False)
+        a.append(np.full(ends.size, n - 1 - h))
+        b.append(ends)
+    a, b = np.concatenate(a), np.concatenate(b)
+    a, b = a[a != b], b[a != b]
+    key = np.unique(np.concatenate([a * n + b, b * n + a]))
+    return sme.Graph(np.searchsorted(key, np.arange(n + 1) * n).astype(np.uint64), (key % n).astype(np.uint32))
+
+
+@pytest.mark.parametrize("q", [6, 8])
+def test_emu_path_runs_under_long_lists(emu, q):
+    g = hubs_over(900, 2, 0.6, 700, 3)
+    want = oracle.light_count(g.row_ptrs, g.cols, q, 3)
+    assert emu(g, q) == (want[0], want[1])
+    bounds = [0, 9, 450, 899, 900]
+    want = [oracle.light_count(g.row_ptrs, g.cols, q, 3, v_begin=a, v_end=b)[0] for a, b in zip(bounds, bounds[1:])]
+    assert emu(g, q, bounds=bounds)[2] == want
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,hubs,share,m", [(8192, 1, 1.0, 8192), (32768, 2, 0.5, 8192), (32768, 1, 1.0, 65536)])
+def test_path_runs_under_long_lists(dev, n, hubs, share, m):
+    """Runs of few short lists are searched; reading the shared lists for each took 3 to 10 times
+    as long as the item schedule, which a setting asks for."""
+    g = hubs_over(n, hubs, share, m, n + hubs)
+    dg = dev.upload(g)
+    for q in (6, 8):
+        want = oracle.light_count(g.row_ptrs, g.cols, q, 3)
+        r = dev.count(dg, sme.Plan(q))
+        assert (r.count, r.levels) == (want[0], want[1])
+        bounds = [0, 9, n // 2, n]
+        got = dev.count_buckets(dg, sme.Plan(q), bounds)[0].tolist()
+        assert got == [oracle.light_count(g.row_ptrs, g.cols, q, 3, v_begin=a, v_end=b)[0]
+                       for a, b in zip(bounds, bounds[1:])]
+    dg.release()
