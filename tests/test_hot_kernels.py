@@ -513,3 +513,19 @@ def test_path_runs_under_long_lists(dev, n, hubs, share, m):
         assert got == [oracle.light_count(g.row_ptrs, g.cols, q, 3, v_begin=a, v_end=b)[0]
                        for a, b in zip(bounds, bounds[1:])]
     dg.release()
+
+
+# dense 4-clique classes of up to 128 rows, 256 (alone or below larger ones) and 512, of fewer and of
+# more vertices than fill them: (upper neighbourhoods, copies)
+@pytest.mark.gpu
+@pytest.mark.parametrize("shapes", [[(100, 3)], [(200, 3)], [(100, 5), (200, 4), (300, 1)], [(200, 130), (300, 2)],
+                                    [(300, 130), (500, 2)], [(500, 129), (600, 2)], [(260, 5)]])
+def test_dense_classes(dev, shapes):
+    g = union(*[fan(d + 1, d, 1, 25 * d, 1000 * d + k) for d, copies in shapes for k in range(copies)])
+    want = oracle.light_count(g.row_ptrs, g.cols, 3, 3)
+    assert want[0] and on_gpu(dev, g, 3) == (want[0], want[1])
+    bounds = [0, 1, g.n // 3, g.n]
+    dg = dev.upload(g)
+    got = dev.count_buckets(dg, sme.Plan(3), bounds)[0].tolist()
+    dg.release()
+    assert got == [oracle.light_count(g.row_ptrs, g.cols, 3, 3, v_begin=a, v_end=b)[0] for a, b in zip(bounds, bounds[1:])]
