@@ -239,6 +239,11 @@ Status RunPlan(Context* ctx, const DevGraph* g, const EnginePlan* plan, uint32_t
                uint32_t v_end, uint64_t* count, uint64_t* level_counts, RunStats* stats,
                std::string* err, bool ranked_ids = false);
 
+// Bytes without which a count over the range, or its buckets, goes through the
+// level engine although its plan and graph have a faster way; 0: no such way, or
+// one without such a limit.
+uint64_t RunBytes(const Context* ctx, const DevGraph* g, const EnginePlan* plan, uint32_t v_begin, uint32_t v_end);
+
 // Same walk over [bounds[0], bounds[nbuckets]); additionally counts[k]
 // receives the embeddings whose first matched vertex lies in
 // [bounds[k], bounds[k+1]).  bounds must be non-decreasing.

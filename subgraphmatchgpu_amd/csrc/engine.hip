@@ -2062,9 +2062,16 @@ bool WedgeApplies(const Context* ctx, const DevGraph* g, const EnginePlan* plan)
          plan->enable_ordering && g->symmetric && !g->self_loops;
 }
 
+// Bytes of which a 4-cycle count takes at most a quarter (a run with less stays
+// with the level engine's batches); 0: not that way, whatever the memory.
+uint64_t SquareBytes(const Context* ctx, const DevGraph* g, const EnginePlan* plan, uint64_t range) {
+  if (plan->query_type != 1 || !WedgeApplies(ctx, g, plan) || g->max_up_degree > kWedgeDegreeMax) return 0;
+  return 4 * (4 * range + (1 << 12));
+}
+
 bool SquareApplies(const Context* ctx, const DevGraph* g, const EnginePlan* plan, uint64_t range) {
-  return plan->query_type == 1 && WedgeApplies(ctx, g, plan) && g->max_up_degree <= kWedgeDegreeMax &&
-         4 * range + (1 << 12) <= ctx->RunAvailable() / 4;
+  const uint64_t need = SquareBytes(ctx, g, plan, range);
+  return need && need <= ctx->RunAvailable();
 }
 
 constexpr int kWedgeAcc = 6;
@@ -2181,12 +2188,20 @@ bool HouseTilesPay(const DevGraph* g, uint32_t vb, uint32_t ve) {
          0.8 * tile_ns * static_cast<double>(ve - vb) * tiles;
 }
 
+// Bytes of which a house count over a range takes at most a quarter; 0: not that
+// way, whatever the memory.
+uint64_t HouseRangeBytes(const Context* ctx, const DevGraph* g, const EnginePlan* plan, uint32_t vb, uint32_t ve,
+                         bool levels) {
+  const bool so = plan->query_type == 4 && WedgeApplies(ctx, g, plan) && (!levels || HouseLevels(plan)) &&
+                  g->max_degree <= kWedgeDegreeMax && g->max_up_degree <= kLocalMax && ve > vb &&
+                  (g->house_work[ve] - g->house_work[vb]) * 128 >= g->house_work[g->n] && HouseTilesPay(g, vb, ve);
+  return so ? 4 * CensusBytes(g) : 0;
+}
+
 bool HouseRangeApplies(const Context* ctx, const DevGraph* g, const EnginePlan* plan, uint32_t vb, uint32_t ve,
                        bool levels) {
-  return plan->query_type == 4 && WedgeApplies(ctx, g, plan) && (!levels || HouseLevels(plan)) &&
-         g->max_degree <= kWedgeDegreeMax && g->max_up_degree <= kLocalMax &&
-         CensusBytes(g) <= ctx->RunAvailable() / 4 && ve > vb &&
-         (g->house_work[ve] - g->house_work[vb]) * 128 >= g->house_work[g->n] && HouseTilesPay(g, vb, ve);
+  const uint64_t need = HouseRangeBytes(ctx, g, plan, vb, ve, levels);
+  return need && need <= ctx->RunAvailable();
 }
 
 void LocalHouseRange(Context* ctx, const DevGraph* g, const EnginePlan* plan, uint32_t vb, uint32_t ve,
@@ -2295,6 +2310,12 @@ bool InMemory(F&& body) {
 }
 
 }  // namespace
+
+uint64_t RunBytes(const Context* ctx, const DevGraph* g, const EnginePlan* plan, uint32_t v_begin, uint32_t v_end) {
+  const uint64_t range = v_end > v_begin ? v_end - v_begin : 0;
+  const uint64_t need = std::max(SquareBytes(ctx, g, plan, range), HouseRangeBytes(ctx, g, plan, v_begin, v_end, false));
+  return need ? need + 4 * range + (1 << 16) : 0;  // (buckets: a table of the range, their bounds and counts)
+}
 
 Status RunPlan(Context* ctx, const DevGraph* g, const EnginePlan* plan, uint32_t v_begin,
                uint32_t v_end, uint64_t* count, uint64_t* level_counts, RunStats* stats,

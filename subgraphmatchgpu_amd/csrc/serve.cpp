@@ -168,7 +168,7 @@ void Server::Dispatch() {
     std::vector<std::pair<uint32_t, uint32_t>> rg;
     for (uint64_t id : job->ids) rg.push_back({reqs_[id].vb, reqs_[id].ve});
     std::sort(rg.begin(), rg.end());
-    uint64_t work = 0;
+    uint64_t work = 0, needed = 0;
     uint32_t cur_b = rg[0].first, cur_e = rg[0].second;
     for (size_t i = 1; i <= rg.size(); ++i) {
       if (i < rg.size() && rg[i].first <= cur_e) {
@@ -176,6 +176,7 @@ void Server::Dispatch() {
         continue;
       }
       work += WorkUnits(cur_b, cur_e);
+      needed = std::max(needed, RunBytes(ctx_[slot].get(), graph_.get(), &plans_[job->q], cur_b, cur_e));
       if (i < rg.size()) {
         cur_b = rg[i].first;
         cur_e = rg[i].second;
@@ -191,6 +192,8 @@ void Server::Dispatch() {
       reserve = est >= static_cast<double>(cfg_.mem_cap) ? cfg_.mem_cap : static_cast<uint64_t>(est);
     }
     reserve = std::max(reserve, cfg_.min_reserve);
+    // what a pass held at its peak may be less than it has to be allowed
+    if (needed <= cfg_.mem_cap) reserve = std::max(reserve, needed);
     if (cfg_.slots == 1) reserve = cfg_.mem_cap;  // one pass at a time: the whole budget
     job->reserve = reserve;
     cv_dispatch_.wait(lk, [&] { return stop_ || reserved_ + reserve <= cfg_.mem_cap; });

@@ -529,3 +529,22 @@ def test_dense_classes(dev, shapes):
     got = dev.count_buckets(dg, sme.Plan(3), bounds)[0].tolist()
     dg.release()
     assert got == [oracle.light_count(g.row_ptrs, g.cols, 3, 3, v_begin=a, v_end=b)[0] for a, b in zip(bounds, bounds[1:])]
+
+
+@pytest.mark.gpu
+def test_served_house_keeps_its_memory():
+    """What a house pass held at its peak is a quarter of what it has to be allowed: the passes
+    after the first take as long as it does (the level engine needs over a second)."""
+    g = sme.gen_rmat(16, 8, seed=5)
+    srv = sme.Server(g, mem_cap_bytes=160 << 20, slots=2, min_reserve_bytes=1 << 20)
+    want = None
+    for k in range(4):
+        count, ms = srv.wait(srv.submit(4, 1, g.n))
+        print(f"pass {k}: {ms:.1f} ms", flush=True)
+        assert want in (None, count)
+        want = count
+        assert ms < 300
+    ids = [srv.submit(4, a, b) for a, b in ((1, 30000), (20000, 65536), (1, g.n))]
+    got = [srv.wait(i) for i in ids]
+    assert got[2][0] == want and max(ms for _, ms in got) < 300
+    srv.close()
