@@ -207,7 +207,8 @@ class DevGraph {
   // house_work[v]: sum of |N+(u)| |N(u)| over u < v, the (edge, further
   // neighbour) pairs that house counts from those start vertices look at
   std::vector<uint64_t> house_work;
-  double list_mean = 0;  // mean |N(u)| over the entries u
+  double wedges = 0;    // sum of |N(v)|^2: entries of the lists that all entries lead to
+  double pair_min = 0;  // mean of the shorter of two lists, of different vertices, that entries lead to
   // Built at upload for the clique bitmap path over all start vertices:
   // the vertices with kLocalSmall < |N+(v)| <= kLocalMax in decreasing
   // |N+(v)| (ties by id) with prefix sums of their rows, row words and

@@ -196,6 +196,7 @@ Status DevGraph::Upload(Context* ctx, const uint64_t* row_ptrs, const uint32_t* 
   nnz = ne;
   self_loops = loops;
   house_work.assign(nv + 1, 0);
+  std::vector<uint64_t> with_degree;
   for (uint64_t v = 0; v < nv; ++v) {
     const uint32_t* b = c + row_ptrs[v];
     const uint32_t* e = c + row_ptrs[v + 1];
@@ -203,7 +204,8 @@ Status DevGraph::Upload(Context* ctx, const uint64_t* row_ptrs, const uint32_t* 
     max_degree = std::max<uint64_t>(max_degree, e - b);
     max_up_degree = std::max<uint64_t>(max_up_degree, dp);
     house_work[v + 1] = house_work[v] + dp * static_cast<uint64_t>(e - b);
-    list_mean += static_cast<double>(e - b) * static_cast<double>(e - b);
+    if (static_cast<uint64_t>(e - b) >= with_degree.size()) with_degree.resize(e - b + 1, 0);
+    with_degree[e - b]++;
     if (dp > kLocalMax) {
       upper.huge.push_back(static_cast<uint32_t>(v));
     } else if (dp > kLocalSmall) {
@@ -213,7 +215,16 @@ Status DevGraph::Upload(Context* ctx, const uint64_t* row_ptrs, const uint32_t* 
       upper.d.push_back(static_cast<uint32_t>(dp));
     }
   }
-  if (nnz) list_mean /= static_cast<double>(nnz);
+  {
+    double above = 0;  // entries of longer lists
+    for (uint64_t k = with_degree.size(); k-- > 0;) {
+      const double d = static_cast<double>(k), c = static_cast<double>(with_degree[k]);
+      wedges += c * d * d;
+      pair_min += 2 * d * d * (c * above + d * c * (c - 1) / 2);
+      above += c * d;
+    }
+    if (ne) pair_min /= static_cast<double>(ne) * static_cast<double>(ne);
+  }
   {
     const uint64_t nb = upper.verts.size();
     std::vector<uint32_t> order(nb);
@@ -2093,16 +2104,19 @@ WedgeArgs WedgeBase(const DevGraph* g, uint32_t vb, uint32_t ve, const BucketRef
 }
 
 // The light kernel finds the start vertices that need tiles, so only then is
-// their number known.  A tile costs 35 ns over the whole chip, its share of the
-// walk included.  The level engine's time per (edge, further neighbour) pair
-// grows with the lists (0.007 ns times their mean), to about 0.28 ns.  Where the
-// tiles would take longer their kernel does nothing and the level engine counts.
-//                     list_mean   items   pairs   engine   light and tiles
-//   G(2^20, 1.26e7)      25       2.6e6   3.2e8    51 ms    92 ms
-//   G(2^22, 5.0e7)       25       4.2e7   1.3e9   229     1388
-//   G(2^20, 2.5e7)       49       9.4e6   1.2e9   341      320
-//   G(300,000, 3.6e6)    25       2.4e5   9.0e7    14        8.9
-//   R-MAT 21, factor 1  276       1.1e6   8.7e8   123       56
+// their number known, and the list entries (acc[3]) that all start vertices look
+// at.  A tile costs 35 ns over the whole chip, its share of the walk included,
+// and the level engine 0.02 ns per entry and 0.008 per entry of the shorter of
+// two lists, within a factor of two.  Where the tiles would take longer their
+// kernel does nothing and the level engine counts.
+//                       tiles   entries  shorter  engine   light and tiles
+//   G(2^20, 1.26e7)     2.6e6   3.2e8     22       51 ms    92 ms
+//   G(2^22, 5.0e7)      4.2e7   1.3e9     22      229     1388
+//   G(2^20, 2.5e7)      9.4e6   9e8       45      341      320
+//   G(300,000, 3.6e6)   2.4e5   9.0e7     22       14        8.9
+//   R-MAT 21, factor 1  1.1e6   1.2e8             123       56
+//   last of 10^6 vertices joined to 60,000
+//                       9.6e5   1.8e9      3       59       31
 // false: that is what is left to do (nothing is counted).
 bool LocalSquare(Context* ctx, const DevGraph* g, const EnginePlan* plan, uint32_t vb, uint32_t ve,
                  const BucketRef& bk, uint64_t* count, uint64_t* levels, RunStats* st) {
@@ -2116,11 +2130,7 @@ bool LocalSquare(Context* ctx, const DevGraph* g, const EnginePlan* plan, uint32
   w.heavy = heavy.get();
   w.nheavy = acc.get() + kWedgeAcc;
   const uint64_t tiles = WedgeTiles(w.n);
-  // (4,096 tiles take no longer than the level engine's launches)
-  if (tiles > 1) {
-    const double pairs = static_cast<double>(g->house_work[ve] - g->house_work[vb]);
-    w.max_items = std::max<uint64_t>(4096, static_cast<uint64_t>(pairs * std::min(0.28, 0.007 * g->list_mean) / 35));
-  }
+  if (tiles > 1) w.items_ratio = static_cast<uint64_t>(65536 * (0.02 + 0.008 * g->pair_min) / 35) + 1;
   {
     Timed t(ctx, s, kSlotHouseWedge, 24.0 * (ve - vb), ve - vb);
     LaunchSquareLight(w, s);
@@ -2130,7 +2140,7 @@ bool LocalSquare(Context* ctx, const DevGraph* g, const EnginePlan* plan, uint32
   SME_HIP(hipMemcpyAsync(pin, acc.get(), (kWedgeAcc + 1) * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
   SME_HIP(hipStreamSynchronize(s));
   st->d2h_syncs++;
-  if (w.max_items && pin[kWedgeAcc] * tiles > w.max_items) {
+  if (w.items_ratio && pin[kWedgeAcc] * tiles > WedgeItemsMax(pin[3], w.items_ratio)) {
     if (bk.bounds) LaunchFill64(reinterpret_cast<uint64_t*>(bk.counts), bk.nbuckets, 0, s);
     return false;
   }
@@ -2167,25 +2177,30 @@ bool HouseLevels(const EnginePlan* plan) {
 //
 // A tile costs a workgroup its counters and a chain of waits whatever it holds:
 // 24 ns a tile over the whole chip (15 n / 65,536 where one tile holds all ids:
-// no list is cut then).  The engine's time goes with the (edge, further
-// neighbour) pairs: from 0.26 ns each (G(n, m) of degree 8) to 1.1 (R-MAT scale
-// 17, mean list 326), within a factor of two of 0.085 list_mean^0.45.
-//                           tiles   engine     walk      pairs ns / tiles ns
-//   G(300,000, 1.2e6)         5      2.9 ms    35.7 ms   0.07
-//   G(1,048,576, 4.2e6)      16      9.8      401        0.02
-//   G(1,048,576, 1.26e7)     16    169        565        0.28
-//   G(1,048,576, 2.5e7)      16   1073        676        1.5
-//   G(100,000, 8e5)           2      5.4        5.4      0.87
-//   R-MAT 19, factor 1        8     81         56        1.1
-//   R-MAT 20, factor 1       16    246        225        0.80
-//   R-MAT 21, factor 1       32    about 800  901        0.57
+// no list is cut then; 3 with the small workgroups), and an entry walked up to
+// 0.016 ns (0.004), both walks together.  The level engine intersects two lists
+// for every (edge, further neighbour) pair: 0.1 ns and 0.02 per entry of the
+// shorter one, within a factor of two.
+//                                      pairs    shorter  engine     walk
+//   G(1,048,576, 4.2e6)                3.8e7      8       9.8 ms   401 ms
+//   G(1,048,576, 1.26e7)               3.2e8     22     169        565
+//   G(1,048,576, 2.5e7)                1.2e9     45    1073        676
+//   G(100,000, 8e5)                    1.4e7     15       5.4        5.4
+//   R-MAT 19, factor 1                 1.3e8             81         56
+//   R-MAT 20, factor 1                 3.4e8            246        225
+//   last vertex joined to all 60,000   2e5        2       0.5       57
+//   last 3 to half of 60,000           5e5     1800      22         26
+//   last 3 to four fifths of 16,000    4.5e5    640       7.0        1.6
+//   first joined to all 16,000         2.6e8      3      31          0.6
 bool HouseTilesPay(const DevGraph* g, uint32_t vb, uint32_t ve) {
   const uint32_t tiles = WedgeTiles(static_cast<uint32_t>(g->n));
-  if (g->n <= kWedgeSmallIds) return true;
-  const double tile_ns = tiles > 1 ? 24.0 : 15.0 / 65536 * static_cast<double>(g->n);
-  const double pair_ns = 0.085 * std::pow(std::max(1.0, g->list_mean), 0.45);
-  return pair_ns * static_cast<double>(g->house_work[ve] - g->house_work[vb]) >=
-         0.8 * tile_ns * static_cast<double>(ve - vb) * tiles;
+  const bool small = g->n <= kWedgeSmallIds;
+  const double n = static_cast<double>(g->n), starts = static_cast<double>(ve - vb);
+  const double tile_ns = small ? 3.0 : tiles > 1 ? 24.0 : 15.0 / 65536 * n;
+  const double walk_ns = small ? 0.004 : 0.016;
+  // (0.1 ms: the engine's launches)
+  const double engine = 1e5 + (0.1 + 0.02 * g->pair_min) * static_cast<double>(g->house_work[ve] - g->house_work[vb]);
+  return engine >= 0.8 * tile_ns * starts * tiles + walk_ns * g->wedges * starts / n;
 }
 
 // Bytes of which a house count over a range takes at most a quarter; 0: not that

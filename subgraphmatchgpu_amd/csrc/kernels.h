@@ -513,18 +513,26 @@ struct WedgeArgs {
   uint32_t* heavy;
   unsigned long long* nheavy;
   unsigned long long* next;     // work counter of LaunchWedgeTiles, zero
-  uint64_t max_items;           // square: with more items (start vertices times tiles) nothing is counted; 0: no limit
+  // square: with more items (start vertices times tiles) than WedgeItemsMax(acc[3],
+  // items_ratio) nothing is counted; 0: no limit
+  uint64_t items_ratio;
   uint32_t ntiles;              // id tiles a start vertex is walked in (set by the launcher)
   const uint32_t* cuts;         // LaunchWedgeCuts' table, or nullptr: lists are searched
   const uint32_t* t;            // house: triangles per CSR entry, both directions
-  // acc[0] += count (apex: that sum); acc[1] += sum of |N+(a)|; square: acc[2] += wedges a - b - w;
+  // acc[0] += count (apex: that sum); acc[1] += sum of |N+(a)|; square: acc[2] += wedges a - b - w,
+  // acc[3] += entries of the lists looked at (64 each where |N+(a)| > 64);
   // house: acc[2] += sum of d(a), acc[3] += sum_{b > a} t(a, b),
   // acc[4] += sum of |N+(a)| (d(a) - 1), acc[5] += sum_{b > a} t(a, b) (d(a) - 2)
   unsigned long long* acc;
   BucketRef bk;
 };
-// 4-cycles of the start vertices with few wedges (one wave each) and acc[1],
-// acc[2] of all of them.
+// (4,096 tiles take no longer than the level engine's launches.)
+__host__ __device__ inline uint64_t WedgeItemsMax(uint64_t entries, uint64_t ratio) {
+  const uint64_t most = (entries >> 16) * ratio + ((entries & 65535) * ratio >> 16);
+  return most > 4096 ? most : 4096;
+}
+// 4-cycles of the start vertices with few wedges (one wave each), acc[1] and
+// acc[3] of all of them.
 void LaunchSquareLight(const WedgeArgs& a, hipStream_t stream);
 // Counts of `use` from heavy[] (or all start vertices): a workgroup per start
 // vertex and tile of ids keeps c in LDS.

@@ -66,7 +66,7 @@ __global__ __launch_bounds__(kThreads, 6) void SquareLightKernel(WedgeArgs a) {
   const uint64_t wave = (blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x) / kWave;
   const uint64_t nwaves = static_cast<uint64_t>(gridDim.x) * blockDim.x / kWave;
   const uint64_t nv = a.v_end - a.v_begin;
-  u64 total = 0, nup = 0, nwedge = 0;
+  u64 total = 0, nup = 0, nwedge = 0, looked = 0;
   BucketAcc bacc{kNoBucket, 0};
   for (uint64_t g = wave * a.group; g < nv; g += nwaves * a.group) {
     const uint64_t ge = g + a.group < nv ? g + a.group : nv;
@@ -77,6 +77,7 @@ __global__ __launch_bounds__(kThreads, 6) void SquareLightKernel(WedgeArgs a) {
       if (lane == 0) nup += d;
       if (d == 0) continue;
       bool heavy = d > kWave;
+      if (heavy && lane == 0) looked += kWave * d;
       uint64_t lb = 0;
       uint32_t len = 0, last = 0;
       uint32_t items = 0, most = 0;
@@ -87,6 +88,7 @@ __global__ __launch_bounds__(kThreads, 6) void SquareLightKernel(WedgeArgs a) {
           const uint64_t le = a.rp[v1 + 1];
           // v0 lies in N(v1): short lists are walked whole and filtered
           if (le - lb >= kCutList) lb = Lower(a.cols, lb, le, v0);
+          looked += le - lb;
           heavy = le - lb > kLightItems;
           len = heavy ? kLightItems : static_cast<uint32_t>(le - lb);
           last = a.cols[le - 1];
@@ -151,7 +153,7 @@ __global__ __launch_bounds__(kThreads, 6) void SquareLightKernel(WedgeArgs a) {
     }
   }
   if (a.bk.bounds) BucketFlush(a.bk, &bacc);
-  BlockAdd<kThreads>(Into{a.acc, total}, Into{a.acc + 1, nup}, Into{a.acc + 2, nwedge});
+  BlockAdd<kThreads>(Into{a.acc, total}, Into{a.acc + 1, nup}, Into{a.acc + 2, nwedge}, Into{a.acc + 3, looked});
 }
 
 // ---------------------------------------------------------------------------
@@ -182,7 +184,8 @@ __global__ __launch_bounds__(kThr) void WedgeTileKernel(WedgeArgs a) {
   WalkLds& s = walk_all[wid];
   const u64 napex = a.heavy ? *a.nheavy : a.v_end - a.v_begin;
   const u64 nitems = napex * a.ntiles;
-  if (kUse == kWedgeSquare && a.max_items && nitems > a.max_items) return;  // (the same for all workgroups)
+  // (the same for all workgroups)
+  if (kUse == kWedgeSquare && a.items_ratio && nitems > WedgeItemsMax(a.acc[3], a.items_ratio)) return;
   u64 total = 0, c1 = 0, c2 = 0, c3 = 0, c4 = 0, c5 = 0;
   while (true) {
     __syncthreads();  // the previous item's readers of item_s, sum_s and the counters are done

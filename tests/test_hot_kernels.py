@@ -437,6 +437,27 @@ def test_house_over_sparse_ids(dev, n, d, m, tiles):
     dg.release()
 
 
+# lists walked for few (edge, further neighbour) pairs: hubs above all their neighbours (level
+# engine), below them (tiles)
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,hubs,share,m,low,tiles", [(9000, 1, 1.0, 9000, False, False), (60000, 1, 1.0, 60000, False, False),
+                                                      (9000, 1, 1.0, 9000, True, True), (70000, 2, 0.4, 70000, False, False)])
+def test_house_under_long_lists(dev, n, hubs, share, m, low, tiles):
+    g = hubs_over(n, hubs, share, m, n)
+    if low:  # ids in reverse
+        src = np.repeat(np.arange(n), np.diff(g.row_ptrs.astype(np.int64)))
+        key = np.sort((n - 1 - src) * n + (n - 1 - g.cols.astype(np.int64)))
+        g = sme.Graph(np.searchsorted(key, np.arange(n + 1) * n).astype(np.uint64), (key % n).astype(np.uint32))
+    dg = dev.upload(g)
+    got = {}
+    assert ("house_wedge" in slots_used(dev, lambda: got.update(r=dev.count(dg, sme.Plan(4))))) == tiles
+    dev.set_tuning(super_chunks=4, census_level_engine=1)
+    want = dev.count(dg, sme.Plan(4))
+    dev.set_tuning(super_chunks=4)
+    assert (got["r"].count, got["r"].levels) == (want.count, want.levels)
+    dg.release()
+
+
 @pytest.mark.gpu
 def test_square_over_sparse_ids(dev):
     """Many start vertices just above the light kernel's limits, 13 tiles of ids: the level engine
