@@ -569,3 +569,80 @@ def test_served_house_keeps_its_memory():
     got = [srv.wait(i) for i in ids]
     assert got[2][0] == want and max(ms for _, ms in got) < 300
     srv.close()
+
+
+def broad_hubs(low, hubs, m, first, seed):
+    """Hubs joined to every one of `low` vertices, on top of G(low, m) among those; the hubs hold the
+    first ids or the last.  With its houses and 4-cycles, in closed form."""
+    s = sme.gen_er(low, m, seed=seed)
+    deg = np.diff(s.row_ptrs.astype(np.int64))
+    src = np.repeat(np.arange(low), deg)
+    cols = s.cols.astype(np.int64)
+    lists = [set(cols[int(s.row_ptrs[v]):int(s.row_ptrs[v + 1])].tolist()) for v in range(low)]
+    # 4-cycles: tr A^4 = sum of squared common-neighbour counts = 8 C4 + 2 sum d^2 - sum d
+    common = {}
+    for v in range(low):
+        for a in lists[v]:
+            for b in lists[v]:
+                common[a, b] = common.get((a, b), 0) + 1
+    sums = sum(common.values()), sum(x * x for x in common.values())
+    trace = hubs * hubs * low * low + 2 * hubs * sums[0] + sums[1]            # two low vertices
+    trace += 2 * hubs * int((deg ** 2).sum()) + hubs * hubs * low * low      # a hub and a low one, two hubs
+    d = np.concatenate([deg + hubs, np.full(hubs, low)])
+    squares, rest = divmod(trace - 2 * int((d ** 2).sum()) + int(d.sum()), 8)
+    assert rest == 0
+    # houses: sum over edges of t p - 2 t (t - 1), t triangles and p = A^3 - d(u) - d(v) + 1 4-cycles on it
+    houses = 0
+    for u, v in zip(src.tolist(), cols.tolist()):
+        if u < v:
+            t = len(lists[u] & lists[v]) + hubs
+            # neighbours x of u, each with its common neighbours with v
+            walks = sum(len(lists[x] & lists[v]) + hubs for x in lists[u]) + hubs * int(deg[v])
+            houses += t * (walks - int(deg[u] + deg[v]) - 2 * hubs + 1) - 2 * t * (t - 1)
+    for v in range(low):  # the edge (hub, v): t = deg(v); x over the low vertices or the neighbours of v
+        t = int(deg[v])
+        walks = sum(len(lists[x]) for x in lists[v]) + hubs * low  # A^3(v, h) = sum over x in N(v) of common(x, h)
+        houses += hubs * (t * (walks - (t + hubs) - low + 1) - 2 * t * (t - 1))
+    ids = np.arange(low) + (hubs if first else 0)
+    hub_ids = np.arange(hubs) + (0 if first else low)
+    n = low + hubs
+    a = np.concatenate([ids[src], np.repeat(hub_ids, low), np.tile(ids, hubs)])
+    b = np.concatenate([ids[cols], np.tile(ids, hubs), np.repeat(hub_ids, low)])
+    key = np.sort(a * n + b)
+    g = sme.Graph(np.searchsorted(key, np.arange(n + 1) * n).astype(np.uint64), (key % n).astype(np.uint32))
+    return g, houses, squares
+
+
+def test_broad_hubs_closed_forms():
+    for first in (True, False):
+        g, houses, squares = broad_hubs(40, 2, 70, first, 3)
+        assert oracle.light_count(g.row_ptrs, g.cols, 4, 3)[0] == houses
+        assert oracle.light_count(g.row_ptrs, g.cols, 1, 3)[0] == squares
+
+
+# apexes and start vertices with more neighbours than 16-bit counters hold: dense arrays, here in one
+# group and in two; the level engine for the 4-cycle
+@pytest.mark.gpu
+@pytest.mark.parametrize("budget,groups", [(1 << 30, 1), (6 << 20, 2)])
+@pytest.mark.parametrize("ranked", [False, True])
+def test_apexes_over_65535_neighbours(budget, groups, ranked):
+    g, houses, squares = broad_hubs(65600, 3, 20000, False, 5)
+    d = sme.Device(0, budget_bytes=budget)
+    d.set_rank_order(ranked)
+    dg = d.upload(g)
+    r = d.count_only(dg, sme.Plan(4))
+    assert r.count == houses and r.batches == 1 + groups
+    assert d.count_only(dg, sme.Plan(1)).count == squares
+    d.close()
+
+
+@pytest.mark.gpu
+def test_start_vertices_over_65535_neighbours(dev):
+    g, _, squares = broad_hubs(65600, 3, 20000, True, 6)
+    dg = dev.upload(g)
+    assert dev.count(dg, sme.Plan(1)).count == squares
+    vb, ve = 3, 40000  # (the hubs are not among the start vertices, but the graph has them)
+    want = oracle.light_count(g.row_ptrs, g.cols, 1, 3, v_begin=vb, v_end=ve)
+    r = dev.count(dg, sme.Plan(1), vb, ve)
+    assert (r.count, r.levels) == (want[0], want[1])
+    dg.release()
