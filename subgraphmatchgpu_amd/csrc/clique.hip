@@ -4,12 +4,19 @@
 // Start vertices with at most 64 upper neighbours are counted by
 // CliqueSmallKernel: a row is one u64, so every set below a row is one u64 and
 // every step of the count is an LDS load, an AND and a popcount.  Larger
-// neighbourhoods are counted in batches: CliqueRowsKernel writes each vertex's
-// rows to device memory (one wave per row, its lanes testing 64 candidates at
-// a time by binary search in the row vertex's own upper list), then
-// CliqueCountKernel takes one row i per wave, keeps the sets it derives from
-// row i in LDS and counts the last level by AND + popcount over whole words,
-// 64 clique members per word.
+// neighbourhoods are counted in batches.  Their rows are found by
+//   CliqueRowsTableKernel  d <= 4,096 and a span of fewer than 65,536 ids: N+(v)
+//                          as an LDS table over its span (with per-edge counts on
+//                          a ranked graph, CliqueMiddleKernel beside it);
+//   CliqueRowsHashKernel   d <= 4,096, wider spans: N+(v) as an LDS hash;
+//   CliqueRowsKernel       d > 4,096: binary search;
+// which count triangles themselves and write rows to device memory for the
+// larger cliques:
+//   CliqueDenseKernel      4-cliques, d <= 512: all rows of a vertex in LDS;
+//   CliqueCount4Kernel     4-cliques, the others: one wave per row;
+//   CliquePackKernel       5- and 6-cliques, one wave per row of up to 128
+//                          members, packed to those; CliqueLongKernel up to 512
+//                          (5-cliques); CliqueUnpackedKernel the others.
 //
 // The reference counts the same cliques by intersecting sorted adjacency
 // lists level by level (src/gpu/impl/light/op/LIGHTCompute.cuh,

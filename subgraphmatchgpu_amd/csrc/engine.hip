@@ -1683,6 +1683,7 @@ void LocalCliqueRange(Context* ctx, const DevGraph* g, const EnginePlan* plan, u
       if (tc) Fail(kErrOom, "bit rows of one start vertex exceed the memory the run may use");
       hh.insert(hh.end(), verts.begin(), verts.begin() + static_cast<int64_t>(first_fit));
     }
+    double after = 0;  // entries that follow another in the batches' lists
     for (uint64_t x0 = first_fit; x0 < nbig;) {
       uint64_t x1 = x0 + 1;
       while (x1 < nbig && fits(wf[x1 + 1] - wf[x0], rf[x1 + 1] - rf[x0])) ++x1;
@@ -1707,16 +1708,18 @@ void LocalCliqueRange(Context* ctx, const DevGraph* g, const EnginePlan* plan, u
                                                        [](uint32_t d) { return d > kRowsHashSmall; }) -
                                   hd_sorted.begin();
       {
-        // per row: the row vertex, its list bounds (20 bytes) and its words
-        // written; per later neighbour of the start vertex: the key and one
+        // per row: the row vertex, its list bounds (20 bytes) and, if they are
+        // kept, its words written; per later neighbour of the start vertex: the key and one
         // probe of the row vertex's list (4 + 4 bytes)
         double keys = 0;
         for (uint64_t x = x0; x < x1; ++x) {
           const double d = static_cast<double>(rf[x + 1] - rf[x]);
           keys += d * (d - 1) / 2;
         }
+        after += keys;
         Timed t(ctx, s, kSlotCliqueRows,
-                8.0 * keys + 20.0 * static_cast<double>(a.nitems) + 8.0 * static_cast<double>(words), a.nitems);
+                8.0 * keys + 20.0 * static_cast<double>(a.nitems) + (K > 3 ? 8.0 * static_cast<double>(words) : 0),
+                a.nitems);
         if (hash_from > x0) {
           CliqueArgs b = a;
           b.nverts = hash_from - x0;
@@ -1786,7 +1789,8 @@ void LocalCliqueRange(Context* ctx, const DevGraph* g, const EnginePlan* plan, u
       CliqueArgs b = a;
       b.v_begin = g->upper.first + 1;
       b.v_end = ve;
-      Timed t(ctx, s, kSlotCliqueRows, 0, 0);
+      // per list of a lower neighbour: its entries after the middle
+      Timed t(ctx, s, kSlotCliqueRows, 4.0 * after, b.v_end - b.v_begin);
       LaunchCliqueMiddles(b, s);
     }
   }
@@ -2132,7 +2136,7 @@ bool LocalSquare(Context* ctx, const DevGraph* g, const EnginePlan* plan, uint32
   const uint64_t tiles = WedgeTiles(w.n);
   if (tiles > 1) w.items_ratio = static_cast<uint64_t>(65536 * (0.02 + 0.008 * g->pair_min) / 35) + 1;
   {
-    Timed t(ctx, s, kSlotHouseWedge, 24.0 * (ve - vb), ve - vb);
+    Timed t(ctx, s, kSlotHouseWedge, 0, 0);  // (known below)
     LaunchSquareLight(w, s);
     LaunchWedgeTiles(w, kWedgeSquare, s);
   }
@@ -2143,6 +2147,12 @@ bool LocalSquare(Context* ctx, const DevGraph* g, const EnginePlan* plan, uint32
   if (w.items_ratio && pin[kWedgeAcc] * tiles > WedgeItemsMax(pin[3], w.items_ratio)) {
     if (bk.bounds) LaunchFill64(reinterpret_cast<uint64_t*>(bk.counts), bk.nbuckets, 0, s);
     return false;
+  }
+  if (ctx->profiling && !ctx->marks.empty()) {
+    // per start vertex its list bounds, per middle the entry and its list
+    // bounds, per wedge the entry
+    ctx->marks.back().bytes = 24.0 * (ve - vb) + 20.0 * static_cast<double>(pin[1]) + 4.0 * static_cast<double>(pin[2]);
+    ctx->marks.back().items = pin[2];
   }
   *count = pin[0];
   if (levels)

@@ -369,7 +369,7 @@ struct CliqueArgs {
   unsigned long long* nbig;
   uint32_t* huge;
   unsigned long long* nhuge;
-  // CliqueRowsKernel / CliqueCountKernel: one batch of big vertices.
+  // Row and count kernels: one batch of big vertices.
   // Vertex t's rows are row items [row_first[t], row_first[t+1]) (one per
   // row) and words [word_first[t], word_first[t+1]) - word_first[0] of rows.
   const uint32_t* verts;
@@ -378,7 +378,7 @@ struct CliqueArgs {
   const uint64_t* row_first;
   const uint64_t* word_first;
   unsigned long long* rows;      // nullptr (k == 3): no rows are written, the row kernels count
-  // CliqueRowsKernel with a hash of N+(v) in LDS (d <= kRowsHashMax): vertex
+  // CliqueRowsHashKernel (d <= kRowsHashMax): vertex
   // t owns chunks [chunk_first[t], chunk_first[t+1]) - chunk_first[0] of 64
   // rows each
   const uint64_t* chunk_first;
@@ -390,7 +390,7 @@ struct CliqueArgs {
   unsigned long long* nlong;
   // k == 3, nullable: tc[p] += the triangles through the edge stored at
   // cols[p] (p an index of some N+(x)), recorded by CliqueSmallKernel and
-  // CliqueRowsKernel as they find each triangle (v, u_i, u_j)
+  // the row kernels as they find each triangle (v, u_i, u_j)
   uint32_t* tc;
   uint32_t middles;              // see LaunchCliqueMiddles
 };
