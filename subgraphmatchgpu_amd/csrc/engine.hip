@@ -1683,7 +1683,6 @@ void LocalCliqueRange(Context* ctx, const DevGraph* g, const EnginePlan* plan, u
       if (tc) Fail(kErrOom, "bit rows of one start vertex exceed the memory the run may use");
       hh.insert(hh.end(), verts.begin(), verts.begin() + static_cast<int64_t>(first_fit));
     }
-    double after = 0;  // entries that follow another in the batches' lists
     for (uint64_t x0 = first_fit; x0 < nbig;) {
       uint64_t x1 = x0 + 1;
       while (x1 < nbig && fits(wf[x1 + 1] - wf[x0], rf[x1 + 1] - rf[x0])) ++x1;
@@ -1716,7 +1715,6 @@ void LocalCliqueRange(Context* ctx, const DevGraph* g, const EnginePlan* plan, u
           const double d = static_cast<double>(rf[x + 1] - rf[x]);
           keys += d * (d - 1) / 2;
         }
-        after += keys;
         Timed t(ctx, s, kSlotCliqueRows,
                 8.0 * keys + 20.0 * static_cast<double>(a.nitems) + (K > 3 ? 8.0 * static_cast<double>(words) : 0),
                 a.nitems);
@@ -1789,8 +1787,8 @@ void LocalCliqueRange(Context* ctx, const DevGraph* g, const EnginePlan* plan, u
       CliqueArgs b = a;
       b.v_begin = g->upper.first + 1;
       b.v_end = ve;
-      // per list of a lower neighbour: its entries after the middle
-      Timed t(ctx, s, kSlotCliqueRows, 4.0 * after, b.v_end - b.v_begin);
+      // (the row pass is credited with these entries)
+      Timed t(ctx, s, kSlotCliqueRows, 0, b.v_end - b.v_begin);
       LaunchCliqueMiddles(b, s);
     }
   }
@@ -1992,8 +1990,8 @@ void LocalHouse(Context* ctx, const DevGraph* g, uint64_t* count, RunStats* st) 
     const uint64_t ncuts = (tiles + 1) * n;
     Buf<uint32_t> cuts(ctx, !dense && tiles > 1 && 4 * ncuts <= ctx->RunAvailable() / 4 ? ncuts : 0);
     if (!dense) {
-      // (walked twice)
-      Timed tm(ctx, s, kSlotHouseWedge, 12.0 * static_cast<double>(wedges[1]), wedges[1]);
+      // (the second walk is not credited)
+      Timed tm(ctx, s, kSlotHouseWedge, 8.0 * static_cast<double>(wedges[1]), wedges[1]);
       if (cuts.get()) LaunchWedgeCuts(w, cuts.get(), s);
       w.cuts = cuts.get();
       LaunchWedgeTiles(w, kWedgeApex, s);
