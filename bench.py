@@ -5,21 +5,23 @@ a/b/c/d = 0.57/0.19/0.19/0.05, seed 1, symmetrized, deduplicated), count the
 4-clique (Q3) and then the diamond (Q2) over every start vertex, each with
 symmetry breaking, through the C ABI (libsme.so).  value = embeddings counted
 per second of step wall time, inputs already in HBM.  The graph keeps a
-degree-ranked copy (the 4-clique's count and levels are those of the
-original ids) and counting levels use the group schedule (group_max 512).
+degree-ranked copy (counts and levels are those of the original ids); the
+4-clique is counted over bit rows and the diamond from per-edge triangle
+counts.  The schedule (super_chunks 4, group_max 512) is the level engine's.
 
 Besides the JSON fields of the harness contract, the line carries
-  roofline     -- the dominant kernel family ("intersect": the set
-                  intersection verify kernels) timed with HIP events on the
-                  engine's stream over the timed steps; achieved = algorithmic
-                  bytes / kernel time against 8 TB/s HBM3E;
+  roofline     -- the kernel family that took the most time (the bit rows),
+                  timed with HIP events on the engine's stream over the timed
+                  steps; achieved = algorithmic bytes / kernel time against
+                  8 TB/s HBM3E;
   cpu_baseline -- a bounded sample of the same workload on the host cores.
 
 Second workload (--workload er-batch): 20,000 seeded Erdos-Renyi graphs
 (n uniform in [64, 8192], average degree uniform in [4, 48]) packed back to
 back; one step counts triangles and 4-cycles of every member in one
 bucketed pass per pattern (value = member graphs per second), after the
-autotuner has picked the schedule; the same members counted with one engine
+autotuner has picked the schedule (of the level engine; neither pattern goes
+through it by default, so all settings time alike); the same members counted with one engine
 pass per member are timed on a sample for comparison.
 
 Third workload (--workload serve): a resident R-MAT graph (scale 16, edge
@@ -38,8 +40,7 @@ so that stream cannot be replayed within a benchmark run.
 
 Fourth workload (--workload rmat22): R-MAT scale 22, edge factor 32, with
 5-clique and house under a 32 GB intermediate cap on the degree-ranked copy,
-as ranked start-range tasks for a bounded time per pattern; the rest of the
-range is projected from a sampled set of start vertices (bench_rmat22).
+each counted in full by one call (bench_rmat22).
 
 The default line (rmat20) also carries, as sub-objects, a bounded run of the
 second workload ("er_batch") and of the third on a 5 s stream replayed in

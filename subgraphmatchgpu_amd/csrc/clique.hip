@@ -97,11 +97,15 @@ __device__ __forceinline__ void AddBucket(const BucketRef& b, uint32_t v, u64 pe
 // choosing the mode on rem * steps < len (67 against 87 us, R-MAT scale 14).
 constexpr uint32_t kSmallGroup = 4;  // start vertices per wave step
 constexpr uint32_t kSmallStream = 32;    // lists up to this length are streamed
-// up to here one start vertex per wave step: 4,096 waves of 4 vertices would
-// leave half the chip idle (R-MAT scale 14: 67 us against 130 us)
+// up to here one start vertex per wave step, since 4,096 waves of 4 vertices
+// leave half the chip idle.  Whole triangle calls, one vertex and four a step:
+// R-MAT 14 148 and 182 us, G(16,000, 160,000) 83 and 81; above the line
+// G(24,000, 240,000) 87 and 83, G(32,000, 320,000) 91 and 87, R-MAT 15 357 and 367
 constexpr uint64_t kSmallAlone = 16384;
-// workgroups: what the chip holds at once; fewer where each would get a few
-// vertices, since every one ends with an atomic on the same counters
+// workgroups: what the chip holds at once; half of it up to 4 kSmallAlone start
+// vertices, where each would get a few, since every one ends with atomics on the
+// same counters (1,024 and 2,048 workgroups: G(40,000, 400,000) 90 and 160 us,
+// R-MAT 18, factor 4, 1.13 and 1.04 ms)
 constexpr uint64_t kSmallGrid = 2048, kSmallGridFew = 1024;
 
 struct SmallLds {

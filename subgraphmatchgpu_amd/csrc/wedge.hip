@@ -166,8 +166,10 @@ __global__ __launch_bounds__(kThreads, 6) void SquareLightKernel(WedgeArgs a) {
 // 38, searching).  The cuts of every list at the tiles' bounds are kept in a
 // table where there is room (one load instead of two searches: 38 -> 25 ms).
 //
-// Bound by the wave instructions of the walks and the list reads.  House from a third of R-MAT scale
-// 14's start vertices: 0.38 ms, where the level engine counted pairs for every
+// Bound by the list reads: on R-MAT scale 19 (below) 121 GB past L2 in 24.5 ms,
+// the rate of a large copy, with the VALU busy in 32 % of the cycles; on graphs
+// that the caches hold by the latency of the walks.  House from a third of R-MAT scale
+// 14's start vertices: 0.31 ms, where the level engine counted pairs for every
 // (v1, v2, v3) path (11.1 ms).  House of R-MAT scale 19, edge factor 32, from
 // its apexes (6.7e9 wedges walked twice): 25 ms, where one 64-bit device atomic
 // per wedge into dense arrays and their reduction took 327 ms.
