@@ -646,3 +646,26 @@ def test_start_vertices_over_65535_neighbours(dev):
     r = dev.count(dg, sme.Plan(1), vb, ve)
     assert (r.count, r.levels) == (want[0], want[1])
     dg.release()
+
+
+# lists of which a wave streams 1,024 entries at a time, just below, at and above one and two such steps
+@pytest.mark.gpu
+@pytest.mark.parametrize("degree", [1000, 1023, 1024, 1025, 2047, 2048, 2049, 9000])
+def test_path_runs_over_long_lists(dev, degree):
+    n = 9216
+    low = np.zeros(0, dtype=np.int64)
+    a, b = [low], [low]
+    for h, step in ((n - 1, 1), (n - 2, 2), (n - 3, 3)):  # (the hubs' lists have ends in common)
+        ends = (np.arange(degree) * step) % (n - 3)
+        a.append(np.full(degree, h))
+        b.append(ends)
+    # the hubs among themselves, and what each path adds
+    a += [np.array([n - 1, n - 1, n - 2]), np.arange(0, 6000, 2)]
+    b += [np.array([n - 2, n - 3, n - 3]), np.arange(1, 6001, 2)]
+    a, b = np.concatenate(a), np.concatenate(b)
+    key = np.unique(np.concatenate([a * n + b, b * n + a]))
+    g = sme.Graph(np.searchsorted(key, np.arange(n + 1) * n).astype(np.uint64), (key % n).astype(np.uint32))
+    for q in (2, 6, 8):
+        for vb, ve in ((0, n), (n - 3, n)):
+            want = oracle.light_count(g.row_ptrs, g.cols, q, 3, v_begin=vb, v_end=ve)
+            assert on_gpu(dev, g, q, vb, ve) == (want[0], want[1])
