@@ -450,7 +450,7 @@ __device__ __forceinline__ bool MiddleTakes(uint32_t d, uint32_t first, uint32_t
 }
 
 // Rows of a vertex v whose N+(v) spans fewer than kRowsTableRange ids: a
-// workgroup takes kTableRows rows at a time (every gridDim.y-th such part).  N+(v) becomes an LDS
+// workgroup takes a.part rows at a time (every gridDim.y-th such part).  N+(v) becomes an LDS
 // table with, per 32 consecutive ids, the bits of those in N+(v) and the local
 // index of the first, so one 8-byte LDS load decides an entry of N+(u_i) and
 // gives its j, without the probe chains of a hash.  Each wave streams N+(u_i)
@@ -467,7 +467,14 @@ __device__ __forceinline__ bool MiddleTakes(uint32_t d, uint32_t first, uint32_t
 // largest whose table (16 KB) still lets 32 waves share a CU; on a ranked
 // graph the 60,000 vertices with d > 64 all lie within it.
 enum RowsMode : int { kRowsBits = 0, kRowsCount = 1, kRowsEdges = 2 };
-constexpr uint32_t kTableRows = 256;
+// Rows a workgroup takes at a time: 256, since each part builds the table anew, but
+// 64 where the launch has fewer than kTableFew workgroups of 256 (the 8 per CU that
+// its LDS lets the chip hold): a wave's 64 rows one after another were most of such
+// a call.  256 and 64 rows, triangle / 4-clique / diamond (us): 5 vertices joined to
+// 300 48 / 88 / 108 and 33 / 67 / 66; R-MAT 10 80 / 154 / 156 and 62 / 124 / 106;
+// R-MAT 12 104 / 343 / 210 and 81 / 305 / 141; above the line the ranked R-MAT 16
+// (3,124 workgroups) 322 / 396 / 726 and 364 / 398 / 753
+constexpr uint32_t kTableRows = 256, kTableRowsFew = 64, kTableFew = 2048;
 
 template <int kMode>
 __global__ __launch_bounds__(kThreads) void CliqueRowsTableKernel(CliqueArgs a) {
@@ -485,7 +492,7 @@ __global__ __launch_bounds__(kThreads) void CliqueRowsTableKernel(CliqueArgs a) 
     const uint32_t v = a.verts[x];
     const uint64_t nb = a.up[v];
     const uint32_t d = static_cast<uint32_t>(a.rp[v + 1] - nb);
-    if (blockIdx.y * kTableRows >= d) continue;
+    if (blockIdx.y * a.part >= d) continue;
     const uint32_t base = a.cols[nb], vmax = a.cols[nb + d - 1];
     if (!TableTakes(d, base, vmax)) continue;
     const uint32_t range = vmax - base + 1;
@@ -500,8 +507,8 @@ __global__ __launch_bounds__(kThreads) void CliqueRowsTableKernel(CliqueArgs a) 
       atomicOr(tab + (off >> 5), add);
     }
     u64 mine = 0;  // triangles from v found by this lane
-    for (uint32_t r0 = blockIdx.y * kTableRows; r0 < d; r0 += gridDim.y * kTableRows) {
-      const uint32_t r1 = r0 + kTableRows < d ? r0 + kTableRows : d;
+    for (uint32_t r0 = blockIdx.y * a.part; r0 < d; r0 += gridDim.y * a.part) {
+      const uint32_t r1 = r0 + a.part < d ? r0 + a.part : d;
       if (kMode == kRowsEdges)
         for (uint32_t k = threadIdx.x; k < (d + 1) / 2; k += kThreads) lds_col[k] = 0;
       __syncthreads();
@@ -1309,15 +1316,17 @@ void LaunchCliqueRowsTable(const CliqueArgs& a, uint32_t dmax, hipStream_t strea
   if (dmax > kRowsTableMax) dmax = kRowsTableMax;
   // parts of one vertex run side by side where the vertices alone would not
   // fill the chip several times over
-  uint32_t parts = (dmax + kTableRows - 1) / kTableRows;
+  CliqueArgs b = a;
+  b.part = a.nverts * ((dmax + kTableRows - 1) / kTableRows) < kTableFew ? kTableRowsFew : kTableRows;
+  uint32_t parts = (dmax + b.part - 1) / b.part;
   if (a.nverts > 4096 && parts > 4) parts = 4;
   const dim3 grid(Grid(a.nverts, 1), parts), block(kThreads);
   if (a.tc)
-    hipLaunchKernelGGL(CliqueRowsTableKernel<kRowsEdges>, grid, block, 0, stream, a);
+    hipLaunchKernelGGL(CliqueRowsTableKernel<kRowsEdges>, grid, block, 0, stream, b);
   else if (a.rows)
-    hipLaunchKernelGGL(CliqueRowsTableKernel<kRowsBits>, grid, block, 0, stream, a);
+    hipLaunchKernelGGL(CliqueRowsTableKernel<kRowsBits>, grid, block, 0, stream, b);
   else
-    hipLaunchKernelGGL(CliqueRowsTableKernel<kRowsCount>, grid, block, 0, stream, a);
+    hipLaunchKernelGGL(CliqueRowsTableKernel<kRowsCount>, grid, block, 0, stream, b);
 }
 
 void LaunchCliqueMiddles(const CliqueArgs& a, hipStream_t stream) {
@@ -1345,7 +1354,7 @@ void LaunchCliqueDense(const CliqueArgs& a, int words, hipStream_t stream) {
   }
 }
 
-void LaunchCliqueCount(const CliqueArgs& a, hipStream_t stream) {
+void LaunchCliqueCount(const CliqueArgs& a, uint32_t dmax, hipStream_t stream) {
   if (a.nitems == 0) return;
   const dim3 grid(Grid(a.nitems, kWaves)), block(kThreads);
   const uint64_t rows = Grid(a.nitems, 1);
@@ -1353,14 +1362,15 @@ void LaunchCliqueCount(const CliqueArgs& a, hipStream_t stream) {
   switch (a.k) {
     case 4: hipLaunchKernelGGL(CliqueCount4Kernel, grid, block, 0, stream, a); break;
     case 5:
+      // (a row has fewer members than the largest d: no launch that finds none)
       hipLaunchKernelGGL(CliquePackKernel<5>, grid, block, 0, stream, a);
-      hipLaunchKernelGGL((CliqueLongKernel<8, false>), longs, block, 0, stream, a);
-      hipLaunchKernelGGL((CliqueLongKernel<16, true>), longs, block, 0, stream, a);
-      hipLaunchKernelGGL(CliqueUnpackedKernel<5>, grid, block, 0, stream, a);
+      if (dmax > kPackWave) hipLaunchKernelGGL((CliqueLongKernel<8, false>), longs, block, 0, stream, a);
+      if (dmax > 256) hipLaunchKernelGGL((CliqueLongKernel<16, true>), longs, block, 0, stream, a);
+      if (dmax > kPackLong) hipLaunchKernelGGL(CliqueUnpackedKernel<5>, grid, block, 0, stream, a);
       break;
     case 6:
       hipLaunchKernelGGL(CliquePackKernel<6>, grid, block, 0, stream, a);
-      hipLaunchKernelGGL(CliqueUnpackedKernel<6>, grid, block, 0, stream, a);
+      if (dmax > kPackWave) hipLaunchKernelGGL(CliqueUnpackedKernel<6>, grid, block, 0, stream, a);
       break;
   }
 }

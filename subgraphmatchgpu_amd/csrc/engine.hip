@@ -1778,7 +1778,7 @@ void LocalCliqueRange(Context* ctx, const DevGraph* g, const EnginePlan* plan, u
         b = a;
         b.nverts = rest - x0;
         b.nitems = rf[rest] - rf[x0];
-        LaunchCliqueCount(b, s);
+        LaunchCliqueCount(b, hd_sorted[x0], s);
       }
       st->batches++;
       x0 = x1;

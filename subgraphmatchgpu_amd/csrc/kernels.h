@@ -393,6 +393,7 @@ struct CliqueArgs {
   // the row kernels as they find each triangle (v, u_i, u_j)
   uint32_t* tc;
   uint32_t middles;              // see LaunchCliqueMiddles
+  uint32_t part;                 // rows that CliqueRowsTableKernel takes at a time (set by the launcher)
 };
 // ---------------------------------------------------------------------------
 // House (5-cycle with one chord closing a triangle) counted from edge
@@ -475,7 +476,8 @@ void LaunchCliqueMiddles(const CliqueArgs& a, hipStream_t stream);
 constexpr uint32_t kRowsHashMax = 4096;
 constexpr uint32_t kRowsHashSmall = 512;
 void LaunchCliqueRowsHash(const CliqueArgs& a, bool small_table, hipStream_t stream);
-void LaunchCliqueCount(const CliqueArgs& a, hipStream_t stream);
+// 4-, 5- and 6-cliques over the rows of a batch, d <= dmax.
+void LaunchCliqueCount(const CliqueArgs& a, uint32_t dmax, hipStream_t stream);
 // 4-cliques of vertices with 32 (words - 4) < d <= 32 words, words 4, 8, 12 or
 // 16 (verts, nverts, row_first, word_first and rows of those vertices).
 constexpr uint32_t kDenseMax = 512;

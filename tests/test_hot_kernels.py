@@ -1,6 +1,7 @@
 """Sizes at which the counting kernels change tile, table or schedule, against
 the oracle: on the CPU through the stand-in runtime of tests/emu (under
 AddressSanitizer) and on the GPU.  Counts are whole numbers and must be equal."""
+import math
 import os
 import subprocess
 
@@ -669,3 +670,29 @@ def test_path_runs_over_long_lists(dev, degree):
         for vb, ve in ((0, n), (n - 3, n)):
             want = oracle.light_count(g.row_ptrs, g.cols, q, 3, v_begin=vb, v_end=ve)
             assert on_gpu(dev, g, q, vb, ve) == (want[0], want[1])
+
+
+# rows of few vertices (64 a workgroup) and of as many as fill the chip (256), in one part and two
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,copies", [(65, 1), (257, 7), (64 + 192, 2), (66, 2047), (66, 2048), (257, 1023), (257, 1024)])
+def test_row_parts(dev, d, copies):
+    g = union(*[fan(d + 1, d, 1, 6 * d, 100 * copies + k) for k in range(min(copies, 8))] * (-(-copies // 8)))
+    assert g.n >= copies * (d + 1)
+    for q in (0, 2, 3, 7):
+        want = oracle.light_count(g.row_ptrs, g.cols, q, 3)
+        assert want[0] and on_gpu(dev, g, q) == (want[0], want[1])
+    dg = dev.upload(g)
+    assert dev.count_only(dg, sme.Plan(4)).count == oracle.light_count(g.row_ptrs, g.cols, 4, 3)[0]
+    dg.release()
+
+
+# cliques whose first rows have as many members as a wave, a workgroup of either size and neither packs,
+# and one more; no kernel is launched for rows that cannot be there
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,q", [(n, 7) for n in (66, 129, 130, 131, 257, 258, 259, 513, 514, 515)] +
+                                [(n, 11) for n in (66, 129, 130, 131, 258)])
+def test_clique_rows_by_size(dev, n, q):
+    k = 5 if q == 7 else 6
+    count, levels = on_gpu(dev, clique(n), q)
+    assert count == math.comb(n, k) == levels[-1]
+    assert sorted(set(levels)) == sorted({math.comb(n, j) for j in range(1, k + 1)})
