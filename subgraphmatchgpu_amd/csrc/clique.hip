@@ -468,13 +468,14 @@ __device__ __forceinline__ bool MiddleTakes(uint32_t d, uint32_t first, uint32_t
 // graph the 60,000 vertices with d > 64 all lie within it.
 enum RowsMode : int { kRowsBits = 0, kRowsCount = 1, kRowsEdges = 2 };
 // Rows a workgroup takes at a time: 256, since each part builds the table anew, but
-// 64 where the launch has fewer than kTableFew workgroups of 256 (the 8 per CU that
-// its LDS lets the chip hold): a wave's 64 rows one after another were most of such
-// a call.  256 and 64 rows, triangle / 4-clique / diamond (us): 5 vertices joined to
-// 300 48 / 88 / 108 and 33 / 67 / 66; R-MAT 10 80 / 154 / 156 and 62 / 124 / 106;
-// R-MAT 12 104 / 343 / 210 and 81 / 305 / 141; above the line the ranked R-MAT 16
-// (3,124 workgroups) 322 / 396 / 726 and 364 / 398 / 753
-constexpr uint32_t kTableRows = 256, kTableRowsFew = 64, kTableFew = 2048;
+// 64 where the launch has fewer than kTableFew workgroups of 256, two per CU: a
+// wave's 64 rows one after another were most of such a call.  256 and 64 rows,
+// triangle / 4-clique / diamond (us): 5 vertices joined to 300 48 / 88 / 108 and 33 /
+// 67 / 66; R-MAT 10 80 / 154 / 156 and 62 / 124 / 106; R-MAT 11 98 / 227 / 195 and 78
+// / 195 / 135.  Above the line some gain (R-MAT 12, 1,092 workgroups: 104 / 343 / 210
+// and 81 / 305 / 141) and others lose (four G(600, 0.3), 1,548: triangles 95 and 114;
+// the ranked R-MAT 16, 3,124: 322 and 364)
+constexpr uint32_t kTableRows = 256, kTableRowsFew = 64, kTableFew = 512;
 
 template <int kMode>
 __global__ __launch_bounds__(kThreads) void CliqueRowsTableKernel(CliqueArgs a) {
@@ -1079,8 +1080,10 @@ __device__ __forceinline__ u64 CountWave(const u64* rows, uint32_t d, uint32_t i
 
 // 4-cliques of the vertices with d > kDenseMax: a wave takes groups of
 // kRowGroup consecutive rows, one search for the group's first vertex, then a
-// walk forward (a row is light next to the search).
-__global__ __launch_bounds__(kThreads) void CliqueCount4Kernel(CliqueArgs a) {
+// walk forward (a row is light next to the search).  A bucket gets one sum per group
+// and vertex: with one per row 16 buckets of R-MAT 14, factor 8, took 0.88 ms, now
+// 0.63.  (Held to 64 registers, without which the sum takes an eighth of the waves.)
+__global__ __launch_bounds__(kThreads, 8) void CliqueCount4Kernel(CliqueArgs a) {
   __shared__ u64 lds_s[kWaves][kWordsMax];
   __shared__ uint32_t lds_q[kWaves][2 * kWave];
   const int lane = threadIdx.x & (kWave - 1);
@@ -1092,15 +1095,21 @@ __global__ __launch_bounds__(kThreads) void CliqueCount4Kernel(CliqueArgs a) {
   const uint64_t base = a.row_first[0];
   for (uint64_t t0 = wave * kRowGroup; t0 < a.nitems; t0 += nwaves * kRowGroup) {
     const uint64_t te = t0 + kRowGroup < a.nitems ? t0 + kRowGroup : a.nitems;
-    uint64_t x = ItemVertexWave(a, t0, lane);
+    uint64_t x = ItemVertexWave(a, t0, lane), of = x;
+    u64 vk = 0;  // this group's share of the 4-cliques from vertex `of`
     for (uint64_t t = t0; t < te; ++t) {
       while (a.row_first[x + 1] - base <= t) ++x;
+      if (a.bk.bounds && x != of) {
+        AddBucket(a.bk, a.verts[of], vk, lane);
+        vk = 0;
+        of = x;
+      }
       const uint32_t d = static_cast<uint32_t>(a.row_first[x + 1] - a.row_first[x]);
       const uint32_t i = static_cast<uint32_t>(t - (a.row_first[x] - base));
       const u64* rows = a.rows + (a.word_first[x] - a.word_first[0]);
-      const u64 vk = CountRow<4>(rows, d, i, lds_s[wid], nullptr, nullptr, lds_q[wid], lane, &cs);
-      if (a.bk.bounds) AddBucket(a.bk, a.verts[x], vk, lane);
+      vk += CountRow<4>(rows, d, i, lds_s[wid], nullptr, nullptr, lds_q[wid], lane, &cs);
     }
+    if (a.bk.bounds) AddBucket(a.bk, a.verts[of], vk, lane);
   }
   FlushSums(a.acc, 4, cs);
 }

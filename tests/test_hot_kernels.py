@@ -674,7 +674,7 @@ def test_path_runs_over_long_lists(dev, degree):
 
 # rows of few vertices (64 a workgroup) and of as many as fill the chip (256), in one part and two
 @pytest.mark.gpu
-@pytest.mark.parametrize("d,copies", [(65, 1), (257, 7), (64 + 192, 2), (66, 2047), (66, 2048), (257, 1023), (257, 1024)])
+@pytest.mark.parametrize("d,copies", [(65, 1), (257, 7), (256, 2), (66, 504), (66, 512), (257, 248), (257, 256), (66, 2048), (257, 1024)])
 def test_row_parts(dev, d, copies):
     g = union(*[fan(d + 1, d, 1, 6 * d, 100 * copies + k) for k in range(min(copies, 8))] * (-(-copies // 8)))
     assert g.n >= copies * (d + 1)
