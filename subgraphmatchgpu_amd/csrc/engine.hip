@@ -2185,8 +2185,10 @@ bool HouseLevels(const EnginePlan* plan) {
 //
 // A tile costs a workgroup its counters and a chain of waits whatever it holds:
 // 24 ns a tile over the whole chip (15 n / 65,536 where one tile holds all ids:
-// no list is cut then; 3 with the small workgroups), and an entry walked up to
-// 0.016 ns (0.004), both walks together.  The level engine intersects two lists
+// no list is cut then; 3 with the small workgroups), and an entry walked 0.0075 ns
+// (0.004), both walks together, of the longest list 0.0158 where it is walked from
+// its vertex's neighbours: one wave of a workgroup reads a list, and several long
+// ones are read side by side.  The level engine intersects two lists
 // for every (edge, further neighbour) pair: 0.1 ns and 0.02 per entry of the
 // shorter one, within a factor of two.
 //                                      pairs    shorter  engine     walk
@@ -2197,7 +2199,10 @@ bool HouseLevels(const EnginePlan* plan) {
 //   R-MAT 19, factor 1                 1.3e8             81         56
 //   R-MAT 20, factor 1                 3.4e8            246        225
 //   last vertex joined to all 60,000   2e5        2       0.5       57
-//   last 3 to half of 60,000           5e5     1800      22         26
+//   last 3 to half of 60,000           5e5     1800      21         26
+//   last 3 to 0.7 of 60,000            1.7e6   1840      61         40
+//   last 3 to 0.7 of 30,000            8.9e5    920      16         10
+//   last 2 to 0.4 of 70,000            2.4e5               5.5       22
 //   last 3 to four fifths of 16,000    4.5e5    640       7.0        1.6
 //   first joined to all 16,000         2.6e8      3      31          0.6
 bool HouseTilesPay(const DevGraph* g, uint32_t vb, uint32_t ve) {
@@ -2205,10 +2210,11 @@ bool HouseTilesPay(const DevGraph* g, uint32_t vb, uint32_t ve) {
   const bool small = g->n <= kWedgeSmallIds;
   const double n = static_cast<double>(g->n), starts = static_cast<double>(ve - vb);
   const double tile_ns = small ? 3.0 : tiles > 1 ? 24.0 : 15.0 / 65536 * n;
-  const double walk_ns = small ? 0.004 : 0.016;
+  const double longest = static_cast<double>(g->max_degree);
+  const double walk = small ? 0.004 * g->wedges : 0.0075 * g->wedges + 0.0083 * longest * longest;
   // (0.1 ms: the engine's launches)
   const double engine = 1e5 + (0.1 + 0.02 * g->pair_min) * static_cast<double>(g->house_work[ve] - g->house_work[vb]);
-  return engine >= 0.8 * tile_ns * starts * tiles + walk_ns * g->wedges * starts / n;
+  return engine >= 0.8 * tile_ns * starts * tiles + walk * starts / n;
 }
 
 // Bytes of which a house count over a range takes at most a quarter; 0: not that

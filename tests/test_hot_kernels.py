@@ -442,7 +442,8 @@ def test_house_over_sparse_ids(dev, n, d, m, tiles):
 # engine), below them (tiles)
 @pytest.mark.gpu
 @pytest.mark.parametrize("n,hubs,share,m,low,tiles", [(9000, 1, 1.0, 9000, False, False), (60000, 1, 1.0, 60000, False, False),
-                                                      (9000, 1, 1.0, 9000, True, True), (70000, 2, 0.4, 70000, False, False)])
+                                                      (9000, 1, 1.0, 9000, True, True), (70000, 2, 0.4, 70000, False, False),
+                                                      (30000, 3, 0.7, 60000, False, True)])
 def test_house_under_long_lists(dev, n, hubs, share, m, low, tiles):
     g = hubs_over(n, hubs, share, m, n)
     if low:  # ids in reverse
